@@ -71,14 +71,14 @@ int two_sided_t(const T* Am, const T* X, const T* Bm, T* out, int64_t batch, int
     const T* P = a_direct ? Am : Ap;
     const int64_t sP = a_direct ? sA : (nA > 1 ? m * ldm : 0);
     GemmArgs g{P, a_direct ? m : ldm, sP, XT, ldm, n * ldm, (int)m, (int)n, (int)ldm, 0, 0, nullptr};
-    EpiStore<T, A> e{AX, ldn, m * ldn, vec_ok<T>(AX, ldn, m * ldn)};
+    EpiStore<T, A> e{AX, ldn, m * ldn};
     if (launch_gemm<T, false>(g, e, nb, stream, name_left)) return -1;
   }
   {
     const T* Q = b_direct ? Bm : Bq;
     const int64_t sQ = b_direct ? sB : (nB > 1 ? n * ldn : 0);
     GemmArgs g{AX, ldn, m * ldn, Q, b_direct ? n : ldn, sQ, (int)m, (int)n, (int)ldn, 0, 0, nullptr};
-    EpiStore<T, A> e{out, n, m * n, vec_ok<T>(out, n, m * n)};
+    EpiStore<T, A> e{out, n, m * n};
     if (launch_gemm<T, false>(g, e, nb, stream, name_right)) return -1;
   }
   return 0;

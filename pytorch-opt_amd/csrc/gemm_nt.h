@@ -323,6 +323,148 @@ struct HasSkip : std::false_type {};
 template <class E>
 struct HasSkip<E, std::void_t<decltype(std::declval<const E&>().skip(0, false))>> : std::true_type {};
 
+// The epilogue of a product kernel, for the fragment rows EFM .. EFM +
+// WTE/16 - 1 of one wave's sub-tile at (wr0, wc0) (all of its rows, or with
+// K groups its half; EFM is a constant so that acc stays in registers).
+//
+// Per wave and staged through LDS so every global access of the
+// functor is a run of up to 8 consecutive elements of one output row.
+// Each wave owns a private slice (RPP rows of its WTM x WTN sub-tile at a
+// time), so no cross-wave synchronisation is needed:
+//   1. the functor's global reads for all of this lane's direct runs are
+//      issued (epi.load), then the wave writes RPP rows of raw
+//      accumulators to its slice while they are in flight;
+//   2. direct pass: runs along output rows (i, j..j+7) -> epi.put, which
+//      hands back the value the transposed pass should see;
+//   3. transposed pass (mirror of a symmetric tile, or the functor's
+//      transposed copy): reads for all runs (epi.load_t), then runs along
+//      (j, i..i+7) -> epi.put_t.
+// Reading before writing keeps one memory latency per pass instead of
+// one per run: a functor may read and write the same array (X' = a·X + v
+// in place), so the compiler cannot hoist a run's read above the
+// previous run's store by itself. Each run reads and writes only its own
+// elements, and the direct and transposed runs of one tile cover
+// disjoint positions, so the early reads see the values from before the
+// launch.
+// In symmetric (UPPER) products the value for (i, j), i <= j, is stored
+// at (i, j) by its own direct pass and at (j, i) by its transposed pass,
+// so the stored matrix is exactly symmetric. On diagonal tiles the 8x8
+// blocks on the diagonal are written whole by the direct pass, each
+// position below the diagonal taking the staged value of its mirror
+// (j, i), so every run stays a full 16-byte access (partial runs there
+// made the diagonal tiles' epilogue 1.5-2x longer than the others' and
+// the last to finish); the transposed pass covers the rest below the
+// diagonal.
+template <typename MF, class Plan, bool UPPER, int EFM, class Epi, int FM, int FN>
+__device__ __forceinline__ void store_rows(const typename MF::cvec_t (&acc)[FM][FN], typename Epi::S* stg, Epi& epi,
+                                           const GemmArgs& g, int b, int wr0, int wc0, bool diag, int lane) {
+  typedef typename Epi::S S;
+  constexpr int RPP = Plan::RPP, SP = Plan::SP, WTE = Plan::WTE, WTN = Plan::WTN;
+  const bool need_t = UPPER || epi.has_t();
+  const int nrem = g.N - wc0;
+  // direct runs: 8 lanes cover 64 consecutive columns of one row
+  constexpr int RUNS = WTN / 8;  // 8-element runs per row
+  // lanes per output row: the largest divisor of RUNS that is at most 8
+  constexpr int LGD = RUNS % 8 == 0 ? 8 : RUNS % 6 == 0 ? 6 : RUNS % 4 == 0 ? 4 : RUNS % 2 == 0 ? 2 : 1;
+  constexpr int RPB = 64 / LGD;
+  constexpr int CBLK = RUNS / LGD;
+  static_assert(RUNS % LGD == 0 && LGD * 8 <= 64, "wave tile width: whole 8-element runs");
+  constexpr int ITEMS = ((RPP + RPB - 1) / RPB) * CBLK;  // direct runs per lane
+  // when LGD does not divide 64 (wave tiles 48 wide) the last 64 % LGD lanes
+  // would repeat the next block's first runs: they sit out
+  const bool lane_ok = LGD * RPB == 64 || lane < LGD * RPB;
+  // transposed runs: 8 lanes share a column c and cover 64 consecutive rows
+  constexpr int CBT = WTN / 8;
+  constexpr int ITEMS_T = ((RPP / 8 + 7) / 8) * CBT;
+#pragma unroll
+  for (int hp = 0; hp < WTE / RPP; ++hp) {
+    const int pr0 = wr0 + EFM * MF::MN + hp * RPP;  // first output row of this pass
+    if (pr0 >= g.M || nrem <= 0) break;
+    const int rows = min(RPP, g.M - pr0);
+    typename Epi::Pre pre[ITEMS];
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+      const int r = (it / CBLK) * RPB + lane / LGD;
+      const int c = ((it % CBLK) * LGD + lane % LGD) * 8;
+      const int i = pr0 + r, j0 = wc0 + c;
+      const int n = min(8, nrem - c);
+      // diagonal tiles: skip runs below the diagonal; a run inside an 8x8 block on it is full
+      const int kbeg = diag && i - j0 >= 8 ? 8 : 0;
+      if (lane_ok && r < rows && c < nrem && kbeg < n) epi.load(b, i, j0, kbeg, n, pre[it]);
+    }
+#pragma unroll
+    for (int fm = EFM + hp * (RPP / MF::MN); fm < EFM + (hp + 1) * (RPP / MF::MN); ++fm)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int r = 0; r < MF::NACC; ++r) {
+          const int li = (fm - EFM) * MF::MN - hp * RPP + MF::row(lane, r);
+          const int lj = fn * MF::MN + MF::col(lane, r);
+          stg[li * SP + lj] = static_cast<S>(acc[fm][fn][r]);
+        }
+    __builtin_amdgcn_s_waitcnt(PTO_LGKM0);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+      const int r = (it / CBLK) * RPB + lane / LGD;
+      const int c = ((it % CBLK) * LGD + lane % LGD) * 8;
+      const int i = pr0 + r, j0 = wc0 + c;
+      const int n = min(8, nrem - c);
+      const int kbeg = diag && i - j0 >= 8 ? 8 : 0;
+      if (!(lane_ok && r < rows && c < nrem && kbeg < n)) continue;
+      // dk in 1..7: the run crosses the diagonal; its positions k < dk lie below it and take the
+      // mirrored value, staged at row j0 + k, column i of the same slab (the 16-aligned slab holds
+      // the whole 8-row group; those diagonal-block entries are never written back)
+      S v[8], vo[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = stg[r * SP + c + k];
+      if (diag && i - j0 > 0) {
+        const int dk = i - j0;
+#pragma unroll
+        for (int k = 0; k < 7; ++k)
+          if (k < dk) v[k] = stg[(c + k - (pr0 - wc0)) * SP + r + (pr0 - wc0)];
+      }
+      epi.put(b, i, j0, v, kbeg, n, pre[it], vo);
+      if (need_t && !Epi::kVoIsV && !(diag && i - j0 >= 0)) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) stg[r * SP + c + k] = vo[k];
+      }
+    }
+    if (need_t) {
+      if constexpr (!Epi::kVoIsV) {  // the write-back above must land first
+        __builtin_amdgcn_s_waitcnt(PTO_LGKM0);
+        __builtin_amdgcn_wave_barrier();
+      }
+      // output row j = wc0 + c, columns i = pr0 + r..r+7
+      typename Epi::PreT pret[ITEMS_T];
+#pragma unroll
+      for (int it = 0; it < ITEMS_T; ++it) {
+        const int c = (it % CBT) * 8 + lane / 8;
+        const int r = ((it / CBT) * 8 + lane % 8) * 8;
+        const int j = wc0 + c, i0 = pr0 + r;
+        int n = min(8, rows - r);
+        if (diag && j - i0 < 8) n = 0;  // below the diagonal, outside its 8x8 blocks
+        if (c < nrem && r < rows && n > 0) epi.load_t(b, j, i0, n, pret[it]);
+      }
+#pragma unroll
+      for (int it = 0; it < ITEMS_T; ++it) {
+        const int c = (it % CBT) * 8 + lane / 8;
+        const int r = ((it / CBT) * 8 + lane % 8) * 8;
+        const int j = wc0 + c, i0 = pr0 + r;
+        int n = min(8, rows - r);
+        if (diag && j - i0 < 8) n = 0;
+        if (!(c < nrem && r < rows && n > 0)) continue;
+        S v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = k < n ? stg[(r + k) * SP + c] : S(0);
+        epi.put_t(b, j, i0, v, n, pret[it]);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(PTO_LGKM0);
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // PT: P is stored [K][M] (M contiguous) and read like a QN operand. For a
 // symmetric P (B' in X' = B'·X, A in A·A) that is P itself: its rows are
 // its columns, so the product reads it with conflict-free transposing LDS
@@ -751,56 +893,12 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
     stage_barrier();
   }
 
-  // Epilogue, per wave and staged through LDS so every global access of the
-  // functor is a run of up to 8 consecutive elements of one output row.
-  // Each wave owns a private slice (RPP rows of its WTM x WTN sub-tile at a
-  // time), so no cross-wave synchronisation is needed:
-  //   1. the functor's global reads for all of this lane's direct runs are
-  //      issued (epi.load), then the wave writes RPP rows of raw
-  //      accumulators to its slice while they are in flight;
-  //   2. direct pass: runs along output rows (i, j..j+7) -> epi.put, which
-  //      hands back the value the transposed pass should see;
-  //   3. transposed pass (mirror of a symmetric tile, or the functor's
-  //      transposed copy): reads for all runs (epi.load_t), then runs along
-  //      (j, i..i+7) -> epi.put_t.
-  // Reading before writing keeps one memory latency per pass instead of
-  // one per run: a functor may read and write the same array (X' = a·X + v
-  // in place), so the compiler cannot hoist a run's read above the
-  // previous run's store by itself. Each run reads and writes only its own
-  // elements, and the direct and transposed runs of one tile cover
-  // disjoint positions, so the early reads see the values from before the
-  // launch.
-  // In symmetric (UPPER) products the value for (i, j), i <= j, is stored
-  // at (i, j) by its own direct pass and at (j, i) by its transposed pass,
-  // so the stored matrix is exactly symmetric. On diagonal tiles the 8x8
-  // blocks on the diagonal are written whole by the direct pass, each
-  // position below the diagonal taking the staged value of its mirror
-  // (j, i), so every run stays a full 16-byte access (partial runs there
-  // made the diagonal tiles' epilogue 1.5-2x longer than the others' and
-  // the last to finish); the transposed pass covers the rest below the
-  // diagonal.
-  constexpr int RPP = Plan::RPP, SP = Plan::SP, WTE = Plan::WTE;
+  // Epilogue (store_rows), each wave staging through its own LDS slice.
   const int wa = wave / Plan::WPA;  // < NS
   char* arr = wa == 0 ? st0 : wa == 1 ? st1 : wa == 2 ? st2 : wa == 3 ? st3 : wa == 4 ? st4 : wa == 5 ? st5 : wa == 6 ? st6 : st7;
-  S* stg = reinterpret_cast<S*>(arr) + (wave % Plan::WPA) * RPP * SP;
+  S* stg = reinterpret_cast<S*>(arr) + (wave % Plan::WPA) * Plan::RPP * Plan::SP;
   const bool diag = UPPER && ti == tj;
-  const bool need_t = UPPER || epi.has_t();
   const int wr0 = row0 + wm * WTM, wc0 = col0 + wn * WTN;  // sub-tile origin
-  const int nrem = g.N - wc0;
-  // direct runs: 8 lanes cover 64 consecutive columns of one row
-  constexpr int RUNS = WTN / 8;  // 8-element runs per row
-  // lanes per output row: the largest divisor of RUNS that is at most 8
-  constexpr int LGD = RUNS % 8 == 0 ? 8 : RUNS % 6 == 0 ? 6 : RUNS % 4 == 0 ? 4 : RUNS % 2 == 0 ? 2 : 1;
-  constexpr int RPB = 64 / LGD;
-  constexpr int CBLK = RUNS / LGD;
-  static_assert(RUNS % LGD == 0 && LGD * 8 <= 64, "wave tile width: whole 8-element runs");
-  constexpr int ITEMS = ((RPP + RPB - 1) / RPB) * CBLK;  // direct runs per lane
-  // when LGD does not divide 64 (wave tiles 48 wide) the last 64 % LGD lanes
-  // would repeat the next block's first runs: they sit out
-  const bool lane_ok = LGD * RPB == 64 || lane < LGD * RPB;
-  // transposed runs: 8 lanes share a column c and cover 64 consecutive rows
-  constexpr int CBT = WTN / 8;
-  constexpr int ITEMS_T = ((RPP / 8 + 7) / 8) * CBT;
   if constexpr (KG == 2) {
     // Sum the two groups' partial tiles: each wave keeps WTE rows of its
     // sub-tile (group 0 the first half, group 1 the second) and hands the
@@ -836,107 +934,14 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
 #undef PTO_EXCHANGE
 #undef PTO_SLOT
   }
-  // The epilogue for the fragment rows EFM .. EFM + WTE/16 - 1 of this
-  // wave's sub-tile (all of them, or with K groups its half), written
-  // out with a constant EFM so that acc stays in registers.
-#define PTO_STORE_ROWS(EFM)                                                                          \
-_Pragma("unroll")                                                                                    \
-  for (int hp = 0; hp < WTE / RPP; ++hp) {                                                           \
-    const int pr0 = wr0 + (EFM) * MF::MN + hp * RPP;  /* first output row of this pass */            \
-    if (pr0 >= g.M || nrem <= 0) break;                                                              \
-    const int rows = min(RPP, g.M - pr0);                                                            \
-    typename Epi::Pre pre[ITEMS];                                                                    \
-_Pragma("unroll")                                                                                    \
-    for (int it = 0; it < ITEMS; ++it) {                                                             \
-      const int r = (it / CBLK) * RPB + lane / LGD;                                                  \
-      const int c = ((it % CBLK) * LGD + lane % LGD) * 8;                                            \
-      const int i = pr0 + r, j0 = wc0 + c;                                                           \
-      const int n = min(8, nrem - c);                                                                \
-      /* diagonal tiles: skip runs below the diagonal; a run inside an 8x8 block on it is full */     \
-      const int kbeg = diag && i - j0 >= 8 ? 8 : 0;                                                  \
-      if (lane_ok && r < rows && c < nrem && kbeg < n) epi.load(b, i, j0, kbeg, n, pre[it]);         \
-    }                                                                                                \
-_Pragma("unroll")                                                                                    \
-    for (int fm = (EFM) + hp * (RPP / MF::MN); fm < (EFM) + (hp + 1) * (RPP / MF::MN); ++fm)         \
-_Pragma("unroll")                                                                                    \
-      for (int fn = 0; fn < FN; ++fn)                                                                \
-_Pragma("unroll")                                                                                    \
-        for (int r = 0; r < MF::NACC; ++r) {                                                         \
-          const int li = (fm - (EFM)) * MF::MN - hp * RPP + MF::row(lane, r);                        \
-          const int lj = fn * MF::MN + MF::col(lane, r);                                             \
-          stg[li * SP + lj] = static_cast<S>(acc[fm][fn][r]);                                        \
-        }                                                                                            \
-    __builtin_amdgcn_s_waitcnt(PTO_LGKM0);                                                           \
-    __builtin_amdgcn_wave_barrier();                                                                 \
-_Pragma("unroll")                                                                                    \
-    for (int it = 0; it < ITEMS; ++it) {                                                             \
-      const int r = (it / CBLK) * RPB + lane / LGD;                                                  \
-      const int c = ((it % CBLK) * LGD + lane % LGD) * 8;                                            \
-      const int i = pr0 + r, j0 = wc0 + c;                                                           \
-      const int n = min(8, nrem - c);                                                                \
-      const int kbeg = diag && i - j0 >= 8 ? 8 : 0;                                                  \
-      if (!(lane_ok && r < rows && c < nrem && kbeg < n)) continue;                                  \
-      /* dk in 1..7: the run crosses the diagonal; its positions k < dk lie below it and take the  \
-         mirrored value, staged at row j0 + k, column i of the same slab (the 16-aligned slab holds \
-         the whole 8-row group; those diagonal-block entries are never written back) */            \
-      S v[8], vo[8];                                                                                 \
-_Pragma("unroll")                                                                                    \
-      for (int k = 0; k < 8; ++k) v[k] = stg[r * SP + c + k];                                        \
-      if (diag && i - j0 > 0) {                                                                      \
-        const int dk = i - j0;                                                                       \
-_Pragma("unroll")                                                                                    \
-        for (int k = 0; k < 7; ++k)                                                                  \
-          if (k < dk) v[k] = stg[(c + k - (pr0 - wc0)) * SP + r + (pr0 - wc0)];                      \
-      }                                                                                              \
-      epi.put(b, i, j0, v, kbeg, n, pre[it], vo);                                                    \
-      if (need_t && !Epi::kVoIsV && !(diag && i - j0 >= 0)) {                                        \
-_Pragma("unroll")                                                                                    \
-        for (int k = 0; k < 8; ++k) stg[r * SP + c + k] = vo[k];                                     \
-      }                                                                                              \
-    }                                                                                                \
-    if (need_t) {                                                                                    \
-      if constexpr (!Epi::kVoIsV) {  /* the write-back above must land first */                      \
-        __builtin_amdgcn_s_waitcnt(PTO_LGKM0);                                                       \
-        __builtin_amdgcn_wave_barrier();                                                             \
-      }                                                                                              \
-  /* output row j = wc0 + c, columns i = pr0 + r..r+7 */                                             \
-      typename Epi::PreT pret[ITEMS_T];                                                              \
-_Pragma("unroll")                                                                                    \
-      for (int it = 0; it < ITEMS_T; ++it) {                                                         \
-        const int c = (it % CBT) * 8 + lane / 8;                                                     \
-        const int r = ((it / CBT) * 8 + lane % 8) * 8;                                               \
-        const int j = wc0 + c, i0 = pr0 + r;                                                         \
-        int n = min(8, rows - r);                                                                    \
-        if (diag && j - i0 < 8) n = 0;  /* below the diagonal, outside its 8x8 blocks */             \
-        if (c < nrem && r < rows && n > 0) epi.load_t(b, j, i0, n, pret[it]);                        \
-      }                                                                                              \
-_Pragma("unroll")                                                                                    \
-      for (int it = 0; it < ITEMS_T; ++it) {                                                         \
-        const int c = (it % CBT) * 8 + lane / 8;                                                     \
-        const int r = ((it / CBT) * 8 + lane % 8) * 8;                                               \
-        const int j = wc0 + c, i0 = pr0 + r;                                                         \
-        int n = min(8, rows - r);                                                                    \
-        if (diag && j - i0 < 8) n = 0;                                                               \
-        if (!(c < nrem && r < rows && n > 0)) continue;                                              \
-        S v[8];                                                                                      \
-_Pragma("unroll")                                                                                    \
-        for (int k = 0; k < 8; ++k) v[k] = k < n ? stg[(r + k) * SP + c] : S(0);                     \
-        epi.put_t(b, j, i0, v, n, pret[it]);                                                         \
-      }                                                                                              \
-    }                                                                                                \
-    __builtin_amdgcn_s_waitcnt(PTO_LGKM0);                                                           \
-    __builtin_amdgcn_wave_barrier();                                                                 \
-  }
   if constexpr (KG == 1) {
-    PTO_STORE_ROWS(0)
+    store_rows<MF, Plan, UPPER, 0>(acc, stg, epi, g, b, wr0, wc0, diag, lane);
   } else {
-    if (kg == 0) {
-      PTO_STORE_ROWS(0)
-    } else {
-      PTO_STORE_ROWS(FM / 2)
-    }
+    if (kg == 0)
+      store_rows<MF, Plan, UPPER, 0>(acc, stg, epi, g, b, wr0, wc0, diag, lane);
+    else
+      store_rows<MF, Plan, UPPER, FM / 2>(acc, stg, epi, g, b, wr0, wc0, diag, lane);
   }
-#undef PTO_STORE_ROWS
   epi.finish(b);
 }
 
@@ -1176,62 +1181,41 @@ int launch_gemm_qn(const GemmArgs& g, const Epi& epi, int batch, hipStream_t str
 //   kVoIsV                               vo is always v (the staged values
 //       then serve the transposed pass as they are);
 //   finish(b)                            once per thread at the end.
-// j0 and i0 are multiples of 8; `vec` (set by the host when the row pitch,
-// batch stride and base allow) enables 16-byte accesses for full runs.
+// j0 and i0 are multiples of 8; full runs use 16-byte accesses at whatever
+// alignment the row has.
 
 struct NoPre {};
 
+// 16 bytes at any element alignment: global_load/store_dwordx4 take any
+// address, so a run of a row whose pitch is no multiple of 16 bytes (a 513- or
+// 2049-wide factor) costs the same instructions as an aligned one. With one
+// access per element such rows waited for eight reads in turn: batched fp32
+// factor update 8 x 1000 x 513 132 -> 114 us, fp32 Gram 8192 x 2049 377 -> 364.
 template <typename T>
-__device__ __forceinline__ bool full_run(bool vec, int kbeg, int n) {
-  return vec && kbeg == 0 && n == 8;
+__device__ __forceinline__ uint4 ld16(const T* p) {
+  uint4 u;
+  __builtin_memcpy(&u, p, sizeof(u));
+  return u;
+}
+template <typename T>
+__device__ __forceinline__ void st16(T* p, const uint4& u) {
+  __builtin_memcpy(p, &u, sizeof(u));
 }
 
-// out[k] = p[k] for k in [kbeg, n)
-template <typename T, typename S>
-__device__ __forceinline__ void ld8(const T* p, S* out, int kbeg, int n, bool vec) {
-  if (full_run<T>(vec, kbeg, n)) {
-    if constexpr (sizeof(T) == 2) {
-      uint4 u = *reinterpret_cast<const uint4*>(p);
-      const T* e = reinterpret_cast<const T*>(&u);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) out[k] = static_cast<S>(to_f(e[k]));
-    } else if constexpr (sizeof(T) == 4) {
-      float4 a = reinterpret_cast<const float4*>(p)[0], c = reinterpret_cast<const float4*>(p)[1];
-      out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
-      out[4] = c.x; out[5] = c.y; out[6] = c.z; out[7] = c.w;
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        double2 d = reinterpret_cast<const double2*>(p)[q];
-        out[2 * q] = static_cast<S>(d.x);
-        out[2 * q + 1] = static_cast<S>(d.y);
-      }
-    }
-  } else {
-    for (int k = kbeg; k < n; ++k) out[k] = static_cast<S>(to_f(p[k]));
-  }
-}
+__device__ __forceinline__ bool full_run(int kbeg, int n) { return kbeg == 0 && n == 8; }
 
 // p[k] = in[k] for k in [kbeg, n), converted to T
 template <typename T, typename S>
-__device__ __forceinline__ void st8(T* p, const S* in, int kbeg, int n, bool vec) {
-  if (full_run<T>(vec, kbeg, n)) {
-    if constexpr (sizeof(T) == 2) {
+__device__ __forceinline__ void st8(T* p, const S* in, int kbeg, int n) {
+  if (full_run(kbeg, n)) {
+    constexpr int E = 16 / (int)sizeof(T);
+#pragma unroll
+    for (int q = 0; q < 8 / E; ++q) {
       uint4 u;
       T* e = reinterpret_cast<T*>(&u);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) e[k] = convert<T>(in[k]);
-      *reinterpret_cast<uint4*>(p) = u;
-    } else if constexpr (sizeof(T) == 4) {
-      reinterpret_cast<float4*>(p)[0] = make_float4(convert<float>(in[0]), convert<float>(in[1]),
-                                                    convert<float>(in[2]), convert<float>(in[3]));
-      reinterpret_cast<float4*>(p)[1] = make_float4(convert<float>(in[4]), convert<float>(in[5]),
-                                                    convert<float>(in[6]), convert<float>(in[7]));
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        reinterpret_cast<double2*>(p)[q] = make_double2(static_cast<double>(in[2 * q]),
-                                                        static_cast<double>(in[2 * q + 1]));
+      for (int k = 0; k < E; ++k) e[k] = convert<T>(in[q * E + k]);
+      st16(p + q * E, u);
     }
   } else {
     for (int k = kbeg; k < n; ++k) p[k] = convert<T>(in[k]);
@@ -1250,10 +1234,10 @@ struct Raw8 {
 // filling single elements of r here would make the compiler split the
 // full-run registers, and so wait for the loads, right after issuing them.
 template <typename T>
-__device__ __forceinline__ void ld8_pre(const T* p, Raw8<T>& r, int kbeg, int n, bool vec) {
-  if (full_run<T>(vec, kbeg, n)) {
+__device__ __forceinline__ void ld8_pre(const T* p, Raw8<T>& r, int kbeg, int n) {
+  if (full_run(kbeg, n)) {
 #pragma unroll
-    for (int q = 0; q < (int)(sizeof(T) / 2); ++q) r.w[q] = reinterpret_cast<const uint4*>(p)[q];
+    for (int q = 0; q < (int)(sizeof(T) / 2); ++q) r.w[q] = ld16(p + q * (16 / (int)sizeof(T)));
   }
 }
 
@@ -1261,8 +1245,8 @@ __device__ __forceinline__ void ld8_pre(const T* p, Raw8<T>& r, int kbeg, int n,
 // unpacking works on whole 32-bit words (a bf16 is the high half of the
 // float with the same value) so the registers stay whole until here.
 template <typename T, typename S>
-__device__ __forceinline__ void ld8_use(const T* p, const Raw8<T>& r, S* out, int kbeg, int n, bool vec) {
-  if (full_run<T>(vec, kbeg, n)) {
+__device__ __forceinline__ void ld8_use(const T* p, const Raw8<T>& r, S* out, int kbeg, int n) {
+  if (full_run(kbeg, n)) {
     if constexpr (sizeof(T) == 2) {
       const unsigned w[4] = {r.w[0].x, r.w[0].y, r.w[0].z, r.w[0].w};
 #pragma unroll
@@ -1290,19 +1274,12 @@ __device__ __forceinline__ void ld8_use(const T* p, const Raw8<T>& r, S* out, in
   }
 }
 
-// Host-side check that a [.., ld] buffer allows 16-byte runs of 8 elements.
-template <typename T>
-inline bool vec_ok(const void* p, int64_t ld, int64_t sb) {
-  return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 8 == 0 && sb % 8 == 0;
-}
-
 // dst = v
 template <typename TO, typename A>
 struct EpiStore {
   typedef A S;
   TO* dst;
   int64_t ld, sd;
-  bool vec;
   typedef NoPre Pre;
   typedef NoPre PreT;
   static constexpr bool kVoIsV = true;
@@ -1310,12 +1287,12 @@ struct EpiStore {
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
   __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
-    st8<TO, S>(dst + (int64_t)b * sd + (int64_t)i * ld + j0, v, kbeg, n, vec);
+    st8<TO, S>(dst + (int64_t)b * sd + (int64_t)i * ld + j0, v, kbeg, n);
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = v[k];
   }
   __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
-    st8<TO, S>(dst + (int64_t)b * sd + (int64_t)j * ld + i0, v, 0, n, vec);
+    st8<TO, S>(dst + (int64_t)b * sd + (int64_t)j * ld + i0, v, 0, n);
   }
   __device__ __forceinline__ void finish(int) const {}
 };
@@ -1327,22 +1304,21 @@ struct EpiBlend {
   TO* dst;
   int64_t ld, sd;
   A beta, alpha;
-  bool vec;
   typedef Raw8<TO> Pre;
   typedef Raw8<TO> PreT;
   static constexpr bool kVoIsV = true;
   __device__ __forceinline__ bool has_t() const { return false; }
   __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
-    if (beta != A(0)) ld8_pre<TO>(dst + (int64_t)b * sd + (int64_t)i * ld + j0, p, kbeg, n, vec);
+    if (beta != A(0)) ld8_pre<TO>(dst + (int64_t)b * sd + (int64_t)i * ld + j0, p, kbeg, n);
   }
   __device__ __forceinline__ void load_t(int b, int j, int i0, int n, PreT& p) const {
-    if (beta != A(0)) ld8_pre<TO>(dst + (int64_t)b * sd + (int64_t)j * ld + i0, p, 0, n, vec);
+    if (beta != A(0)) ld8_pre<TO>(dst + (int64_t)b * sd + (int64_t)j * ld + i0, p, 0, n);
   }
   __device__ __forceinline__ void blend(TO* p, const S* v, int kbeg, int n, const Raw8<TO>& raw) const {
     S r[8];
     if (beta != A(0)) {
       S old[8];
-      ld8_use<TO, S>(p, raw, old, kbeg, n, vec);
+      ld8_use<TO, S>(p, raw, old, kbeg, n);
       // one fixed rounding (an explicit fma), the same in every kernel
       // instantiation that blends (single and batched factor updates)
 #pragma unroll
@@ -1351,7 +1327,7 @@ struct EpiBlend {
 #pragma unroll
       for (int k = 0; k < 8; ++k) r[k] = alpha * v[k];
     }
-    st8<TO, S>(p, r, kbeg, n, vec);
+    st8<TO, S>(p, r, kbeg, n);
   }
   __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre,
                                       S* vo) const {
@@ -1375,11 +1351,10 @@ struct EpiBlendTab {
   TO* dst[kBlendTab];
   int64_t ld;
   A beta, alpha;
-  bool vec;
   typedef Raw8<TO> Pre;
   typedef Raw8<TO> PreT;
   static constexpr bool kVoIsV = true;
-  __device__ __forceinline__ EpiBlend<TO, A> one(int b) const { return EpiBlend<TO, A>{dst[b], ld, 0, beta, alpha, vec}; }
+  __device__ __forceinline__ EpiBlend<TO, A> one(int b) const { return EpiBlend<TO, A>{dst[b], ld, 0, beta, alpha}; }
   __device__ __forceinline__ bool has_t() const { return false; }
   __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
     one(b).load(0, i, j0, kbeg, n, p);

@@ -56,12 +56,12 @@ int kron_t(T* L, T* R, const T* G, int64_t m, int64_t n, double beta2, void* ws,
   const A alpha = beta2 == 1.0 ? A(1) : static_cast<A>(1.0 - beta2);
   {
     GemmArgs g{Grows, ldg, 0, Grows, ldg, 0, (int)m, (int)m, (int)ldn, 0, 0, nullptr};
-    EpiBlend<T, A> e{L, m, 0, beta, alpha, vec_ok<T>(L, m, 0)};
+    EpiBlend<T, A> e{L, m, 0, beta, alpha};
     if (launch_gemm<T, true>(g, e, 1, stream, "kron_left")) return -1;
   }
   {
     GemmArgs g{GT, ldm, 0, GT, ldm, 0, (int)n, (int)n, (int)ldm, 0, 0, nullptr};
-    EpiBlend<T, A> e{R, n, 0, beta, alpha, vec_ok<T>(R, n, 0)};
+    EpiBlend<T, A> e{R, n, 0, beta, alpha};
     if (launch_gemm<T, true>(g, e, 1, stream, "kron_right")) return -1;
   }
   return 0;
@@ -116,11 +116,7 @@ int kron_batched_t(T* const* L, T* const* R, const T* G, int64_t batch, int64_t 
     e.ld = d;
     e.beta = beta;
     e.alpha = alpha;
-    e.vec = true;
-    for (int64_t b = 0; b < batch; ++b) {
-      e.dst[b] = F[b];
-      e.vec = e.vec && vec_ok<T>(F[b], d, 0);
-    }
+    for (int64_t b = 0; b < batch; ++b) e.dst[b] = F[b];
     return e;
   };
   {
@@ -171,7 +167,7 @@ int gram_t(TF* F, const TX* X, int64_t rows, int64_t d, int append_ones, double 
       PTO_REQUIRE((reinterpret_cast<uintptr_t>(X) & 15) == 0,
                   "gram_update_: X must be 16-byte aligned (it is read in place)");
       GemmArgs g{X, d, 0, X, d, 0, (int)dd, (int)dd, (int)rows, 0, 0, nullptr};
-      EpiBlend<TF, A> e{F, dd, 0, static_cast<A>(beta), static_cast<A>(alpha), vec_ok<TF>(F, dd, 0)};
+      EpiBlend<TF, A> e{F, dd, 0, static_cast<A>(beta), static_cast<A>(alpha)};
       return launch_gemm_qn<EpiBlend<TF, A>, true, true>(g, e, 1, stream, "gram_update_direct", tile);
     }
   }
@@ -182,7 +178,7 @@ int gram_t(TF* F, const TX* X, int64_t rows, int64_t d, int append_ones, double 
   if (launch_pack<TX, TX, A>(X, rows, d, d, 0, nullptr, nullptr, 0, 0, XT, ldr, 0, append_ones != 0, 1, stream))
     return -1;
   GemmArgs g{XT, ldr, 0, XT, ldr, 0, (int)dd, (int)dd, (int)ldr, 0, 0, nullptr};
-  EpiBlend<TF, A> e{F, dd, 0, static_cast<A>(beta), static_cast<A>(alpha), vec_ok<TF>(F, dd, 0)};
+  EpiBlend<TF, A> e{F, dd, 0, static_cast<A>(beta), static_cast<A>(alpha)};
   return launch_gemm<TX, true>(g, e, 1, stream, "gram_update");
 }
 

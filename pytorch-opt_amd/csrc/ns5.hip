@@ -49,7 +49,6 @@ struct EpiNsGram {
   T* dst;
   int64_t ld, sd;
   const A* scale;
-  bool vec;
   typedef NoPre Pre;
   typedef NoPre PreT;
   static constexpr bool kVoIsV = true;
@@ -58,14 +57,14 @@ struct EpiNsGram {
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
   __device__ __forceinline__ void store(T* p, int b, const S* v, int kbeg, int n) const {
     if (scale == nullptr) {
-      st8<T, S>(p, v, kbeg, n, vec);
+      st8<T, S>(p, v, kbeg, n);
       return;
     }
     const S s2 = scale[b] * scale[b];
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = s2 * v[k];
-    st8<T, S>(p, w, kbeg, n, vec);
+    st8<T, S>(p, w, kbeg, n);
   }
   __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
     store(dst + (int64_t)b * sd + (int64_t)i * ld + j0, b, v, kbeg, n);
@@ -86,28 +85,27 @@ struct EpiNsSq {
   T* dst;
   int64_t ld, sd;
   A ac, bc, cc;
-  bool vec;
   typedef Raw8<T> Pre;
   typedef NoPre PreT;
   static constexpr bool kVoIsV = false;  // the mirror stores B', not the raw product
   __device__ __forceinline__ bool has_t() const { return false; }
   __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
-    ld8_pre<T>(Asrc + (int64_t)b * sd + (int64_t)i * ld + j0, p, kbeg, n, vec);
+    ld8_pre<T>(Asrc + (int64_t)b * sd + (int64_t)i * ld + j0, p, kbeg, n);
   }
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
   __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre,
                                       S* vo) const {
     const int64_t o = (int64_t)b * sd + (int64_t)i * ld + j0;
     S a[8];
-    ld8_use<T, S>(Asrc + o, pre, a, kbeg, n, vec);
+    ld8_use<T, S>(Asrc + o, pre, a, kbeg, n);
     // explicit fused multiply-adds fix the rounding, so it cannot depend on
     // how the compiler contracts this expression in a given build
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = fma(cc, v[k], fma(bc, a[k], i == j0 + k ? ac : A(0)));
-    st8<T, S>(dst + o, vo, kbeg, n, vec);
+    st8<T, S>(dst + o, vo, kbeg, n);
   }
   __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
-    st8<T, S>(dst + (int64_t)b * sd + (int64_t)j * ld + i0, v, 0, n, vec);
+    st8<T, S>(dst + (int64_t)b * sd + (int64_t)j * ld + i0, v, 0, n);
   }
   __device__ __forceinline__ void finish(int) const {}
 };
@@ -122,7 +120,6 @@ struct EpiNsUpdate {
   int64_t ld_d, s_d;
   T* dstT;
   int64_t ld_t, s_t;
-  bool vec_d, vec_t;
   const A* scale;
   typedef NoPre Pre;
   typedef NoPre PreT;
@@ -130,24 +127,24 @@ struct EpiNsUpdate {
   __device__ __forceinline__ bool has_t() const { return dstT != nullptr; }
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
-  __device__ __forceinline__ void store(T* p, int b, const S* v, int kbeg, int n, bool vec) const {
+  __device__ __forceinline__ void store(T* p, int b, const S* v, int kbeg, int n) const {
     if (scale == nullptr) {
-      st8<T, S>(p, v, kbeg, n, vec);
+      st8<T, S>(p, v, kbeg, n);
       return;
     }
     const S s = scale[b];
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = s * v[k];
-    st8<T, S>(p, w, kbeg, n, vec);
+    st8<T, S>(p, w, kbeg, n);
   }
   __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = v[k];
-    if (dst) store(dst + (int64_t)b * s_d + (int64_t)i * ld_d + j0, b, v, kbeg, n, vec_d);
+    if (dst) store(dst + (int64_t)b * s_d + (int64_t)i * ld_d + j0, b, v, kbeg, n);
   }
   __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
-    store(dstT + (int64_t)b * s_t + (int64_t)j * ld_t + i0, b, v, 0, n, vec_t);
+    store(dstT + (int64_t)b * s_t + (int64_t)j * ld_t + i0, b, v, 0, n);
   }
   __device__ __forceinline__ void finish(int) const {}
 };
@@ -289,14 +286,13 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
     // 1. A = X·Xᵀ
     {
       GemmArgs g{Xc, ldn, sX, Xc, ldn, sX, (int)m, (int)m, (int)ldn, 0, 0, nullptr};
-      EpiNsGram<T, A> e{Ab, ldm, sAB, s0, vec_ok<T>(Ab, ldm, sAB)};
+      EpiNsGram<T, A> e{Ab, ldm, sAB, s0};
       if (launch_gemm<T, true>(g, e, nb, stream, "ns5_gram")) return -1;
     }
     // 2. B' = a·I + b·A + c·A·A
     {
       GemmArgs g{Ab, ldm, sAB, Ab, ldm, sAB, (int)m, (int)m, (int)ldm, 0, 0, nullptr};
-      EpiNsSq<T, A> e{Ab, Bb, ldm, sAB, static_cast<A>(a), static_cast<A>(b), static_cast<A>(c),
-                      vec_ok<T>(Ab, ldm, sAB) && vec_ok<T>(Bb, ldm, sAB)};
+      EpiNsSq<T, A> e{Ab, Bb, ldm, sAB, static_cast<A>(a), static_cast<A>(b), static_cast<A>(c)};
       // A is symmetric: both operands read as its own transpose (PT), on
       // any of the three symmetric tiles; without the transposing reads
       // (fp32, fp64) A's rows are its columns, so the NT launch reads A too
@@ -324,8 +320,6 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
         e.dst = nullptr;
         e.dstT = out; e.ld_t = cols; e.s_t = sG;
       }
-      e.vec_d = e.dst && vec_ok<T>(e.dst, e.ld_d, e.s_d);
-      e.vec_t = e.dstT && vec_ok<T>(e.dstT, e.ld_t, e.s_t);
       if constexpr (QN) {
         // B' is symmetric: read as its own transpose (PT), like X (QN)
         GemmArgs g{Bb, ldm, sAB, Xc, ldn, sX, (int)m, (int)n, (int)ldm, 0, 0, nullptr};

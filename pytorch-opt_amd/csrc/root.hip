@@ -174,7 +174,6 @@ struct EpiMk {
   typename Bits<R>::U* err;
   int err_stride;
   typename Bits<R>::U mx;
-  bool vec;
   typedef NoPre Pre;
   typedef NoPre PreT;
   static constexpr bool kVoIsV = true;
@@ -198,8 +197,8 @@ struct EpiMk {
         mx = u > mx ? u : mx;
       }
     }
-    st8<R, R>(Mk + o, v, kbeg, n, vec);
-    st8<R, R>(Mi + o, mi, kbeg, n, vec);
+    st8<R, R>(Mk + o, v, kbeg, n);
+    st8<R, R>(Mi + o, mi, kbeg, n);
   }
   __device__ __forceinline__ void put(int b, int i, int j0, const R* v, int kbeg, int n, const Pre&, R* vo) {
     run(b, i, j0, v, kbeg, n);
@@ -456,7 +455,7 @@ int root_t(const TI* A, TI* out, int64_t batch, int64_t n, int64_t p, double dam
   // product is symmetric too, computed on upper tiles and mirrored.
   auto product = [&](const R* P, const R* Q, R* dst, bool upper, const char* name) -> int {
     GemmArgs g{P, ld, sb, Q, ld, sb, (int)n, (int)n, (int)ld, 0, 0, guard, guard_stride};
-    EpiStore<R, R> e{dst, ld, sb, vec_ok<R>(dst, ld, sb)};
+    EpiStore<R, R> e{dst, ld, sb};
     if (upper) return launch_gemm<R, true, EpiStore<R, R>, true>(g, e, nb, stream, name);
     return launch_gemm<R, false, EpiStore<R, R>, true>(g, e, nb, stream, name);
   };
@@ -469,7 +468,7 @@ int root_t(const TI* A, TI* out, int64_t batch, int64_t n, int64_t p, double dam
   const bool pair = nb == 1 && p >= 2;
   // The first launch of iteration it >= 1 decides iteration it - 1 itself.
   auto decider = [&](int it, R* dst, int64_t sd, bool per_matrix) {
-    return EpiStoreDecide<R>{{dst, ld, sd, vec_ok<R>(dst, ld, sd)},
+    return EpiStoreDecide<R>{{dst, ld, sd},
                              slot(it - 2),
                              slot(it - 1),
                              err + (int64_t)(it - 1) * (each ? nb : 1) * kErrSub,
@@ -485,7 +484,7 @@ int root_t(const TI* A, TI* out, int64_t batch, int64_t n, int64_t p, double dam
       g.guard = nullptr;
       return launch_gemm<R, true, EpiStoreDecide<R>, true>(g, decider(it, d0, sd, false), 2, stream, name);
     }
-    EpiStore<R, R> e{d0, ld, sd, vec_ok<R>(d0, ld, sd)};
+    EpiStore<R, R> e{d0, ld, sd};
     return launch_gemm<R, true, EpiStore<R, R>, true>(g, e, 2, stream, name);
   };
 
@@ -555,7 +554,7 @@ int root_t(const TI* A, TI* out, int64_t batch, int64_t n, int64_t p, double dam
     {
       GemmArgs g{S, ld, sb, Mk[cur], ld, sb, (int)n, (int)n, (int)ld, 0, 0, guard, guard_stride};
       EpiMk<R> e{Mk[nxt], Mi[nxt], ld, sb, c1, alpha,
-                 reinterpret_cast<U*>(err + (int64_t)it * (each ? nb : 1) * kErrSub), each ? kErrSub : 0, U(0), vec_ok<R>(Mk[nxt], ld, sb) && vec_ok<R>(Mi[nxt], ld, sb)};
+                 reinterpret_cast<U*>(err + (int64_t)it * (each ? nb : 1) * kErrSub), each ? kErrSub : 0, U(0)};
       if (launch_gemm<R, true, EpiMk<R>, true>(g, e, nb, stream, "root_mk")) return -1;
     }
     return 0;
