@@ -38,6 +38,23 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
+// fp32 operands as pairs of fp16 ("split"): x·2^-e = h + l with h = fp16(x·2^-e)
+// and l = fp16(x·2^-e - h), held as two planes of the same layout, l's at
+// GemmArgs::pP (pQ) elements from h's. e is an exponent per row of the
+// operand (or one per matrix) that puts the row's largest value at 2^13..2^14,
+// so h + l keeps 22-24 bits of every value down to 2^-16 of that largest one
+// and 2^-39 of it below. A product is h·h + h·l + l·h in fp32 accumulators
+// (l·l is below 2^-24 of h·h), in 3/16 of the fp32 MFMA's time. That one
+// rounds its accumulator after every k; the fp16 one after every eight (its
+// products are exact, and subnormal operands are kept), so the errors come out
+// below those of the fp32 MFMA: fp32 NS5 12 x 2048² 2.7e-6 against 4.2e-6 of
+// the exact result, at 16.3 -> 5.4 ms (126 -> 380 TFLOP/s; 256² tiles of the
+// update sustain 467, the MFMAs 56% of the time busy).
+struct sp16 {
+  _Float16 v;
+};
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
 // Per element type: which MFMA, its fragment shapes and output lane map.
 //   MN  : output block is MN x MN
 //   KPL : consecutive k values one lane feeds per instruction
@@ -58,6 +75,19 @@ struct Mfma<bf16> {  // v_mfma_f32_16x16x32_bf16
   __device__ static __forceinline__ cvec_t mma(const uint4& a, const uint4& b, int, cvec_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
                                                    __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
+  __device__ static __forceinline__ int row(int lane, int r) { return (lane >> 4) * 4 + r; }
+  __device__ static __forceinline__ int col(int lane, int) { return lane & 15; }
+};
+
+template <>
+struct Mfma<sp16> {  // v_mfma_f32_16x16x32_f16, the bf16 shape's lane maps
+  typedef float acc_t;
+  typedef f32x4_t cvec_t;
+  static constexpr int MN = 16, KPL = 8, G = 4, NACC = 4;
+  __device__ static __forceinline__ cvec_t mma(const uint4& a, const uint4& b, int, cvec_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
+                                                  0, 0);
   }
   __device__ static __forceinline__ int row(int lane, int r) { return (lane >> 4) * 4 + r; }
   __device__ static __forceinline__ int col(int lane, int) { return lane & 15; }
@@ -123,6 +153,7 @@ struct GemmArgs {
   const int* guard;  // if non-null and guard[b * guard_stride] != 0, matrix b is skipped
   int guard_stride;  // ints between the guard words of consecutive matrices (0: one word)
   int cus;           // compute units of the device (set by the launcher)
+  int64_t pP = 0, pQ = 0;  // split operands: elements from the h plane to the l plane
 };
 
 // Workgroups are dispatched to the 8 XCDs round-robin by linear id, each
@@ -489,17 +520,20 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
   constexpr int PRB = PT ? BM * (int)sizeof(T) : kRowBytes;  // bytes per P row in LDS
   constexpr int CPRP = PRB / 16;                   // 16-byte chunks per P row
   static_assert((BM + BN) % (16 * NW) == 0 && IPW >= 1, "DMA split");
-  static_assert(!PT || (QN && CPRP >= 16 && (PRB % 256 == 0 || PRB % 256 == 128)),
+  static_assert(!PT || (QN && CPRP >= 8 && (PRB % 256 == 0 || PRB % 256 == 128)),
                 "PT layout: with QN, P rows of 256·k or 256·k + 128 bytes");
   static_assert(WTM % MF::MN == 0 && WTN % MF::MN == 0 && WTM % 16 == 0, "wave tile");
   static_assert(KSPAN % VEC == 0 && NRG >= 1, "fragment runs");
   constexpr int NS = Cfg::NS;
+  // split operands: K tile t is the h (t even) or l plane's tile t / 2
+  constexpr bool kSplit = std::is_same<T, sp16>::value;
+  static_assert(!kSplit || (Cfg::KG == 1 && NRG == 1 && IPR == 1), "split: one K group, one MFMA per fragment");
   static_assert((NS - 2) * IPW <= 63, "vmcnt range");
   static_assert(Plan::RPP % MF::MN == 0 && Plan::WTE % Plan::RPP == 0, "epilogue passes");
   constexpr int KG = Cfg::KG, NWG = Cfg::WM * Cfg::WN;  // K groups, waves per group
   static_assert(KG == 1 || (FM % 2 == 0 && Plan::WTE % MF::MN == 0), "K groups: halves of whole fragments");
   static_assert(Cfg::NS * Plan::ARR <= Plan::kLdsMax, "LDS budget");
-  static_assert(!QN || (sizeof(T) == 2 && (!UPPER || PT) && CPR >= 16 && (QRB % 256 == 0 || QRB % 256 == 128) &&
+  static_assert(!QN || (sizeof(T) == 2 && (!UPPER || PT) && CPR >= 8 && (QRB % 256 == 0 || QRB % 256 == 128) &&
                         (BM * kRowBytes) % 1024 == 0 && NRG == 1),
                 "QN layout: bf16, Q rows of 256·k or 256·k + 128 bytes; symmetric products only with PT");
 
@@ -558,6 +592,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
   // (rows of PRB bytes, columns from row0).
   const char* src[IPW];
   unsigned step[IPW];  // bytes between consecutive K tiles (the launcher bounds it)
+  int64_t plane[IPW];  // split: bytes from the h plane to the l plane
   int dst_off[IPW];
 #pragma unroll
   for (int q = 0; q < IPW; ++q) {
@@ -588,13 +623,16 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
       step[q] = (unsigned)(kRowBytes * g.ldq);
     }
     src[q] = reinterpret_cast<const char*>(s);
+    if constexpr (kSplit) plane[q] = (R0 < BM ? g.pP : g.pQ) * (int64_t)sizeof(T);
     dst_off[q] = R0 * kRowBytes;
   }
   auto issue = [&](int kt, char* stage) {
 #pragma unroll
-    for (int q = 0; q < IPW; ++q)
-      __builtin_amdgcn_global_load_lds((gbl_void_t*)(src[q] + (uint64_t)(unsigned)kt * step[q]),
-                                       (lds_void_t*)(stage + dst_off[q]), 16, 0, 0);
+    for (int q = 0; q < IPW; ++q) {
+      uint64_t off = (uint64_t)(unsigned)kt * step[q];
+      if constexpr (kSplit) off = (uint64_t)(unsigned)(kt >> 1) * step[q] + ((kt & 1) ? plane[q] : 0);
+      __builtin_amdgcn_global_load_lds((gbl_void_t*)(src[q] + off), (lds_void_t*)(stage + dst_off[q]), 16, 0, 0);
+    }
   };
 
   cvec_t acc[FM][FN];
@@ -641,41 +679,38 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
   // between the MFMA groups (measured faster for the QN layout, slower for
   // the symmetric K-contiguous products).
   constexpr bool kSpreadReads = QN;
+  auto load_a = [&](const char* stage, int rg, int fm) -> uint4 {
+    if constexpr (PT) {
+      const char* Ps = stage + 8 * rg * PRB;
+      v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Ps + poff[fm]));
+      v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Ps + poff[fm] + 4 * PRB));
+      uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+      return make_uint4(l2.x, l2.y, h2.x, h2.y);
+    } else {
+      const char* Pw = stage + (wm * WTM + lr) * kRowBytes;
+      return *reinterpret_cast<const uint4*>(Pw + fm * MF::MN * kRowBytes + ((lg * NRG + rg) ^ sw) * 16);
+    }
+  };
+  auto load_b = [&](const char* stage, int rg, int fn) -> uint4 {
+    if constexpr (QN) {
+      // lanes of k-group lg, step rg: k = KSPAN*lg + 8*rg + 0..7
+      const char* Qs = stage + BM * kRowBytes + 8 * rg * QRB;
+      v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Qs + qoff[fn]));
+      v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Qs + qoff[fn] + 4 * QRB));
+      uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+      return make_uint4(l2.x, l2.y, h2.x, h2.y);
+    } else {
+      const char* Qw = stage + (BM + wn * WTN + lr) * kRowBytes;
+      return *reinterpret_cast<const uint4*>(Qw + fn * MF::MN * kRowBytes + ((lg * NRG + rg) ^ sw) * 16);
+    }
+  };
   auto load_frags = [&](const char* stage, Frag& f) {
-    const char* Pw = stage + (wm * WTM + lr) * kRowBytes;
 #pragma unroll
     for (int rg = 0; rg < NRG; ++rg) {
-      const int off = ((lg * NRG + rg) ^ sw) * 16;
-      if constexpr (PT) {
-        const char* Ps = stage + 8 * rg * PRB;
 #pragma unroll
-        for (int fm = 0; fm < FM; ++fm) {
-          v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Ps + poff[fm]));
-          v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Ps + poff[fm] + 4 * PRB));
-          uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-          f.a[rg][fm] = make_uint4(l2.x, l2.y, h2.x, h2.y);
-        }
-      } else {
+      for (int fm = 0; fm < FM; ++fm) f.a[rg][fm] = load_a(stage, rg, fm);
 #pragma unroll
-        for (int fm = 0; fm < FM; ++fm)
-          f.a[rg][fm] = *reinterpret_cast<const uint4*>(Pw + fm * MF::MN * kRowBytes + off);
-      }
-      if constexpr (QN) {
-        // lanes of k-group lg, step rg: k = KSPAN*lg + 8*rg + 0..7
-        const char* Qs = stage + BM * kRowBytes + 8 * rg * QRB;
-#pragma unroll
-        for (int fn = 0; fn < FN; ++fn) {
-          v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Qs + qoff[fn]));
-          v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(Qs + qoff[fn] + 4 * QRB));
-          uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-          f.b[rg][fn] = make_uint4(l2.x, l2.y, h2.x, h2.y);
-        }
-      } else {
-        const char* Qw = stage + (BM + wn * WTN + lr) * kRowBytes;
-#pragma unroll
-        for (int fn = 0; fn < FN; ++fn)
-          f.b[rg][fn] = *reinterpret_cast<const uint4*>(Qw + fn * MF::MN * kRowBytes + off);
-      }
+      for (int fn = 0; fn < FN; ++fn) f.b[rg][fn] = load_b(stage, rg, fn);
     }
   };
   // COMP (fp32 only): blocked accumulation. gfx950's fp32 MFMA rounds
@@ -721,6 +756,52 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
     }
   };
 
+  // Split operands, plain (COMP false): the h tile's products (mma), then with
+  // the l tile of the same k in hand the two cross products, all into the
+  // accumulator. The MFMA rounds that after every eight k, twelve times per K
+  // block of 32.
+  auto mma_cross = [&](const Frag& h, const Frag& l) {
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = MF::mma(h.a[0][fm], l.b[0][fn], 0, acc[fm][fn]);
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = MF::mma(l.a[0][fm], h.b[0][fn], 0, acc[fm][fn]);
+  };
+  // Split operands, COMP: the three products of a K block, small terms first,
+  // summed apart for fragment rows [F0, F0 + NF) and added to the accumulator
+  // once (each row's adds beside the next row's MFMAs). The plain form's twelve
+  // roundings per block are fewer than the fp32 MFMA's 32, but those of its
+  // cross products repeat on the diagonal of a Gram: 3.8e-7 against the fp32
+  // MFMA's 1.6e-7 on a 257-deep one, 1.2e-7 this way, and below it at every
+  // depth. 10-20% slower; the factor updates use it, the orthogonalisation
+  // (whose errors are below the fp32 chain's either way) does not.
+  constexpr bool kBlockSums = COMP && kSplit;
+  auto mma_split = [&](const uint4* ha, const uint4* la, const uint4* hb, const uint4* lb, auto first, auto count) {
+    constexpr int F0 = decltype(first)::value, NF = decltype(count)::value;
+    cvec_t t[2][FN];
+    auto add = [&](int fm) {
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int r = 0; r < MF::NACC; ++r) acc[F0 + fm][fn][r] += t[fm & 1][fn][r];
+    };
+#pragma unroll
+    for (int fm = 0; fm < NF; ++fm) {
+      cvec_t* u = t[fm & 1];
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn) u[fn] = MF::mma(ha[fm], lb[fn], 0, cvec_t{0, 0, 0, 0});
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn) u[fn] = MF::mma(la[fm], hb[fn], 0, u[fn]);
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn) u[fn] = MF::mma(ha[fm], hb[fn], 0, u[fn]);
+      if (fm > 0) add(fm - 1);
+    }
+    add(NF - 1);
+  };
+
   // Skewed pipeline: during step s the wave issues the LDS reads of tile
   // s+1 into one register set, then the MFMAs of tile s from the other set
   // (read during step s-1), with the DMA of tile s+NS-1 spread between
@@ -732,7 +813,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
   // outstanding). The launchers require K to be a multiple of NS tiles, so
   // every step of the unrolled group is a real one and the MFMAs need no
   // branch.
-  const int KT = g.K / BK;
+  const int KT = (kSplit ? 2 : 1) * (g.K / BK);
   if constexpr (KG == 2) {
     // K groups: waves 0..NWG-1 (group 0) take the even K tiles, the others
     // the odd ones, each group accumulating the whole tile in its own
@@ -792,6 +873,71 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
       __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));
       stage_barrier();
     }
+  } else if constexpr (Cfg::PP && kBlockSums) {
+    // The ping-pong schedule below over K blocks (an h and an l tile each, two
+    // blocks in the ring), with the wave's fragment rows in two halves so that
+    // both planes' fragments fit the registers beside the accumulators:
+    //   R1: LDS reads of both planes' Q fragments and half the P fragments of
+    //       block p, DMA of block p+1 into the stages of p-1;   M1: their MFMAs;
+    //   R2: reads of the other P fragments;   M2: their MFMAs.
+    // Group 1 runs one phase behind. Block p-1 was last read in R2(p-1), which
+    // group 1 ends before group 0's R1(p); every wave waits for its part of
+    // block p+1 at the end of R2(p), before either group's R1(p+1).
+    if (KT > 0) {
+      static_assert(FM % 2 == 0, "halves of the fragment rows");
+      constexpr int HM = FM / 2;
+      const int grp = wm;
+      uint4 ha[HM], la[HM], hb[FN], lb[FN];
+      issue(0, st0);
+      issue(1, st1);
+      __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));
+      stage_barrier();
+      if (grp) {
+        __builtin_amdgcn_sched_barrier(0);
+        stage_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      constexpr std::integral_constant<int, HM> half{};
+      for (int kt = 0; kt < KT; kt += kStages) {
+#define PTO_PHASE_END()                                       \
+  __builtin_amdgcn_sched_barrier(0);                          \
+  stage_barrier();                                            \
+  __builtin_amdgcn_sched_barrier(0);
+#define PTO_BLOCK(J, H, L, DH, DL)                            \
+  if (!idle) {                                                \
+    _Pragma("unroll") for (int x = 0; x < FN; ++x) {          \
+      hb[x] = load_b(H, 0, x);                                \
+      lb[x] = load_b(L, 0, x);                                \
+    }                                                         \
+    _Pragma("unroll") for (int x = 0; x < HM; ++x) {          \
+      ha[x] = load_a(H, 0, x);                                \
+      la[x] = load_a(L, 0, x);                                \
+    }                                                         \
+  }                                                           \
+  issue(min(kt + (J) + 2, KT - 2), DH);                       \
+  issue(min(kt + (J) + 3, KT - 1), DL);                       \
+  PTO_PHASE_END()                                             \
+  if (!idle) mma_split(ha, la, hb, lb, std::integral_constant<int, 0>{}, half); \
+  PTO_PHASE_END()                                             \
+  if (!idle) {                                                \
+    _Pragma("unroll") for (int x = 0; x < HM; ++x) {          \
+      ha[x] = load_a(H, 0, HM + x);                           \
+      la[x] = load_a(L, 0, HM + x);                           \
+    }                                                         \
+  }                                                           \
+  __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));                   \
+  PTO_PHASE_END()                                             \
+  if (!idle) mma_split(ha, la, hb, lb, half, half);           \
+  PTO_PHASE_END()
+        PTO_BLOCK(0, st0, st1, st2, st3)
+        PTO_BLOCK(2, st2, st3, st0, st1)
+#undef PTO_BLOCK
+#undef PTO_PHASE_END
+      }
+      if (!grp) stage_barrier();
+      __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));
+      stage_barrier();
+    }
   } else if constexpr (Cfg::PP) {
     // Ping-pong: waves 0-3 (group 0) and 4-7 (group 1), one of each per
     // SIMD, run the same sequence of phases, group 1 one phase behind:
@@ -807,7 +953,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
     // apart). Both groups execute 2·KT + 3 barriers.
     if (KT > 0) {
       const int grp = wm;
-      Frag f;
+      Frag f, fl;  // fl: split operands' l tile beside f's h
       issue(0, st0);
       issue(min(1, KT - 1), st1);
       issue(min(2, KT - 1), st2);
@@ -820,13 +966,18 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
       }
       for (int kt = 0; kt < KT; kt += kStages) {
 #define PTO_PP(J, RD, DMA)                                    \
-  if (!idle) load_frags(RD, f);                               \
+  if (!idle) load_frags(RD, kSplit && ((J) & 1) ? fl : f);    \
   issue(min(kt + (J) + 3, KT - 1), DMA);                      \
   __builtin_amdgcn_s_waitcnt(PTO_VMCNT(2 * IPW));             \
   __builtin_amdgcn_sched_barrier(0);                          \
   stage_barrier();                                            \
   __builtin_amdgcn_sched_barrier(0);                          \
-  if (!idle) mma(f);                                          \
+  if (!idle) {                                                \
+    if constexpr (kSplit && ((J) & 1))                        \
+      mma_cross(f, fl);                                       \
+    else                                                      \
+      mma(f);                                                 \
+  }                                                           \
   __builtin_amdgcn_s_waitcnt(PTO_VMCNT(2 * IPW));             \
   __builtin_amdgcn_sched_barrier(0);                          \
   stage_barrier();                                            \
@@ -839,6 +990,119 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
       }
       if (!grp) stage_barrier();
       __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));
+      stage_barrier();
+    }
+  } else if constexpr (kBlockSums) {
+    // The skewed pipeline over h, l, h, l, ... tiles, one block (two tiles)
+    // further ahead: during step s the wave reads tile s+2 (s even: the next
+    // block's h, s odd: its l) while it issues the MFMAs of half the fragment
+    // rows of the block whose planes it holds, and the DMA of tile s+NS into
+    // the stage of tile s (read in step s-2).
+    if (KT > 0) {
+      static_assert(FM % 2 == 0, "halves of the fragment rows");
+      constexpr int HM = FM / 2;
+      Frag h0, l0, h1, l1;
+      issue(0, st0);
+      issue(1, st1);
+      issue(2, st2);
+      issue(3, st3);
+      if constexpr (NS == 8) {
+        issue(min(4, KT - 1), st4);
+        issue(min(5, KT - 1), st5);
+        issue(min(6, KT - 1), st6);
+        issue(min(7, KT - 1), st7);
+      }
+      __builtin_amdgcn_s_waitcnt(PTO_VMCNT((NS - 2) * IPW));
+      stage_barrier();
+      load_frags(st0, h0);
+      load_frags(st1, l0);
+      constexpr std::integral_constant<int, HM> half{};
+      constexpr std::integral_constant<int, 0> none{};
+      for (int kt = 0; kt < KT; kt += NS) {
+#define PTO_STEP(J, H, L, PART, NXT, RD, DMA)                         \
+  __builtin_amdgcn_s_waitcnt(PTO_VMCNT((NS - 3) * IPW));              \
+  stage_barrier();                                                    \
+  load_frags(RD, NXT);                                                \
+  issue(min(kt + (J) + NS, KT - 1), DMA);                             \
+  mma_split(H.a[0] + (PART), L.a[0] + (PART), H.b[0], L.b[0], PART, half); \
+  for (int q = 0; q < IPW; ++q) {                                     \
+    __builtin_amdgcn_sched_group_barrier(0x100, kFragReads / IPW, 0); \
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                \
+    __builtin_amdgcn_sched_group_barrier(0x008, 3 * HM * FN / IPW, 0); \
+  }
+        PTO_STEP(0, h0, l0, none, h1, st2, st0)
+        PTO_STEP(1, h0, l0, half, l1, st3, st1)
+        if constexpr (NS == 4) {
+          PTO_STEP(2, h1, l1, none, h0, st0, st2)
+          PTO_STEP(3, h1, l1, half, l0, st1, st3)
+        } else {
+          PTO_STEP(2, h1, l1, none, h0, st4, st2)
+          PTO_STEP(3, h1, l1, half, l0, st5, st3)
+          PTO_STEP(4, h0, l0, none, h1, st6, st4)
+          PTO_STEP(5, h0, l0, half, l1, st7, st5)
+          PTO_STEP(6, h1, l1, none, h0, st0, st6)
+          PTO_STEP(7, h1, l1, half, l0, st1, st7)
+        }
+#undef PTO_STEP
+      }
+      __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));  // stray prefetches land before reuse
+      stage_barrier();
+    }
+  } else if constexpr (kSplit) {
+    // The skewed pipeline below over h, l, h, l, ... tiles: an h step issues
+    // h·h (from f0 or f1, alternating) and reads l, an l step the cross
+    // products and reads the next h into the other set.
+    if (KT > 0) {
+      Frag f0, f1, fl;
+      issue(0, st0);
+      issue(1, st1);
+      issue(2, st2);
+      if constexpr (NS == 8) {
+        issue(3, st3);
+        issue(min(4, KT - 1), st4);
+        issue(min(5, KT - 1), st5);
+        issue(min(6, KT - 1), st6);
+      }
+      __builtin_amdgcn_s_waitcnt(PTO_VMCNT((NS - 2) * IPW));
+      stage_barrier();
+      load_frags(st0, f0);
+      for (int kt = 0; kt < KT; kt += NS) {
+#define PTO_STEP(J, READ, RD, DMA, MMA, COUNT)                        \
+  __builtin_amdgcn_s_waitcnt(PTO_VMCNT((NS - 3) * IPW));              \
+  stage_barrier();                                                    \
+  load_frags(RD, READ);                                               \
+  issue(min(kt + (J) + NS - 1, KT - 1), DMA);                         \
+  MMA;                                                                \
+  if constexpr (!kSpreadReads)                                        \
+    __builtin_amdgcn_sched_group_barrier(0x100, kFragReads, 0);       \
+  for (int q = 0; q < IPW; ++q) {                                     \
+    if constexpr (kSpreadReads)                                       \
+      __builtin_amdgcn_sched_group_barrier(0x100, kFragReads / IPW, 0); \
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                \
+    __builtin_amdgcn_sched_group_barrier(0x008, (COUNT) / IPW, 0);    \
+  }
+#define PTO_STEP_H(J, CUR, RD, DMA) PTO_STEP(J, fl, RD, DMA, mma(CUR), kTileMfma)
+#define PTO_STEP_L(J, CUR, NXT, RD, DMA) PTO_STEP(J, NXT, RD, DMA, mma_cross(CUR, fl), 2 * kTileMfma)
+        if constexpr (NS == 4) {
+          PTO_STEP_H(0, f0, st1, st3)
+          PTO_STEP_L(1, f0, f1, st2, st0)
+          PTO_STEP_H(2, f1, st3, st1)
+          PTO_STEP_L(3, f1, f0, st0, st2)
+        } else {
+          PTO_STEP_H(0, f0, st1, st7)
+          PTO_STEP_L(1, f0, f1, st2, st0)
+          PTO_STEP_H(2, f1, st3, st1)
+          PTO_STEP_L(3, f1, f0, st4, st2)
+          PTO_STEP_H(4, f0, st5, st3)
+          PTO_STEP_L(5, f0, f1, st6, st4)
+          PTO_STEP_H(6, f1, st7, st5)
+          PTO_STEP_L(7, f1, f0, st0, st6)
+        }
+#undef PTO_STEP_H
+#undef PTO_STEP_L
+#undef PTO_STEP
+      }
+      __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));  // stray prefetches land before reuse
       stage_barrier();
     }
   } else if (KT > 0) {
@@ -975,6 +1239,28 @@ struct TileSet<bf16> {
   static constexpr double kMidRate = 1.35;
   static constexpr double kTinyRate = 0.0;
 };
+// Split operands: the bf16 tiles' schedules, with three MFMAs per fragment
+// pair. The 192² tile is a ping-pong one (not K groups), so that every tile
+// sums a position's products in the same order (batched and single calls
+// give the same bits), and full products use it too. The 128² tile has eight
+// waves of 64 x 32 (four of 64 x 64 left the 2048² products 10-25% slower);
+// the 64² tile keeps small products on the CUs. Rates from forcing each tile
+// on 17 shapes: one K = 1024 tile takes a CU 66 us at 256², 44 at 192², 26-27
+// at 128² and 10.4 at 64², but never less than 15.5 at 64² (its chain of
+// loads), which kTinyFloor says in the units of pick_tile's loads.
+template <>
+struct TileSet<sp16> {
+  typedef Tile<256, 256, 32, 2, 4, 4, true> big;
+  typedef Tile<128, 128, 32, 2, 4> small;
+  typedef big sym_big;
+  typedef small sym_small;
+  typedef Tile<192, 192, 32, 2, 4, 4, true> sym_mid;
+  typedef Tile<64, 64, 32, 2, 2, 8> sym_tiny;
+  static constexpr bool kHasMid = true, kHasTiny = true, kMidAll = true;
+  static constexpr double kBigRate = 1.67;
+  static constexpr double kMidRate = 1.41;
+  static constexpr double kTinyRate = 0.66;
+};
 // fp32 symmetric products also have a 32 x 32 "tiny" tile (4 waves of
 // 16 x 16): an n = 1024 product is 136 upper tiles of 64² (120 of 256 CUs
 // idle) but 528 of 32², about two co-resident workgroups per CU.
@@ -1021,9 +1307,10 @@ constexpr int ring_k() {
                 S::sym_small::NS * S::sym_small::BK, S::sym_mid::NS * S::sym_mid::BK,
                 S::sym_tiny::NS * S::sym_tiny::BK})
     r = v > r ? v : r;
-  return r;
+  return std::is_same<T, sp16>::value ? r / 2 : r;  // split: every K block is two ring tiles, h and l
 }
-static_assert(kPadK % ring_k<bf16>() == 0 && kPadK % ring_k<float>() == 0 && kPadK % ring_k<double>() == 0,
+static_assert(kPadK % ring_k<bf16>() == 0 && kPadK % ring_k<float>() == 0 && kPadK % ring_k<double>() == 0 &&
+                  kPadK % ring_k<sp16>() == 0,
               "padded K covers every ring");
 
 // Compute units of the current device (256 on a full MI355X), cached per
@@ -1074,6 +1361,11 @@ struct PickTiles<T, true> {
 // type's kMidAll). At the same number of tiles per CU the big tile wins; a
 // big tiling that leaves half the CUs idle (e.g. 64 big tiles against 256
 // small ones) loses. Returns 0 = small, 1 = big, 2 = mid, 3 = tiny.
+template <typename T>
+constexpr bool tiny_all() {  // the tiny tile serves full products too
+  return std::is_same<T, sp16>::value;
+}
+constexpr double kTinyFloor = 9200;  // split operands' 64² tile
 template <typename T, bool UPPER>
 int pick_tile(int64_t M, int64_t N, int64_t batch) {
   typedef typename PickTiles<T, UPPER>::Big Big;
@@ -1096,9 +1388,11 @@ int pick_tile(int64_t M, int64_t N, int64_t batch) {
     best = load(Mid::BM, Mid::BN, TileSet<T>::kMidRate);
     pick = 2;
   }
-  if (UPPER && TileSet<T>::kHasTiny) {
+  if ((UPPER || tiny_all<T>()) && TileSet<T>::kHasTiny) {
     typedef typename TileSet<T>::sym_tiny Tiny;
-    if (load(Tiny::BM, Tiny::BN, TileSet<T>::kTinyRate) < best) pick = 3;
+    double tiny = load(Tiny::BM, Tiny::BN, TileSet<T>::kTinyRate);
+    if (std::is_same<T, sp16>::value && tiny < kTinyFloor) tiny = kTinyFloor;
+    if (tiny < best) pick = 3;
   }
   return pick;
 }
@@ -1123,7 +1417,7 @@ int launch_gemm(const GemmArgs& g, const Epi& epi, int batch, hipStream_t stream
     static_assert(Mid::BM == Mid::BN && Mid::BK == Big::BK, "mid tile: square, same K tile");
     if (pick == 2) return launch_gemm_cfg<T, Mid, UPPER, Epi, false, false, COMP>(g, epi, batch, stream, name);
   }
-  if constexpr (UPPER && TileSet<T>::kHasTiny) {
+  if constexpr ((UPPER || tiny_all<T>()) && TileSet<T>::kHasTiny) {
     typedef typename TileSet<T>::sym_tiny Tiny;
     static_assert(Tiny::BM == Tiny::BN && Tiny::BK == Big::BK, "tiny tile: square, same K tile");
     if (pick == 3) return launch_gemm_cfg<T, Tiny, UPPER, Epi, false, false, COMP>(g, epi, batch, stream, name);
@@ -1133,37 +1427,41 @@ int launch_gemm(const GemmArgs& g, const Epi& epi, int batch, hipStream_t stream
 }
 
 // C[b](i,j) = sum_k P[b](i,k) * Q[b](k,j) with Q stored [K][N] (row pitch
-// ldq, N contiguous), bf16 only. Q must hold K rows of ldq elements, and
+// ldq, N contiguous), bf16 and split operands only. Q must hold K rows of ldq elements, and
 // its rows past the true contraction length must be zero (as the pad
 // columns of P are). With PT, P is stored [K][M] as well (row pitch ldp,
 // ldp >= M, K rows, the rows past the true K zero) — for a symmetric P
 // that is P itself. UPPER (with PT): a symmetric product on upper tiles,
 // mirrored, as in launch_gemm.
 // pick: the tile (pick_tile's codes), or -1 to let pick_tile choose.
-template <class Epi, bool PT = false, bool UPPER = false>
+template <class Epi, bool PT = false, bool UPPER = false, typename T = bf16>
 int launch_gemm_qn(const GemmArgs& g, const Epi& epi, int batch, hipStream_t stream, const char* name,
                    int pick = -1) {
   static_assert(PT || !UPPER, "symmetric QN products need PT");
-  typedef typename PickTiles<bf16, UPPER>::Big Big;
-  typedef typename PickTiles<bf16, UPPER>::Small Small;
+  typedef typename PickTiles<T, UPPER>::Big Big;
+  typedef typename PickTiles<T, UPPER>::Small Small;
   PTO_REQUIRE(g.M >= 0 && g.N >= 0 && g.K >= 0, std::string(name) + ": negative extent");
   PTO_REQUIRE(!UPPER || g.M == g.N, std::string(name) + ": symmetric product needs M == N");
-  PTO_REQUIRE(g.K % ring_k<bf16>() == 0, std::string(name) + ": K not padded");
+  PTO_REQUIRE(g.K % ring_k<T>() == 0, std::string(name) + ": K not padded");
   PTO_REQUIRE(g.ldq < (int64_t(1) << 26) && g.ldp < (int64_t(1) << 26),
               std::string(name) + ": row pitch too large");  // 64-byte K steps in 32 bits
   PTO_REQUIRE(g.ldp % 8 == 0 && g.ldq % 8 == 0 && g.ldq >= g.N && g.ldq >= 8 && (!PT || (g.ldp >= g.M && g.ldp >= 8)) &&
                   (reinterpret_cast<uintptr_t>(g.P) & 15) == 0 && (reinterpret_cast<uintptr_t>(g.Q) & 15) == 0,
               std::string(name) + ": operands not 16-byte aligned");
-  PTO_REQUIRE(pick >= -1 && pick <= 2 && (UPPER || pick != 2), std::string(name) + ": tile choice");
-  if (pick < 0) pick = pick_tile<bf16, UPPER>(g.M, g.N, batch);
-  if constexpr (UPPER) {
-    // the 192² tile: 384-byte transposing rows (swzq's second form)
-    typedef typename TileSet<bf16>::sym_mid Mid;
-    static_assert(Mid::BM == Mid::BN && Mid::BK == Big::BK, "mid tile: square, same K tile");
-    if (pick == 2) return launch_gemm_cfg<bf16, Mid, UPPER, Epi, true, PT>(g, epi, batch, stream, name);
+  PTO_REQUIRE(pick >= -1 && pick <= (tiny_all<T>() ? 3 : 2) && (UPPER || TileSet<T>::kMidAll || pick != 2), std::string(name) + ": tile choice");
+  if (pick < 0) pick = pick_tile<T, UPPER>(g.M, g.N, batch);
+  if constexpr (tiny_all<T>()) {
+    // the 64² tile: 128-byte transposing rows (swzq's second form)
+    if (pick == 3) return launch_gemm_cfg<T, typename TileSet<T>::sym_tiny, UPPER, Epi, true, PT>(g, epi, batch, stream, name);
   }
-  if (pick == 1) return launch_gemm_cfg<bf16, Big, UPPER, Epi, true, PT>(g, epi, batch, stream, name);
-  return launch_gemm_cfg<bf16, Small, UPPER, Epi, true, PT>(g, epi, batch, stream, name);
+  if constexpr (UPPER || TileSet<T>::kMidAll) {
+    // the 192² tile: 384-byte transposing rows (swzq's second form)
+    typedef typename TileSet<T>::sym_mid Mid;
+    static_assert(Mid::BM == Mid::BN && Mid::BK == Big::BK, "mid tile: square, same K tile");
+    if (pick == 2) return launch_gemm_cfg<T, Mid, UPPER, Epi, true, PT>(g, epi, batch, stream, name);
+  }
+  if (pick == 1) return launch_gemm_cfg<T, Big, UPPER, Epi, true, PT>(g, epi, batch, stream, name);
+  return launch_gemm_cfg<T, Small, UPPER, Epi, true, PT>(g, epi, batch, stream, name);
 }
 
 // ------------------------------------------------------------- epilogues

@@ -23,11 +23,14 @@
 // and fp64 the update reads a stored Xᵀ, which its epilogue writes beside
 // X'. bf16 inputs keep X, A, B in bf16 between launches with fp32
 // accumulation (short side 128 or more; smaller ones run the fp32 chain,
-// see ns5_bf16); fp32 and fp64 inputs stay in their own precision.
+// see ns5_bf16); fp32 and fp64 inputs stay in their own precision
+// (fp32 above the smallest sizes with its products on split operands, see
+// ns5_split_run).
 #include <algorithm>
 
 #include "aux_kernels.h"
 #include "gemm_nt.h"
+#include "split.h"
 
 namespace pto {
 
@@ -186,6 +189,282 @@ size_t ns5_ws_bytes_t(int64_t batch, int64_t rows, int64_t cols) {
   return bytes + 256;
 }
 
+// ------------------------------------------------ fp32 on split operands
+//
+// The fp32 chain with X, A and B' held as fp16 pairs (split.h) and its
+// products on the fp16 MFMA. Their power-of-two scales come from bounds that
+// need no data beyond the norm: ‖X_0‖₂ <= ‖X_0‖_F = ρ, every entry of a matrix
+// is at most its spectral norm, and X' = p(X) on the singular values with
+// p(s) = a·s + b·s³ + c·s⁵, so x_{t+1} = max |p| over [0, x_t] bounds X_{t+1}.
+struct NsExp {
+  int x, a, b, xn;  // planes hold X·2^x, A·2^a, B'·2^b; the next iterate's x
+};
+constexpr int kNsSplitSteps = 32;  // per matrix: exponents of this many steps
+
+// Clamped to exponents that fp32 values (and so their bounds) have.
+__device__ __forceinline__ int ns_exp(double bound) {
+  int k = 0;
+  if (!(bound > 0.0)) bound = 1.0;  // zero or NaN: any scale does
+  (void)frexp(fmin(bound, 3e38), &k);
+  return max(-120, min(120, kSplitTop - k));
+}
+
+// 1 / (‖G‖ + eps) as ns_scale_kernel gives it, and the exponents of all steps.
+__global__ void __launch_bounds__(256) ns_split_scale_kernel(const double* __restrict__ partial, double eps, int steps,
+                                                             double a, double b, double c, float* __restrict__ scale,
+                                                             NsExp* __restrict__ ex) {
+  const double s = block_sum_partials(partial, blockIdx.x);
+  if (threadIdx.x != 0) return;
+  const float norm = static_cast<float>(sqrt(s));
+  const float sc = 1.f / (norm + static_cast<float>(eps));
+  scale[blockIdx.x] = sc;
+  NsExp* e = ex + (int64_t)blockIdx.x * kNsSplitSteps;
+  double x = (double)norm * sc;
+  int ex_t = ns_exp(x);
+  for (int t = 0; t < steps; ++t) {
+    const double u = x * x;
+    // |p| is largest at the end of [0, x] or where p' = a + 3b·s² + 5c·s⁴ = 0
+    auto p = [&](double q) { return fabs(a + q * (b + q * c)) * sqrt(q); };  // q = s²
+    double top = p(u);
+    const double disc = 9.0 * b * b - 20.0 * a * c;
+    if (c != 0.0 && disc >= 0.0) {
+      for (int sg = -1; sg <= 1; sg += 2) {
+        const double q = (-3.0 * b + sg * sqrt(disc)) / (10.0 * c);
+        if (q > 0.0 && q < u) top = fmax(top, p(q));
+      }
+    } else if (c == 0.0 && b != 0.0) {
+      const double q = -a / (3.0 * b);
+      if (q > 0.0 && q < u) top = fmax(top, p(q));
+    }
+    x = 1.01 * top;  // the products' rounding
+    const int nxt = ns_exp(x);
+    e[t] = NsExp{ex_t, ns_exp(u), ns_exp(fabs(a) + fabs(b) * u + fabs(c) * u * u), nxt};
+    ex_t = nxt;
+  }
+}
+
+// A = v·2^-2x, into its planes
+struct EpiNsGramSplit {
+  typedef float S;
+  sp16* dst;
+  int64_t pl, ld, sd;
+  const NsExp* ex;  // matrix b: ex[b * kNsSplitSteps]
+  typedef NoPre Pre;
+  typedef NoPre PreT;
+  static constexpr bool kVoIsV = true;
+  __device__ __forceinline__ bool has_t() const { return false; }
+  __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
+  __device__ __forceinline__ void store(int b, int64_t o, const S* v, int kbeg, int n) const {
+    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+    S w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], e.a - 2 * e.x);
+    st8_split(dst + (int64_t)b * sd + o, pl, w, kbeg, n);
+  }
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
+    store(b, (int64_t)i * ld + j0, v, kbeg, n);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) vo[k] = v[k];
+  }
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
+    store(b, (int64_t)j * ld + i0, v, 0, n);
+  }
+  __device__ __forceinline__ void finish(int) const {}
+};
+
+// B' = a·I + b·A + c·v·2^-2a
+struct EpiNsSqSplit {
+  typedef float S;
+  const sp16* Asrc;
+  sp16* dst;
+  int64_t pl, ld, sd;
+  float ac, bc, cc;
+  const NsExp* ex;
+  struct Pre {
+    uint4 h, l;
+  };
+  typedef NoPre PreT;
+  static constexpr bool kVoIsV = false;  // the mirror stores B', not the raw product
+  __device__ __forceinline__ bool has_t() const { return false; }
+  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
+    if (full_run(kbeg, n)) {
+      const sp16* q = Asrc + (int64_t)b * sd + (int64_t)i * ld + j0;
+      p.h = ld16(q);
+      p.l = ld16(q + pl);
+    }
+  }
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre,
+                                      S* vo) const {
+    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+    const int64_t o = (int64_t)b * sd + (int64_t)i * ld + j0;
+    S a[8];
+    if (full_run(kbeg, n)) {
+      const f16x8_t h = __builtin_bit_cast(f16x8_t, pre.h), l = __builtin_bit_cast(f16x8_t, pre.l);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) a[k] = static_cast<S>(h[k]) + static_cast<S>(l[k]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        a[k] = k >= kbeg && k < n ? static_cast<S>(Asrc[o + k].v) + static_cast<S>(Asrc[o + pl + k].v) : S(0);
+    }
+    S w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      vo[k] = fma(cc, ldexpf(v[k], -2 * e.a), fma(bc, ldexpf(a[k], -e.a), i == j0 + k ? ac : 0.f));
+      w[k] = ldexpf(vo[k], e.b);
+    }
+    st8_split(dst + o, pl, w, kbeg, n);
+  }
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
+    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+    S w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], e.b);
+    st8_split(dst + (int64_t)b * sd + (int64_t)j * ld + i0, pl, w, 0, n);
+  }
+  __device__ __forceinline__ void finish(int) const {}
+};
+
+// X' = v·2^-(b + x): into the next iterate's planes, or (last iteration) as
+// fp32 into out, row-major (dst) or transposed (dstT).
+struct EpiNsUpdateSplit {
+  typedef float S;
+  sp16* planes;
+  int64_t pl, ld, sd;
+  float* dst;
+  float* dstT;
+  int64_t ld_o, s_o;
+  const NsExp* ex;
+  typedef NoPre Pre;
+  typedef NoPre PreT;
+  static constexpr bool kVoIsV = true;
+  __device__ __forceinline__ bool has_t() const { return dstT != nullptr; }
+  __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
+    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) vo[k] = v[k];
+    S w[8];
+    if (planes) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], e.xn - e.b - e.x);
+      st8_split(planes + (int64_t)b * sd + (int64_t)i * ld + j0, pl, w, kbeg, n);
+    } else if (dst) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], -e.b - e.x);
+      st8<float, S>(dst + (int64_t)b * s_o + (int64_t)i * ld_o + j0, w, kbeg, n);
+    }
+  }
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
+    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+    S w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], -e.b - e.x);
+    st8<float, S>(dstT + (int64_t)b * s_o + (int64_t)j * ld_o + i0, w, 0, n);
+  }
+  __device__ __forceinline__ void finish(int) const {}
+};
+
+size_t ns5_split_ws_bytes(int64_t batch, int64_t m, int64_t n) {
+  const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
+  size_t bytes = 0;
+  auto add = [&](size_t b) { bytes = round_up(bytes, 256) + b; };
+  add(sizeof(double) * kRedBlocks * batch);
+  add(sizeof(float) * batch);
+  add(sizeof(NsExp) * kNsSplitSteps * batch);
+  add(sizeof(sp16) * 2 * batch * ldm * ldm);  // A
+  add(sizeof(sp16) * 2 * batch * ldm * ldm);  // B'
+  add(sizeof(sp16) * 2 * batch * ldm * ldn);  // X ping
+  add(sizeof(sp16) * 2 * batch * ldm * ldn);  // X pong
+  return bytes + 256;
+}
+
+// Sizes that run on split operands. Below batch·m² = 512² the launches have
+// too few of the split products' 64² tiles and wait for their loads (one
+// 256 x 4096 273 us against 229 on the fp32 MFMA's 32² tiles, 384 x 1536 186
+// against 164, 512 x 512 the same, 768 x 768 183 against 221, 2048 x 2048 800
+// against 1569; eight of 256 x 1024 178 against 210, of 2048 x 2048 3.85 ms
+// against 11.3). Sides just above a multiple of 128, whose planes would not
+// fit the workspace of the fp32 chain, keep that chain.
+constexpr int64_t kNsSplitMinSide = 128, kNsSplitMinWork = 512 * 512;
+inline bool ns5_split(int64_t batch, int64_t m, int64_t n, int64_t steps) {
+  return m >= kNsSplitMinSide && batch * m * m >= kNsSplitMinWork && steps >= 1 && steps <= kNsSplitSteps &&
+         ns5_split_ws_bytes(batch, m, n) <= ns5_ws_bytes_t<float>(batch, m, n);
+}
+
+int ns5_split_run(const float* G, float* out, int64_t batch, int64_t rows, int64_t cols, int64_t steps, double a,
+                  double b, double c, double eps, void* ws, size_t ws_bytes, hipStream_t stream) {
+  const bool transposed = rows > cols;
+  const int64_t m = std::min(rows, cols), n = std::max(rows, cols);
+  const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
+  const int64_t plA = ldm * ldm, sA = 2 * plA, plX = ldm * ldn, sX = 2 * plX, sG = rows * cols;
+  const int nb = (int)batch;
+  Carver cv(ws, ws_bytes);
+  double* partial = cv.take<double>(kRedBlocks * batch);
+  float* scale = cv.take<float>(batch);
+  NsExp* ex = cv.take<NsExp>(kNsSplitSteps * batch);
+  sp16* Ab = cv.take<sp16>(batch * sA);
+  sp16* Bb = cv.take<sp16>(batch * sA);
+  sp16* X[2];
+  for (sp16*& x : X) x = cv.take<sp16>(batch * sX);
+  PTO_REQUIRE(!cv.overflow, "newton_schulz_orthogonalize: workspace too small");
+
+  if (launch_sumsq<float>(G, rows, cols, cols, sG, nb, partial, stream)) return -1;
+  hipLaunchKernelGGL(ns_split_scale_kernel, dim3(nb), dim3(256), 0, stream, partial, eps, (int)steps, a, b, c, scale,
+                     ex);
+  PTO_LAUNCHED("ns_split_scale");
+  const int* ex0 = &ex->x;
+  const int ex_stride = kNsSplitSteps * (int)(sizeof(NsExp) / sizeof(int));
+  if (!transposed) {
+    const unsigned gx = (unsigned)std::min<int64_t>((ldm * (ldn / 8) + 255) / 256, 4096);
+    hipLaunchKernelGGL(split_pack_kernel, dim3(gx, (unsigned)nb), dim3(256), 0, stream, G, rows, cols, cols, sG, scale,
+                       ex0, ex_stride, X[0], plX, ldm, ldn, sX);
+  } else {
+    const dim3 grid((unsigned)(ldm / 64), (unsigned)(ldn / 64), (unsigned)nb);
+    PTO_REQUIRE(grid.y < 65536, "newton_schulz_orthogonalize: shape too large");
+    hipLaunchKernelGGL(split_pack_t_kernel, grid, dim3(256), 0, stream, G, rows, cols, cols, sG, scale, ex0, ex_stride,
+                       X[0], plX, ldm, ldn, sX);
+  }
+  PTO_LAUNCHED("split_pack");
+  PadList pads;
+  for (sp16* p : {Ab, Bb}) pads.add(p, m, ldm, m, ldm, plA, 2 * nb);
+  if (steps > 1) pads.add(X[1], m, ldm, n, ldn, plX, 2 * nb);
+  if (launch_zero_pads(pads, stream)) return -1;
+
+  for (int64_t t = 0; t < steps; ++t) {
+    const bool last = t == steps - 1;
+    const sp16* Xc = X[t & 1];
+    {
+      GemmArgs g{Xc, ldn, sX, Xc, ldn, sX, (int)m, (int)m, (int)ldn, 0, 0, nullptr, 0, 0, plX, plX};
+      EpiNsGramSplit e{Ab, plA, ldm, sA, ex + t};
+      if (launch_gemm<sp16, true>(g, e, nb, stream, "ns5_gram")) return -1;
+    }
+    {
+      GemmArgs g{Ab, ldm, sA, Ab, ldm, sA, (int)m, (int)m, (int)ldm, 0, 0, nullptr, 0, 0, plA, plA};
+      EpiNsSqSplit e{Ab, Bb, plA, ldm, sA, (float)a, (float)b, (float)c, ex + t};
+      // A's rows are its columns: read K-contiguous by the 256² and 192² tiles
+      // (12 x 2048²: 310 us against 325 with transposing reads), transposing
+      // by the smaller ones, whose LDS reads bound them (128² 317 against 350)
+      const int pick = pick_tile<sp16, true>(m, m, nb);
+      if (pick == 1 || pick == 2) {
+        if (launch_gemm<sp16, true>(g, e, nb, stream, "ns5_square")) return -1;
+      } else if (launch_gemm_qn<EpiNsSqSplit, true, true, sp16>(g, e, nb, stream, "ns5_square", pick)) {
+        return -1;
+      }
+    }
+    {
+      GemmArgs g{Bb, ldm, sA, Xc, ldn, sX, (int)m, (int)n, (int)ldm, 0, 0, nullptr, 0, 0, plA, plX};
+      EpiNsUpdateSplit e{last ? nullptr : X[(t & 1) ^ 1], plX, ldn, sX, last && !transposed ? out : nullptr,
+                         last && transposed ? out : nullptr, cols, sG, ex + t};
+      if (launch_gemm_qn<EpiNsUpdateSplit, true, false, sp16>(g, e, nb, stream, "ns5_update")) return -1;
+    }
+  }
+  return 0;
+}
+
 template <typename T>
 int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t steps, double a, double b, double c,
           double eps, void* ws, size_t ws_bytes, hipStream_t stream) {
@@ -195,6 +474,21 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
   const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   PTO_REQUIRE(m <= INT32_MAX && n <= INT32_MAX && batch <= 65535, "newton_schulz_orthogonalize: shape too large");
   if (batch == 0 || rows == 0 || cols == 0) return 0;
+
+  // `out` may alias G exactly or not at all: every path below reads G only
+  // in kernels that end before `out` is written, except the steps == 0
+  // pack, which is tile-local (each element read before it is rewritten
+  // in place) only when the two coincide.
+  const int64_t sG = rows * cols;
+  const uintptr_t g0 = reinterpret_cast<uintptr_t>(G), g1 = g0 + sizeof(T) * (uintptr_t)(batch * sG);
+  const uintptr_t o0 = reinterpret_cast<uintptr_t>(out), o1 = o0 + sizeof(T) * (uintptr_t)(batch * sG);
+  const bool aliased = g0 < o1 && o0 < g1;
+  PTO_REQUIRE(!aliased || g0 == o0, "newton_schulz_orthogonalize: out partially overlaps G");
+
+  if constexpr (std::is_same<T, float>::value) {
+    if (ns5_split(batch, m, n, steps))
+      return ns5_split_run(G, out, batch, rows, cols, steps, a, b, c, eps, ws, ws_bytes, stream);
+  }
 
   constexpr bool QN = ns5_qn<T>();
   Carver cv(ws, ws_bytes);
@@ -218,21 +512,11 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
   }
   PTO_REQUIRE(!cv.overflow, "newton_schulz_orthogonalize: workspace too small");
   const int nb = (int)batch;
-  const int64_t sG = rows * cols;
 
   // ‖X‖_F per matrix (deterministic two-stage sum), then 1/(‖X‖+eps).
   if (launch_sumsq<T>(G, rows, cols, cols, sG, nb, partial, stream)) return -1;
   hipLaunchKernelGGL(ns_scale_kernel<A>, dim3(nb), dim3(256), 0, stream, partial, eps, scale);
   PTO_LAUNCHED("ns_scale");
-
-  // `out` may alias G exactly or not at all: every path below reads G only
-  // in kernels that end before `out` is written, except the steps == 0
-  // pack, which is tile-local (each element read before it is rewritten
-  // in place) only when the two coincide.
-  const uintptr_t g0 = reinterpret_cast<uintptr_t>(G), g1 = g0 + sizeof(T) * (uintptr_t)(batch * sG);
-  const uintptr_t o0 = reinterpret_cast<uintptr_t>(out), o1 = o0 + sizeof(T) * (uintptr_t)(batch * sG);
-  const bool aliased = g0 < o1 && o0 < g1;
-  PTO_REQUIRE(!aliased || g0 == o0, "newton_schulz_orthogonalize: out partially overlaps G");
 
   if (steps == 0) {  // the normalised input, in the input's layout
     if (launch_pack<T, T, A>(G, rows, cols, cols, sG, scale, out, cols, sG, nullptr, 0, 0, false, nb, stream)) return -1;
