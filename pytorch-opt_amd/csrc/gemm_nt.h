@@ -882,7 +882,8 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
     //   R2: reads of the other P fragments;   M2: their MFMAs.
     // Group 1 runs one phase behind. Block p-1 was last read in R2(p-1), which
     // group 1 ends before group 0's R1(p); every wave waits for its part of
-    // block p+1 at the end of R2(p), before either group's R1(p+1).
+    // block p+1 before group 0's R1(p+1): group 0 at the end of M2(p), group 1
+    // at the end of R2(p), which runs beside it.
     if (KT > 0) {
       static_assert(FM % 2 == 0, "halves of the fragment rows");
       constexpr int HM = FM / 2;
@@ -925,9 +926,10 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
       la[x] = load_a(L, 0, HM + x);                           \
     }                                                         \
   }                                                           \
-  __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));                   \
+  if (grp) __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));          \
   PTO_PHASE_END()                                             \
   if (!idle) mma_split(ha, la, hb, lb, half, half);           \
+  if (!grp) __builtin_amdgcn_s_waitcnt(PTO_VMCNT(0));         \
   PTO_PHASE_END()
         PTO_BLOCK(0, st0, st1, st2, st3)
         PTO_BLOCK(2, st2, st3, st0, st1)

@@ -14,17 +14,86 @@
 //
 // Each factor is one symmetric MFMA launch: only upper tiles are computed,
 // the blend with the old factor is fused into the epilogue, and both
-// (i, j) and (j, i) are written, so each factor is read and written once.
+// (i, j) and (j, i) are written, so each factor is read and written once. Large
+// fp32 products run on split operands (split.h).
 #include <algorithm>
 
 #include "aux_kernels.h"
 #include "gemm_nt.h"
+#include "split.h"
 
 namespace pto {
 namespace {
 
+// ------------------------------------------------ fp32 on split operands
+//
+// Both factors' products on the fp16 MFMA (split.h): L from the planes of G
+// with a scale per row, R from those of Gᵀ with a scale per column. The rule
+// looks at one matrix only, so that a batched call gives each factor the bits
+// of its single call.
+// Above a short side of 1024 and this work; below, the pass for the scales and
+// the two more launches cost what the products save (1536² 102 us against 92 on
+// the fp32 MFMA, 4096 x 512 139 against 132; 1024 x 4096 157 against 223, 2048²
+// 133 against 192, 4096² 542 against 1126: 55 in the two passes over G, 246 in
+// each product, the rest in launches).
+constexpr int64_t kKronSplitSide = 1024;
+constexpr double kKronSplitWork = 1.2e10;  // m·n·(m + n)
+inline bool kron_split(int64_t m, int64_t n) {
+  return std::min(m, n) >= kKronSplitSide && (double)m * n * (m + n) >= kKronSplitWork;
+}
+
+struct KronSplitWs {
+  sp16 *Gp, *GT;
+  unsigned *rpart, *cpart;
+  int *bad, *er, *ec;
+  int64_t mw, nw;
+  KronSplitWs(Carver& cv, int64_t batch, int64_t m, int64_t n) : mw(round_up(m, 8)), nw(round_up(n, 8)) {
+    Gp = cv.take<sp16>(2 * batch * m * round_up(n, kPadK));
+    GT = cv.take<sp16>(2 * batch * n * round_up(m, kPadK));
+    rpart = cv.take<unsigned>(batch * mw * absmax_row_parts(n));
+    cpart = cv.take<unsigned>(batch * nw * absmax_col_parts(m));
+    bad = cv.take<int>(batch);
+    er = cv.take<int>(batch * mw);
+    ec = cv.take<int>(batch * nw);
+  }
+  static size_t bytes(int64_t batch, int64_t m, int64_t n) {
+    const int64_t mw = round_up(m, 8), nw = round_up(n, 8);
+    return sizeof(sp16) * 2 * (size_t)(batch * (m * round_up(n, kPadK) + n * round_up(m, kPadK))) +
+           4 * (size_t)(batch * (mw * (1 + absmax_row_parts(n)) + nw * (1 + absmax_col_parts(m)) + 1)) + 8 * 256;
+  }
+};
+
+template <class EpiL>
+int kron_split_run(const EpiL& el, const EpiL& er, const float* G, int64_t batch, int64_t m, int64_t n, void* ws,
+                   size_t ws_bytes, hipStream_t stream) {
+  const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
+  const int nb = (int)batch;
+  Carver cv(ws, ws_bytes);
+  const KronSplitWs w(cv, batch, m, n);
+  PTO_REQUIRE(!cv.overflow, "kron_factor_update_: workspace too small");
+  const SplitPack p{G,    m,       n,   n,           m * n, w.rpart, w.cpart, w.mw,        w.nw, w.er, w.ec, w.bad,
+                    w.Gp, m * ldn, ldn, 2 * m * ldn, w.GT,  n * ldm, ldm,     2 * n * ldm, 0};
+  if (launch_split_pack_max(p, nb, stream)) return -1;
+  {
+    GemmArgs g{w.Gp, ldn, 2 * m * ldn, w.Gp, ldn, 2 * m * ldn, (int)m, (int)m, (int)ldn, 0, 0, w.bad, 1, 0, m * ldn,
+               m * ldn};
+    const EpiDescale<EpiL> e{el, w.er, w.er, w.mw, w.mw};
+    if (launch_gemm<sp16, true, EpiDescale<EpiL>, true>(g, e, nb, stream, "kron_left")) return -1;
+  }
+  {
+    GemmArgs g{w.GT, ldm, 2 * n * ldm, w.GT, ldm, 2 * n * ldm, (int)n, (int)n, (int)ldm, 0, 0, w.bad, 1, 0, n * ldm,
+               n * ldm};
+    const EpiDescale<EpiL> e{er, w.ec, w.ec, w.nw, w.nw};
+    if (launch_gemm<sp16, true, EpiDescale<EpiL>, true>(g, e, nb, stream, "kron_right")) return -1;
+  }
+  const PlainOperand gl{G, n, 1, m * n, -1}, gr{G, 1, n, m * n, -1};
+  const PlainProduct<EpiL> left{gl, gl, m, m, n, el}, right{gr, gr, n, n, m, er};
+  return launch_plain_product(w.bad, nb, left, &right, stream);
+}
+
 template <typename T>
 size_t kron_ws_bytes_t(int64_t m, int64_t n) {
+  if (std::is_same<T, float>::value && kron_split(m, n)) return KronSplitWs::bytes(1, m, n);
   int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   size_t bytes = 0;
   auto add = [&](size_t b) { bytes = round_up(bytes, 256) + b; };
@@ -39,6 +108,13 @@ int kron_t(T* L, T* R, const T* G, int64_t m, int64_t n, double beta2, void* ws,
   typedef typename AccOf<T>::type A;
   PTO_REQUIRE(m <= INT32_MAX && n <= INT32_MAX, "kron_factor_update_: shape too large");
   if (m == 0 || n == 0) return 0;
+  const A beta = beta2 == 1.0 ? A(1) : static_cast<A>(beta2);
+  const A alpha = beta2 == 1.0 ? A(1) : static_cast<A>(1.0 - beta2);
+  if constexpr (std::is_same<T, float>::value) {
+    if (kron_split(m, n))
+      return kron_split_run(EpiBlend<T, A>{L, m, 0, beta, alpha}, EpiBlend<T, A>{R, n, 0, beta, alpha}, G, 1, m, n, ws,
+                            ws_bytes, stream);
+  }
   const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   Carver cv(ws, ws_bytes);
   T* Gp = cv.take<T>(m * ldn);
@@ -52,8 +128,6 @@ int kron_t(T* L, T* R, const T* G, int64_t m, int64_t n, double beta2, void* ws,
                            stream))
     return -1;
 
-  const A beta = beta2 == 1.0 ? A(1) : static_cast<A>(beta2);
-  const A alpha = beta2 == 1.0 ? A(1) : static_cast<A>(1.0 - beta2);
   {
     GemmArgs g{Grows, ldg, 0, Grows, ldg, 0, (int)m, (int)m, (int)ldn, 0, 0, nullptr};
     EpiBlend<T, A> e{L, m, 0, beta, alpha};
@@ -75,6 +149,7 @@ int kron_t(T* L, T* R, const T* G, int64_t m, int64_t n, double beta2, void* ws,
 // the bits a single-matrix call gives.
 template <typename T>
 size_t kron_batched_ws_bytes_t(int64_t batch, int64_t m, int64_t n) {
+  if (std::is_same<T, float>::value && kron_split(m, n)) return KronSplitWs::bytes(batch, m, n);
   int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   size_t bytes = 0;
   auto add = [&](size_t b) { bytes = round_up(bytes, 256) + b; };
@@ -96,6 +171,19 @@ int kron_batched_t(T* const* L, T* const* R, const T* G, int64_t batch, int64_t 
       PTO_REQUIRE(L[b] != R[c] && (c == b || (L[b] != L[c] && R[b] != R[c])),
                   "kron_factor_update_batched_: factors must be distinct tensors");
   }
+  const A beta = beta2 == 1.0 ? A(1) : static_cast<A>(beta2);
+  const A alpha = beta2 == 1.0 ? A(1) : static_cast<A>(1.0 - beta2);
+  auto table = [&](T* const* F, int64_t d) {
+    EpiBlendTab<T, A> e{};
+    e.ld = d;
+    e.beta = beta;
+    e.alpha = alpha;
+    for (int64_t b = 0; b < batch; ++b) e.dst[b] = F[b];
+    return e;
+  };
+  if constexpr (std::is_same<T, float>::value) {
+    if (kron_split(m, n)) return kron_split_run(table(L, m), table(R, n), G, batch, m, n, ws, ws_bytes, stream);
+  }
   const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   Carver cv(ws, ws_bytes);
   T* Gp = cv.take<T>(batch * m * ldn);
@@ -109,16 +197,6 @@ int kron_batched_t(T* const* L, T* const* R, const T* G, int64_t batch, int64_t 
                            (int)batch, stream))
     return -1;
 
-  const A beta = beta2 == 1.0 ? A(1) : static_cast<A>(beta2);
-  const A alpha = beta2 == 1.0 ? A(1) : static_cast<A>(1.0 - beta2);
-  auto table = [&](T* const* F, int64_t d) {
-    EpiBlendTab<T, A> e{};
-    e.ld = d;
-    e.beta = beta;
-    e.alpha = alpha;
-    for (int64_t b = 0; b < batch; ++b) e.dst[b] = F[b];
-    return e;
-  };
   {
     GemmArgs g{Grows, ldg, sg, Grows, ldg, sg, (int)m, (int)m, (int)ldn, 0, 0, nullptr};
     if (launch_gemm<T, true>(g, table(L, m), (int)batch, stream, "kron_left")) return -1;
@@ -128,6 +206,40 @@ int kron_batched_t(T* const* L, T* const* R, const T* G, int64_t batch, int64_t 
     if (launch_gemm<T, true>(g, table(R, n), (int)batch, stream, "kron_right")) return -1;
   }
   return 0;
+}
+
+// fp32 X on split operands: the planes of X̃ᵀ with a scale per column of X̃.
+// As kron_split: 4096 x 1024 76 us against 70 on the fp32 MFMA, 16384 x 1024
+// 212 against 235, 2048² 78 against 100, 8192 x 2048 217 against 360.
+constexpr int64_t kGramSplitSide = 1024;
+constexpr double kGramSplitWork = 8e9;  // rows·d²
+template <typename TX>
+bool gram_split(int64_t rows, int64_t d) {
+  return std::is_same<TX, float>::value && d >= kGramSplitSide && (double)rows * d * d >= kGramSplitWork;
+}
+inline size_t gram_split_ws_bytes(int64_t rows, int64_t dd) {
+  return sizeof(sp16) * 2 * (size_t)(dd * round_up(rows, kPadK)) +
+         4 * (size_t)(round_up(dd, 8) * (1 + absmax_col_parts(rows)) + 1) + 5 * 256;
+}
+template <class Epi>
+int gram_split_run(const Epi& epi, const float* X, int64_t rows, int64_t d, int ones, void* ws, size_t ws_bytes,
+                   hipStream_t stream) {
+  const int64_t dd = d + ones, ldr = round_up(rows, kPadK), dw = round_up(dd, 8);
+  Carver cv(ws, ws_bytes);
+  sp16* XT = cv.take<sp16>(2 * dd * ldr);
+  unsigned* cpart = cv.take<unsigned>(dw * absmax_col_parts(rows));
+  int* bad = cv.take<int>(1);
+  int* ec = cv.take<int>(dw);
+  PTO_REQUIRE(!cv.overflow, "gram_update_: workspace too small");
+  const SplitPack p{X, rows, d, d, 0, nullptr, cpart, 0, dw, nullptr, ec, bad, nullptr, 0, 0, 0, XT, dd * ldr, ldr,
+                    0, ones};
+  if (launch_split_pack_max(p, 1, stream)) return -1;
+  GemmArgs g{XT, ldr, 0, XT, ldr, 0, (int)dd, (int)dd, (int)ldr, 0, 0, bad, 0, 0, dd * ldr, dd * ldr};
+  const EpiDescale<Epi> e{epi, ec, ec, 0, 0};
+  if (launch_gemm<sp16, true, EpiDescale<Epi>, true>(g, e, 1, stream, "gram_update")) return -1;
+  const PlainOperand x{X, 1, d, 0, ones ? d : -1};
+  return launch_plain_product(bad, 1, PlainProduct<Epi>{x, x, dd, dd, rows, epi}, (const PlainProduct<Epi>*)nullptr,
+                              stream);
 }
 
 // bf16 X without the ones column is already the [K][M] operand of the
@@ -149,6 +261,7 @@ template <typename TX>
 size_t gram_ws_bytes_t(int64_t rows, int64_t d, int append_ones) {
   if (gram_direct_tile<TX>(rows, d, append_ones) >= 0) return 0;
   int64_t dd = d + (append_ones ? 1 : 0);
+  if (gram_split<TX>(rows, d)) return gram_split_ws_bytes(rows, dd);
   return sizeof(TX) * dd * round_up(rows, kPadK) + 512;
 }
 
@@ -170,6 +283,11 @@ int gram_t(TF* F, const TX* X, int64_t rows, int64_t d, int append_ones, double 
       EpiBlend<TF, A> e{F, dd, 0, static_cast<A>(beta), static_cast<A>(alpha)};
       return launch_gemm_qn<EpiBlend<TF, A>, true, true>(g, e, 1, stream, "gram_update_direct", tile);
     }
+  }
+  if constexpr (std::is_same<TX, float>::value && std::is_same<TF, float>::value) {
+    if (gram_split<TX>(rows, d))
+      return gram_split_run(EpiBlend<TF, A>{F, dd, 0, static_cast<A>(beta), static_cast<A>(alpha)}, X, rows, d,
+                            append_ones ? 1 : 0, ws, ws_bytes, stream);
   }
   Carver cv(ws, ws_bytes);
   TX* XT = cv.take<TX>(dd * ldr);

@@ -13,13 +13,15 @@
 
 namespace pto {
 
-// Exponent e with max·2^e in (2^13, 2^14] for a bound max > 0 (0 for zero,
-// infinite and NaN bounds; non-finite operands never reach the products that
-// read planes, or are meant to come out as NaN).
-constexpr int kSplitTop = 14;
+// Exponent e with max·2^e in (2^13, 2^14] for a finite bound max > 0. Non-finite
+// operands never reach the products that read these planes; an empty row or
+// column says "tiny" (its values are all zero, and where its exponent scales
+// another operand's row that row must not outweigh the others).
+constexpr int kSplitTop = 14, kSplitZero = 120;
 __device__ __forceinline__ int split_exp(float bound) {
   int k = 0;
-  if (!(bound > 0.f) || bound > 3.0e38f * 2.f) return 0;
+  if (bound == 0.f) return kSplitZero;
+  if (!(bound < INFINITY)) return 0;
   (void)frexpf(bound, &k);  // bound <= 2^k
   return kSplitTop - k;
 }
@@ -63,7 +65,7 @@ __device__ __forceinline__ void st8_split(sp16* p, int64_t pl, const float* in, 
 // orows) zero. e = e_mat[b * e_mat_stride] (per matrix).
 // Each thread takes eight consecutive output columns: 32 bytes in, 16 + 16
 // out. Bound by memory: 8 bytes per element.
-static __global__ void __launch_bounds__(256) split_pack_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
+[[maybe_unused]] static __global__ void __launch_bounds__(256) split_pack_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
                                                          int64_t ld_in, int64_t s_in, const float* __restrict__ scale,
                                                          const int* __restrict__ e_mat, int e_mat_stride,
                                                          sp16* __restrict__ out, int64_t pl, int64_t orows, int64_t ld,
@@ -96,7 +98,7 @@ static __global__ void __launch_bounds__(256) split_pack_kernel(const float* __r
 // The planes of the transpose: out [orows][ld], out(c, r) = in(r, c)·scale_b·2^e,
 // through a 64 x 64 LDS tile (65-word rows: both its accesses spread over the
 // banks).
-static __global__ void __launch_bounds__(256) split_pack_t_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
+[[maybe_unused]] static __global__ void __launch_bounds__(256) split_pack_t_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
                                                            int64_t ld_in, int64_t s_in, const float* __restrict__ scale,
                                                            const int* __restrict__ e_mat, int e_mat_stride,
                                                            sp16* __restrict__ out, int64_t pl, int64_t orows,
@@ -109,8 +111,9 @@ static __global__ void __launch_bounds__(256) split_pack_t_kernel(const float* _
   const float sc = scale ? scale[b] : 1.f;
   const int e = e_mat[(int64_t)b * e_mat_stride];
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-#pragma unroll 8
-  for (int rr = ty; rr < 64; rr += 4) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int rr = ty + 4 * i;
     const int64_t r = r0 + rr, c = c0 + tx;
     tile[rr][tx] = r < rows && c < cols ? ldexpf(ib[r * ld_in + c] * sc, e) : 0.f;
   }
@@ -126,6 +129,311 @@ static __global__ void __launch_bounds__(256) split_pack_t_kernel(const float* _
     *reinterpret_cast<uint4*>(ob + c * ld + r) = s.h;
     *reinterpret_cast<uint4*>(ob + pl + c * ld + r) = s.l;
   }
+}
+
+// Largest |x| of the parts of a fp32 matrix's rows and columns, as bit patterns
+// (which order like the values, NaN above infinity): rpart[cb][r] of columns
+// 256·cb .. + 255, cpart[rb][c] of rows nr·rb .. + nr - 1; either may be null.
+// A workgroup takes nr rows (a multiple of 32) x 256 columns, a wave eight
+// rows at a time, 16 bytes per lane and all eight in flight (one row at a time
+// waited 32 times for memory: 30 us whatever the size). Parts need neither
+// zeroing nor atomics. Bound by memory: 4 bytes per element. Also clears
+// bad[b] (bad != nullptr). pre: x counts as x·2^-pre, pre per row or per column.
+[[maybe_unused]] static __global__ void __launch_bounds__(256) absmax_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
+                                                     int64_t ld, int64_t s_in, int nr, unsigned* __restrict__ rpart,
+                                                     int64_t mw, unsigned* __restrict__ cpart, int64_t nw,
+                                                     int* __restrict__ bad, const int* __restrict__ pre_r,
+                                                     const int* __restrict__ pre_c, int64_t s_pre) {
+  __shared__ unsigned cw[4][256];
+  const int b = blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t r0 = (int64_t)blockIdx.y * nr, c0 = (int64_t)blockIdx.x * 256 + lane * 4;
+  const float* ib = in + (int64_t)b * s_in;
+  if (bad && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) bad[b] = 0;
+  int pc[4] = {0, 0, 0, 0};
+  if (pre_c)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) pc[k] = c0 + k < cols ? pre_c[(int64_t)b * s_pre + c0 + k] : 0;
+  unsigned cm[4] = {0, 0, 0, 0};
+  for (int rr = wave * 8; rr < nr; rr += 32) {
+    uint4 q[8];
+    unsigned rm[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int64_t r = r0 + rr + i;
+      q[i] = make_uint4(0, 0, 0, 0);
+      if (r < rows) {
+        if (c0 + 4 <= cols) {
+          q[i] = ld16(ib + r * ld + c0);
+        } else {
+          if (c0 < cols) q[i].x = __float_as_uint(ib[r * ld + c0]);
+          if (c0 + 1 < cols) q[i].y = __float_as_uint(ib[r * ld + c0 + 1]);
+          if (c0 + 2 < cols) q[i].z = __float_as_uint(ib[r * ld + c0 + 2]);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      unsigned u[4] = {q[i].x & 0x7fffffffu, q[i].y & 0x7fffffffu, q[i].z & 0x7fffffffu, q[i].w & 0x7fffffffu};
+      if (pre_r || pre_c) {
+        const int64_t r = r0 + rr + i;
+        const int pr = pre_r && r < rows ? pre_r[(int64_t)b * s_pre + r] : 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) u[k] = __float_as_uint(ldexpf(__uint_as_float(u[k]), -pr - pc[k]));
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) cm[k] = max(cm[k], u[k]);
+      rm[i] = max(max(u[0], u[1]), max(u[2], u[3]));
+    }
+    if (rpart) {
+      // eight rows over 64 lanes: three exchanges that halve the rows a lane
+      // holds, three more within its eight lanes (10 shuffles for 48)
+      unsigned m4[4], m2[2];
+      const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        m4[i] = max(b5 ? rm[i + 4] : rm[i], (unsigned)__shfl_xor((int)(b5 ? rm[i] : rm[i + 4]), 32, 64));
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        m2[i] = max(b4 ? m4[i + 2] : m4[i], (unsigned)__shfl_xor((int)(b4 ? m4[i] : m4[i + 2]), 16, 64));
+      unsigned m = max(b3 ? m2[1] : m2[0], (unsigned)__shfl_xor((int)(b3 ? m2[0] : m2[1]), 8, 64));
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, 64));
+      const int64_t r = r0 + rr + 4 * b5 + 2 * b4 + b3;
+      if ((lane & 7) == 0 && r < rows) rpart[((int64_t)b * gridDim.x + blockIdx.x) * mw + r] = m;
+    }
+  }
+  if (!cpart) return;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) cw[wave][lane * 4 + k] = cm[k];
+  __syncthreads();
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c < cols)
+    cpart[((int64_t)b * gridDim.y + blockIdx.y) * nw + c] =
+        max(max(cw[0][threadIdx.x], cw[1][threadIdx.x]), max(cw[2][threadIdx.x], cw[3][threadIdx.x]));
+}
+// Parts of a matrix: row parts per 256 columns; column parts per 64 rows, or
+// per 256 where that leaves enough workgroups.
+inline int absmax_rows(int64_t rows) { return rows <= 4096 ? 64 : 256; }
+inline int64_t absmax_row_parts(int64_t cols) { return (cols + 255) / 256; }
+inline int64_t absmax_col_parts(int64_t rows) { return (rows + absmax_rows(rows) - 1) / absmax_rows(rows); }
+
+constexpr unsigned kInfBits = 0x7f800000u;
+
+// Planes of a fp32 matrix in either or both layouts, from one read:
+//   out_s [rows][ld_s]: in(r, c)·2^er(r), out_t [cols + ones][ld_t]:
+//   in(r, c)·2^ec(c) transposed (with `ones`, a last row of ones),
+// pad columns zero, er and ec the split exponents of the parts' maxima, which
+// are stored too (batch strides mw, nw). A row or column with a non-finite
+// value sets bad[b].
+struct SplitPack {
+  const float* in;
+  int64_t rows, cols, ld_in, s_in;
+  unsigned* rpart;
+  unsigned* cpart;
+  int64_t mw, nw;
+  int* er;
+  int* ec;
+  int* bad;
+  sp16* out_s;
+  int64_t pl_s, ld_s, s_s;
+  sp16* out_t;
+  int64_t pl_t, ld_t, s_t;
+  int ones;
+  // x is taken as x·2^-pre (after absmax's reading of the parts alike)
+  const int* pre_r = nullptr;
+  const int* pre_c = nullptr;
+  int64_t s_pre = 0;
+  int one_flag = 0;  // bad is one word for the whole batch, cleared by the caller's first pack only
+};
+[[maybe_unused]] static __global__ void __launch_bounds__(256) split_pack_max_kernel(SplitPack a, int row_parts, int col_parts) {
+  __shared__ float tile[64][65];
+  __shared__ unsigned mx[4][64];
+  __shared__ int xr[64], xc[64];
+  const int b = blockIdx.z;
+  const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
+  const float* ib = a.in + (int64_t)b * a.s_in;
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int rr = ty + 4 * i;
+    const int64_t r = r0 + rr, c = c0 + tx;
+    float x = a.ones && r < a.rows && c == a.cols ? 1.f : 0.f;
+    if (r < a.rows && c < a.cols) {
+      x = ib[r * a.ld_in + c];
+      if (a.pre_r) x = ldexpf(x, -a.pre_r[(int64_t)b * a.s_pre + r]);
+      if (a.pre_c) x = ldexpf(x, -a.pre_c[(int64_t)b * a.s_pre + c]);
+    }
+    tile[rr][tx] = x;
+  }
+  // the tile's exponents: waves 0, 1 its rows' parts, waves 2, 3 its columns'
+  {
+    const bool row = ty < 2;
+    const int64_t at = row ? r0 + tx : c0 + tx, n = row ? a.rows : a.cols, w = row ? a.mw : a.nw;
+    const unsigned* p = row ? a.rpart : a.cpart;
+    const int parts = row ? row_parts : col_parts;
+    unsigned m = 0;
+    if (p && at < n)
+      for (int i = ty & 1; i < parts; i += 2) m = max(m, p[((int64_t)b * parts + i) * w + at]);
+    if (!row && a.ones && at == n) m = __float_as_uint(1.f);
+    mx[ty][tx] = m;
+  }
+  __syncthreads();
+  if (ty == 0 && a.out_s) {
+    const unsigned u = max(mx[0][tx], mx[1][tx]);
+    xr[tx] = split_exp(__uint_as_float(u));
+    if (blockIdx.x == 0 && r0 + tx < a.rows) a.er[(int64_t)b * a.mw + r0 + tx] = xr[tx];
+    if (u >= kInfBits) a.bad[a.one_flag ? 0 : b] = 1;
+  } else if (ty == 1 && a.out_t) {
+    const unsigned u = max(mx[2][tx], mx[3][tx]);
+    xc[tx] = split_exp(__uint_as_float(u));
+    if (blockIdx.y == 0 && c0 + tx < a.cols + a.ones) a.ec[(int64_t)b * a.nw + c0 + tx] = xc[tx];
+    if (u >= kInfBits) a.bad[a.one_flag ? 0 : b] = 1;
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < 64 * 8; q += 256) {
+    const int u = q / 8, w = (q % 8) * 8;
+    float v[8];
+    if (a.out_s && r0 + u < a.rows && c0 + w < a.ld_s) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = c0 + w + k < a.cols ? ldexpf(tile[u][w + k], xr[u]) : 0.f;
+      const Split8 s = split8(v);
+      sp16* o = a.out_s + (int64_t)b * a.s_s + (r0 + u) * a.ld_s + c0 + w;
+      *reinterpret_cast<uint4*>(o) = s.h;
+      *reinterpret_cast<uint4*>(o + a.pl_s) = s.l;
+    }
+    if (a.out_t && c0 + u < a.cols + a.ones && r0 + w < a.ld_t) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = ldexpf(tile[w + k][u], xc[u]);
+      const Split8 s = split8(v);
+      sp16* o = a.out_t + (int64_t)b * a.s_t + (c0 + u) * a.ld_t + r0 + w;
+      *reinterpret_cast<uint4*>(o) = s.h;
+      *reinterpret_cast<uint4*>(o + a.pl_t) = s.l;
+    }
+  }
+}
+inline int launch_split_pack_max(const SplitPack& a, int batch, hipStream_t stream, bool clear = true) {
+  const int nr = absmax_rows(a.rows);
+  const dim3 gm((unsigned)absmax_row_parts(a.cols), (unsigned)absmax_col_parts(a.rows), (unsigned)batch);
+  const int64_t rext = a.out_t ? std::max(a.rows, a.ld_t) : a.rows;
+  const int64_t cext = std::max(a.cols + a.ones, a.out_s ? a.ld_s : 0);
+  const dim3 gp((unsigned)((cext + 63) / 64), (unsigned)((rext + 63) / 64), (unsigned)batch);
+  PTO_REQUIRE(gm.y < 65536 && gp.y < 65536 && batch < 65536, "split_pack: grid too large");
+  hipLaunchKernelGGL(absmax_kernel, gm, dim3(256), 0, stream, a.in, a.rows, a.cols, a.ld_in, a.s_in, nr,
+                     a.out_s ? a.rpart : nullptr, a.mw, a.out_t ? a.cpart : nullptr, a.nw, clear ? a.bad : nullptr,
+                     a.pre_r, a.pre_c, a.s_pre);
+  PTO_LAUNCHED("absmax");
+  hipLaunchKernelGGL(split_pack_max_kernel, gp, dim3(256), 0, stream, a, (int)gm.x, (int)gm.y);
+  PTO_LAUNCHED("split_pack_max");
+  return 0;
+}
+
+// Epilogue of a product of split operands: takes the rows' and columns' scales
+// out (v·2^(off - er(i) - ec(j)); one ldexp, so no intermediate leaves the range of
+// the result) and hands the value to In.
+template <class In>
+struct EpiDescale {
+  typedef float S;
+  In in;
+  const int* er;
+  const int* ec;
+  int64_t s_r, s_c;
+  int off = 0;  // both operands' planes together carry 2^(er + ec - off)
+  typedef typename In::Pre Pre;
+  typedef typename In::PreT PreT;
+  static constexpr bool kVoIsV = true;  // the transposed pass takes the raw value and scales it itself
+  __device__ __forceinline__ bool has_t() const { return false; }
+  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
+    in.load(b, i, j0, kbeg, n, p);
+  }
+  __device__ __forceinline__ void load_t(int b, int j, int i0, int n, PreT& p) const { in.load_t(b, j, i0, n, p); }
+  __device__ __forceinline__ void scaled(int b, int i, int j0, const S* v, int n, S* w) const {
+    const int ei = er[(int64_t)b * s_r + i];
+    const int* ej = ec + (int64_t)b * s_c + j0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = k < n ? ldexpf(v[k], off - ei - ej[k]) : 0.f;
+  }
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre,
+                                      S* vo) const {
+    S w[8], drop[8];
+    scaled(b, i, j0, v, n, w);
+    in.put(b, i, j0, w, kbeg, n, pre, drop);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) vo[k] = v[k];
+  }
+  // symmetric products only (er == ec)
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT& pre) const {
+    S w[8];
+    scaled(b, j, i0, v, n, w);
+    in.put_t(b, j, i0, w, n, pre);
+  }
+  __device__ __forceinline__ void finish(int) const {}
+};
+
+// The products of matrices with a non-finite value (bad[b] != 0), which the
+// split products skip: plain fp32 multiply-adds in k order, so that infinities
+// and NaN land where fp32 arithmetic puts them. C(i, j) = sum_k P(i, k)·Q(j, k)
+// with element strides for rows and k; row `ones_at` of an operand is all ones
+// (-1: none). One launch whatever the batch; with nothing flagged its blocks
+// leave after one read each (3 us).
+struct PlainOperand {
+  const float* p;
+  int64_t row, k, batch;
+  int64_t ones_at;
+  __device__ __forceinline__ float at(int b, int64_t r, int64_t kk) const {
+    return r == ones_at ? 1.f : p[(int64_t)b * batch + r * row + kk * k];
+  }
+};
+template <class Epi>
+struct PlainProduct {
+  PlainOperand P, Q;
+  int64_t M, N, K;
+  Epi epi;
+};
+template <class Epi>
+__global__ void __launch_bounds__(128) plain_product_kernel(const int* __restrict__ bad, int bad_stride, int nb,
+                                                            PlainProduct<Epi> one, PlainProduct<Epi> two) {
+  __shared__ float ps[32][33], qs[32][33];
+  PlainProduct<Epi>& a = blockIdx.y ? two : one;
+  const int64_t tn = (a.N + 31) / 32, tiles = (a.M + 31) / 32 * tn;
+  const int r = threadIdx.x / 4, c = threadIdx.x % 4 * 8;
+  for (int b = 0; b < nb; ++b) {
+    if (bad[b * bad_stride] == 0) continue;
+    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+      const int64_t i0 = t / tn * 32, j0 = t % tn * 32;
+      float v[8] = {0, 0, 0, 0, 0, 0, 0, 0}, vo[8];
+      for (int64_t k0 = 0; k0 < a.K; k0 += 32) {
+        for (int e = threadIdx.x; e < 1024; e += 128) {
+          const int64_t rr = e / 32, kk = k0 + e % 32;
+          ps[rr][e % 32] = i0 + rr < a.M && kk < a.K ? a.P.at(b, i0 + rr, kk) : 0.f;
+          qs[rr][e % 32] = j0 + rr < a.N && kk < a.K ? a.Q.at(b, j0 + rr, kk) : 0.f;
+        }
+        __syncthreads();
+        const int kn = (int)min((int64_t)32, a.K - k0);
+        for (int kk = 0; kk < kn; ++kk)
+#pragma unroll
+          for (int x = 0; x < 8; ++x) v[x] = fmaf(ps[r][kk], qs[c + x][kk], v[x]);
+        __syncthreads();
+      }
+      const int n = (int)min((int64_t)8, a.N - j0 - c);
+      if (i0 + r < a.M && n > 0) {
+        typename Epi::Pre pre;
+        a.epi.load(b, (int)(i0 + r), (int)(j0 + c), 0, n, pre);
+        a.epi.put(b, (int)(i0 + r), (int)(j0 + c), v, 0, n, pre, vo);
+      }
+    }
+  }
+}
+// One product, or two of the same kind (two != nullptr).
+template <class Epi>
+int launch_plain_product(const int* bad, int nb, const PlainProduct<Epi>& one, const PlainProduct<Epi>* two,
+                         hipStream_t stream, bool one_flag = false) {
+  auto tiles = [](const PlainProduct<Epi>& a) { return ((a.M + 31) / 32) * ((a.N + 31) / 32); };
+  const int64_t t = std::max(tiles(one), two ? tiles(*two) : 0);
+  const unsigned gx = (unsigned)std::min<int64_t>(t, 2 * device_cus());
+  hipLaunchKernelGGL((plain_product_kernel<Epi>), dim3(gx, two ? 2 : 1), dim3(128), 0, stream, bad, one_flag ? 0 : 1, nb, one,
+                     two ? *two : one);
+  PTO_LAUNCHED("plain_product");
+  return 0;
 }
 
 // Zero the pads of up to kPadBufs batched [rows][ld] buffers in one launch:
@@ -144,7 +452,7 @@ struct PadList {
     buf[n++] = Buf{static_cast<uint16_t*>(p), rows, prows, cols, ld, stride, batch};
   }
 };
-static __global__ void __launch_bounds__(256) zero_pads_kernel(PadList l) {
+[[maybe_unused]] static __global__ void __launch_bounds__(256) zero_pads_kernel(PadList l) {
   const PadList::Buf f = l.buf[blockIdx.y];
   const int64_t w = f.ld - f.cols, side = f.rows * w, total = side + (f.prows - f.rows) * f.ld;
   for (int b = blockIdx.z; b < f.batch; b += gridDim.z) {

@@ -99,3 +99,68 @@ def test_ns5_split_non_finite_matrix_only(bad):
     _no_worse(got[0], _ns64(G[0], 5, NS), _ns_chain(G[0], 5, NS))
     Z = torch.zeros(520, 530, device="cuda")
     assert torch.equal(ops.newton_schulz_orthogonalize(Z), Z)
+
+
+# ---------------------------------------------------------------- factor updates
+
+KRON = [(1025, 3500), (2049, 2050), (3001, 1030)]
+
+
+def _kron_plain(L, R, G, beta2, mm):
+    keep, add = (1.0, 1.0) if beta2 == 1.0 else (beta2, 1.0 - beta2)
+    return keep * L + add * mm(G, G), keep * R + add * mm(G.mT, G.mT)
+
+
+@pytest.mark.parametrize("m,n", KRON)
+@pytest.mark.parametrize("beta2", [1.0, 0.95])
+def test_kron_split_error_is_fp32s(m, n, beta2):
+    G, L, R = _randn(m, m, n), _randn(m + 1, m, m), _randn(n + 2, n, n)
+    G[3] *= 1e-12   # a row and a column far below the others keep their own scales
+    G[:, 5] *= 1e-9
+    L, R = L + L.mT, R + R.mT
+    L[3], L[:, 3], R[5], R[:, 5] = 0, 0, 0, 0
+    Lg, Rg = L.cuda(), R.cuda()
+    ops.kron_factor_update_(Lg, Rg, G.cuda(), beta2=beta2)
+    want = _kron_plain(L.double(), R.double(), G.double(), beta2, lambda p, q: p @ q.mT)
+    plain = _kron_plain(L.cuda(), R.cuda(), G.cuda(), beta2, _chain)
+    for got, w, p in zip((Lg, Rg), want, plain):
+        assert torch.equal(got, got.mT)
+        _no_worse(got, w, p)
+    assert _rel(Lg[3], want[0][3]) < 2e-6 and _rel(Rg[5], want[1][5]) < 2e-6
+
+
+def test_kron_split_batch_gives_single_bits_and_non_finite_stays_put():
+    k, m, n = 3, 1030, 3400
+    Gs = [_randn(i, m, n).cuda() for i in range(k)]
+    Gs[1][4, 6], Gs[1][9, 6], Gs[1][11, 8] = math.inf, -math.inf, math.nan
+    Ls, Rs = [torch.zeros(m, m, device="cuda") for _ in range(k)], [torch.zeros(n, n, device="cuda") for _ in range(k)]
+    ops.kron_factor_update_batched_(Ls, Rs, Gs, beta2=1.0)
+    for i in range(k):
+        L1, R1 = torch.zeros(m, m, device="cuda"), torch.zeros(n, n, device="cuda")
+        ops.kron_factor_update_(L1, R1, Gs[i], beta2=1.0)
+        assert torch.equal(Ls[i].nan_to_num(7.0), L1.nan_to_num(7.0)) and torch.equal(Rs[i].nan_to_num(7.0),
+                                                                                      R1.nan_to_num(7.0))
+    G = Gs[1].cpu()
+    for got, plain in ((Ls[1].cpu(), G @ G.mT), (Rs[1].cpu(), G.mT @ G)):
+        for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(kind(got), kind(plain))
+        ok = torch.isfinite(plain)
+        assert _rel(got[ok], plain[ok].double()) < 2e-6
+
+
+@pytest.mark.parametrize("rows,d,ones", [(2000, 2049, True), (8193, 1024, False), (1111, 2751, True)])
+def test_gram_split_error_is_fp32s(rows, d, ones):
+    X = torch.relu(_randn(rows, rows, d, scale=1e3))
+    X[:, 2] = 0.0
+    Xt = torch.cat([X, torch.ones(rows, 1)], 1) if ones else X
+    F = torch.eye(d + ones)
+    got = F.cuda()
+    ops.gram_update_(got, X.cuda(), beta=0.5, alpha=1.0 / rows, append_ones=ones)
+    assert torch.equal(got, got.mT)
+    _no_worse(got, 0.5 * F.double() + (Xt.double().mT @ Xt.double()) / rows, 0.5 * F.cuda() + _chain(Xt.mT, Xt.mT) * (1.0 / rows))
+    X[1, 3] = math.nan
+    ops.gram_update_(got, X.cuda(), beta=0.5, alpha=1.0 / rows, append_ones=ones)
+    hit = torch.zeros(d + ones, d + ones, dtype=torch.bool)
+    hit[3], hit[:, 3] = True, True
+    assert torch.equal(torch.isnan(got).cpu(), hit)
+
