@@ -4,7 +4,7 @@
 // (pytorch_opt/ops/__init__.py:81-84, csrc/pytorch_opt_ops.cpp:96-99),
 // following pytorch_opt/ops/reference.py:117-121: out = (L_root·G)·R_root,
 // associated left to right with the intermediate held in the op dtype.
-// Both products run as MFMA "NT" launches over packed transposes of G and
+// Both products run as MFMA "NT" launches (large fp32 ones on split operands) over packed transposes of G and
 // R_root (an O(n²) pass each, small next to the O(n³) products).
 //
 // The same code serves pto_two_sided_product, out = op(A)·X·op(B) with
@@ -15,12 +15,147 @@
 
 #include "aux_kernels.h"
 #include "gemm_nt.h"
+#include "split.h"
 
 namespace pto {
 namespace {
 
+// ------------------------------------------------ fp32 on split operands
+//
+// Both products on the fp16 MFMA (split.h). op(A)'s planes carry a scale per
+// row, X's one per column, so the raw sums of op(A)·X carry both, and are at
+// most K·2^28: scaled by 2^-(14 + log2 K) they are the planes of the second
+// product's left operand as they stand. The column scales, which that product
+// contracts over, go into op(B)'s rows before op(B)'s own column scales are
+// taken, so a column of X far smaller than the others keeps its weight.
+// From a short side of 512 and this work up: below, the passes for the scales
+// and five more launches cost what the products save (one 1300² 127 us against
+// 117 on the fp32 MFMA, one 4096 x 512 178 against 161, 8 x 256 x 4096 850
+// against 749; 8 x 512 x 2048 314 against 384, 8 x 1024² 202 against 284, one
+// 2048² 180 against 282, eight 942 against 2068, one 4096² 749 against 2006).
+constexpr int64_t kApplySplitSide = 512;
+constexpr double kApplySplitWork = 1.2e10;  // batch·m·n·(m + n)
+inline bool apply_split(int64_t batch, int64_t m, int64_t n) {
+  return std::min(m, n) >= kApplySplitSide && (double)batch * m * n * (m + n) >= kApplySplitWork;
+}
+
+struct ApplySplitWs {
+  sp16 *A, *XT, *AX, *B;
+  unsigned* part;
+  int *bad, *ea, *ex, *eb;
+  int64_t mw, nw;
+  template <class Take>
+  void layout(Take&& take, int64_t m, int64_t n, int64_t nx, int64_t na) {
+    const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
+    mw = round_up(m, 8);
+    nw = round_up(n, 8);
+    take(A, 2 * na * m * ldm);
+    take(XT, 2 * nx * n * ldm);
+    take(AX, 2 * nx * m * ldn);
+    take(B, 2 * nx * n * ldn);
+    // one operand's parts at a time: as many as its rows' or columns'
+    const int64_t pa = na * mw * std::max(absmax_row_parts(m), absmax_col_parts(m));
+    const int64_t px = nx * nw * absmax_col_parts(m);
+    const int64_t pb = nx * nw * std::max(absmax_row_parts(n), absmax_col_parts(n));
+    take(part, std::max(pa, std::max(px, pb)));
+    take(bad, 1);
+    take(ea, na * mw);
+    take(ex, nx * nw);
+    take(eb, nx * nw);
+  }
+  static size_t bytes(int64_t m, int64_t n, int64_t nx, int64_t na) {
+    ApplySplitWs w;
+    size_t total = 256;
+    w.layout([&](auto*& p, int64_t count) { total = round_up(total, 256) + sizeof(*p) * (size_t)count; }, m, n, nx, na);
+    return total + 256;
+  }
+};
+
+// The raw sums of op(A)·X, scaled by 2^sh, as planes
+struct EpiPlanes {
+  typedef float S;
+  sp16* dst;
+  int64_t pl, ld, sd;
+  int sh;
+  typedef NoPre Pre;
+  typedef NoPre PreT;
+  static constexpr bool kVoIsV = true;
+  __device__ __forceinline__ bool has_t() const { return false; }
+  __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
+    S w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      w[k] = ldexpf(v[k], sh);
+      vo[k] = v[k];
+    }
+    st8_split(dst + (int64_t)b * sd + (int64_t)i * ld + j0, pl, w, kbeg, n);
+  }
+  __device__ __forceinline__ void put_t(int, int, int, const S*, int, const PreT&) const {}
+  __device__ __forceinline__ void finish(int) const {}
+};
+
+int two_sided_split(const float* Am, const float* X, const float* Bm, float* out, int64_t batch, int64_t m, int64_t n,
+                    int64_t sA, int64_t sX, int64_t sB, bool trans_a, bool trans_b, void* ws, size_t ws_bytes,
+                    hipStream_t stream, const char* name_left, const char* name_right) {
+  const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
+  const int nb = (int)batch, na = sA ? nb : 1;
+  Carver cv(ws, ws_bytes);
+  ApplySplitWs w;
+  w.layout([&](auto*& p, int64_t count) { p = cv.take<std::remove_reference_t<decltype(*p)>>(count); }, m, n, batch, na);
+  PTO_REQUIRE(!cv.overflow, "two-sided product: workspace too small");
+  if (launch_fill<int>(w.bad, 1, 0, stream)) return -1;
+  // planes of rows (straight) or of columns (transposed) of one operand
+  auto pack = [&](const float* in, int64_t r, int64_t c, int64_t s_in, bool t, sp16* o, int64_t ld, int* e, int64_t ew,
+                  const int* pre, int cnt) {
+    const int64_t orows = t ? c : r;
+    SplitPack p{in, r, c, c, s_in, t ? nullptr : w.part, t ? w.part : nullptr, t ? 0 : ew, t ? ew : 0,
+                t ? nullptr : e, t ? e : nullptr, w.bad, t ? nullptr : o, orows * ld, ld, 2 * orows * ld,
+                t ? o : nullptr, orows * ld, ld, 2 * orows * ld, 0};
+    p.pre_r = t ? pre : nullptr;
+    p.pre_c = t ? nullptr : pre;
+    p.s_pre = w.nw;
+    p.one_flag = 1;
+    return launch_split_pack_max(p, cnt, stream, false);
+  };
+  if (pack(Am, m, m, sA, trans_a, w.A, ldm, w.ea, w.mw, nullptr, na)) return -1;
+  if (pack(X, m, n, sX, true, w.XT, ldm, w.ex, w.nw, nullptr, nb)) return -1;
+  if (pack(Bm, n, n, sB, !trans_b, w.B, ldn, w.eb, w.nw, w.ex, nb)) return -1;
+  PadList pads;
+  pads.add(w.AX, m, m, n, ldn, m * ldn, 2 * nb);
+  if (launch_zero_pads(pads, stream)) return -1;
+  int lk = 0;
+  while ((int64_t(1) << lk) < m) ++lk;
+  const int sh = -(kSplitTop + lk);
+  {
+    GemmArgs g{w.A, ldm, na > 1 ? 2 * m * ldm : 0, w.XT, ldm, 2 * n * ldm, (int)m, (int)n, (int)ldm, 0, 0, w.bad, 0, 0,
+               m * ldm, n * ldm};
+    const EpiPlanes e{w.AX, m * ldn, ldn, 2 * m * ldn, sh};
+    if (launch_gemm<sp16, false>(g, e, nb, stream, name_left)) return -1;
+  }
+  {
+    GemmArgs g{w.AX, ldn, 2 * m * ldn, w.B, ldn, 2 * n * ldn, (int)m, (int)n, (int)ldn, 0, 0, w.bad, 0, 0, m * ldn,
+               n * ldn};
+    EpiDescale<EpiStore<float, float>> e{{out, n, m * n}, w.ea, w.eb, na > 1 ? w.mw : 0, w.nw};
+    e.off = -sh;
+    if (launch_gemm<sp16, false>(g, e, nb, stream, name_right)) return -1;
+  }
+  // a non-finite value anywhere: both products in plain fp32, op(A)·X where its planes would be
+  float* AX = reinterpret_cast<float*>(w.AX);
+  typedef EpiStore<float, float> Store;
+  const PlainOperand a{Am, trans_a ? 1 : m, trans_a ? m : 1, sA, -1}, x{X, 1, n, sX, -1};
+  const PlainOperand ax{AX, ldn, 1, m * ldn, -1}, b{Bm, trans_b ? n : 1, trans_b ? 1 : n, sB, -1};
+  const PlainProduct<Store> left{a, x, m, n, m, Store{AX, ldn, m * ldn}};
+  const PlainProduct<Store> right{ax, b, m, n, n, Store{out, n, m * n}};
+  if (launch_plain_product(w.bad, nb, left, (const PlainProduct<Store>*)nullptr, stream, true)) return -1;
+  return launch_plain_product(w.bad, nb, right, (const PlainProduct<Store>*)nullptr, stream, true);
+}
+
 template <typename T>
 size_t apply_ws_bytes_t(int64_t m, int64_t n, int64_t batch = 1, bool shared_a = false, bool shared_b = false) {
+  if (std::is_same<T, float>::value && apply_split(batch, m, n))
+    return ApplySplitWs::bytes(m, n, batch, shared_a ? 1 : batch);
   int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   size_t bytes = 0;
   auto add = [&](size_t b) { bytes = round_up(bytes, 256) + b; };
@@ -47,6 +182,11 @@ int two_sided_t(const T* Am, const T* X, const T* Bm, T* out, int64_t batch, int
   PTO_REQUIRE(batch >= 0 && batch < 65536, "two-sided product: batch must be below 65536");
   PTO_REQUIRE(sA >= 0 && sX >= 0 && sB >= 0, "two-sided product: negative stride");
   if (m == 0 || n == 0 || batch == 0) return 0;
+  if constexpr (std::is_same<T, float>::value) {
+    if (apply_split(batch, m, n))
+      return two_sided_split(Am, X, Bm, out, batch, m, n, sA, sX, sB, trans_a, trans_b, ws, ws_bytes, stream, name_left,
+                             name_right);
+  }
   const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   const int nb = (int)batch, nA = sA ? nb : 1, nB = sB ? nb : 1;
   Carver cv(ws, ws_bytes);

@@ -164,3 +164,34 @@ def test_gram_split_error_is_fp32s(rows, d, ones):
     hit[3], hit[:, 3] = True, True
     assert torch.equal(torch.isnan(got).cpu(), hit)
 
+
+# ---------------------------------------------------------------- two-sided products
+
+
+def _sides(b, m, n):
+    A, X, B = _randn(m, b, m, m), _randn(m + n, b, m, n, scale=1e-3), _randn(n, b, n, n)
+    return A / math.sqrt(m) + 3 * torch.eye(m), X, B / math.sqrt(n) + 3 * torch.eye(n)
+
+
+@pytest.mark.parametrize("m,n", [(1830, 1900), (560, 4400), (4700, 520), (2049, 1700)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_two_sided_split_error_is_fp32s(m, n, ta, tb):
+    A, X, B = _sides(1, m, n)
+    X[..., 2], X[..., 5], X[:, 3] = 0.0, X[..., 5] * 1e-12, 0.0  # empty and tiny columns, an empty row
+    got = ops.two_sided_product(A[0].cuda(), X[0].cuda(), B[0].cuda(), transpose_a=ta, transpose_b=tb)
+    op = lambda T, t: T.mT if t else T
+    want = op(A[0], ta).double() @ X[0].double() @ op(B[0], tb).double()
+    a, b = op(A[0], ta).cuda(), op(B[0], tb).cuda()
+    _no_worse(got, want, _chain(_chain(a, X[0].cuda().mT), b.mT))
+
+
+def test_two_sided_split_batch_shared_factors_and_non_finite():
+    A, X, B = (t.cuda() for t in _sides(3, 1830, 1840))
+    for a, b in ((A, B), (A[:1], B), (A, B[:1])):
+        got = ops.precond_apply_two_sided(a, X, b)
+        for i in range(3):
+            assert torch.equal(got[i], ops.precond_apply_two_sided(a[i % len(a)], X[i], b[i % len(b)]))
+    X[1, 4, 6] = math.nan
+    got = ops.precond_apply_two_sided(A, X, B)
+    assert torch.isnan(got[1]).all() and torch.isfinite(got[[0, 2]]).all()
+    assert _rel(got[2], (A[2].double() @ X[2].double() @ B[2].double()).cpu()) < 5e-6
