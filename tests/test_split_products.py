@@ -148,7 +148,7 @@ def test_kron_split_batch_gives_single_bits_and_non_finite_stays_put():
         assert _rel(got[ok], plain[ok].double()) < 2e-6
 
 
-@pytest.mark.parametrize("rows,d,ones", [(2000, 2049, True), (8193, 1024, False), (1111, 2751, True)])
+@pytest.mark.parametrize("rows,d,ones", [(2000, 2049, True), (8193, 1024, False), (1111, 2751, True), (16500, 1024, True)])
 def test_gram_split_error_is_fp32s(rows, d, ones):
     X = torch.relu(_randn(rows, rows, d, scale=1e3))
     X[:, 2] = 0.0
