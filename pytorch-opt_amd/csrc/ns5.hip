@@ -531,6 +531,10 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
   // first update reads G while its epilogue writes `out` (with one
   // iteration, the only update), so an aliased call is packed as well.
   const bool direct = QN && !transposed && m == ldm && n == ldn && (g0 & 15) == 0 && !aliased;
+  // all pads are cleared by one launch (one per buffer and side were up to
+  // seven, 3 us each)
+  PadList pads;
+  constexpr int64_t E = sizeof(T) / 2;  // its units
   if (QN && direct) {
     // no pads: X[1] is written in full by the first update
   } else if (QN) {
@@ -542,9 +546,8 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
         return -1;
     }
     // pad columns of the pong buffer, pad rows of both
-    if (launch_zero_cols<T>(X[1], m, ldn, n, sX, nb, stream)) return -1;
-    for (int i = 0; i < 2; ++i)
-      if (launch_zero_cols<T>(X[i] + m * ldn, ldm - m, ldn, 0, sX, nb, stream)) return -1;
+    pads.add(X[1], m, ldm, n * E, ldn * E, sX * E, nb);
+    pads.add(X[0], m, ldm, ldn * E, ldn * E, sX * E, nb);
   } else {
     if (!transposed) {
       if (launch_pack<T, T, A>(G, rows, cols, cols, sG, scale, X[0], ldn, sX, XT[0], ldm, n * ldm, false, nb, stream))
@@ -553,12 +556,10 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
       if (launch_pack<T, T, A>(G, rows, cols, cols, sG, scale, XT[0], ldm, n * ldm, X[0], ldn, sX, false, nb, stream))
         return -1;
     }
-    if (launch_zero_cols<T>(XT[1], n, ldm, m, n * ldm, nb, stream)) return -1;
+    pads.add(XT[1], n, n, m * E, ldm * E, n * ldm * E, nb);
   }
-  if (launch_zero_cols<T>(Ab, m, ldm, m, sAB, nb, stream)) return -1;
-  if (launch_zero_cols<T>(Bb, m, ldm, m, sAB, nb, stream)) return -1;
-  if (launch_zero_cols<T>(Ab + m * ldm, ldm - m, ldm, 0, sAB, nb, stream)) return -1;  // pad rows
-  if (launch_zero_cols<T>(Bb + m * ldm, ldm - m, ldm, 0, sAB, nb, stream)) return -1;
+  for (T* p : {Ab, Bb}) pads.add(p, m, ldm, m * E, ldm * E, sAB * E, nb);
+  if (launch_zero_pads(pads, stream)) return -1;
 
   int cur = 0;  // X[cur] (QN) or XT[cur] holds the current iterate
   for (int64_t t = 0; t < steps; ++t) {
