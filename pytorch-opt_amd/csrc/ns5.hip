@@ -59,11 +59,7 @@ struct EpiNsGram {
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
   __device__ __forceinline__ void store(T* p, int b, const S* v, int kbeg, int n) const {
-    if (scale == nullptr) {
-      st8<T, S>(p, v, kbeg, n);
-      return;
-    }
-    const S s2 = scale[b] * scale[b];
+    const S s2 = scale ? scale[b] * scale[b] : S(1);
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = s2 * v[k];
@@ -131,11 +127,7 @@ struct EpiNsUpdate {
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
   __device__ __forceinline__ void store(T* p, int b, const S* v, int kbeg, int n) const {
-    if (scale == nullptr) {
-      st8<T, S>(p, v, kbeg, n);
-      return;
-    }
-    const S s = scale[b];
+    const S s = scale ? scale[b] : S(1);
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = s * v[k];
