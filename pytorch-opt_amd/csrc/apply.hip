@@ -22,17 +22,20 @@ namespace {
 
 // ------------------------------------------------ fp32 on split operands
 //
-// Both products on the fp16 MFMA (split.h). op(A)'s planes carry a scale per
-// row, X's one per column, so the raw sums of op(A)·X carry both, and are at
-// most K·2^28: scaled by 2^-(14 + log2 K) they are the planes of the second
-// product's left operand as they stand. The column scales, which that product
-// contracts over, go into op(B)'s rows before op(B)'s own column scales are
-// taken, so a column of X far smaller than the others keeps its weight.
+// Both products on the fp16 MFMA (split.h). X's planes carry a scale per row
+// and one per column, so that a row or a column far below the others keeps its
+// bits; the row scales, which op(A)·X contracts over, go into op(A)'s columns
+// before op(A)'s own row scales are taken, and the column scales into op(B)'s
+// rows likewise. op(A)·X is kept in fp32 (scaled by both) and packed with a
+// scale per row of its own maxima: with one shift for its largest possible value
+// a row at 1e-6 of the others was 2e-2 off. Without the row scales and that pass
+// 16 x 2048² takes 1.98 ms instead of 2.24.
 // From a short side of 512 and this work up: below, the passes for the scales
-// and five more launches cost what the products save (one 1300² 127 us against
-// 117 on the fp32 MFMA, one 4096 x 512 178 against 161, 8 x 256 x 4096 850
-// against 749; 8 x 512 x 2048 314 against 384, 8 x 1024² 202 against 284, one
-// 2048² 180 against 282, eight 942 against 2068, one 4096² 749 against 2006).
+// and eight more launches cost what the products save (one 1300² 127 us against
+// 117 on the fp32 MFMA, one 4096 x 512 178 against 161, before the row scales;
+// with them 8 x 512 x 2048 345 against 383, 8 x 1024² 238 against 282, one
+// 1024 x 4096 247 against 359, one 2048² 206 against 279, sixteen 2240 against
+// 4076, one 4096² 807 against 2006).
 constexpr int64_t kApplySplitSide = 512;
 constexpr double kApplySplitWork = 1.2e10;  // batch·m·n·(m + n)
 inline bool apply_split(int64_t batch, int64_t m, int64_t n) {
@@ -40,109 +43,85 @@ inline bool apply_split(int64_t batch, int64_t m, int64_t n) {
 }
 
 struct ApplySplitWs {
-  sp16 *A, *XT, *AX, *B;
+  sp16 *A, *XA, *B;  // XA: X's planes, then those of op(A)·X
+  float* AX;
   unsigned* part;
-  int *bad, *ea, *ex, *eb;
+  int *bad, *rx, *ea, *ex, *eb, *eax;
   int64_t mw, nw;
   template <class Take>
-  void layout(Take&& take, int64_t m, int64_t n, int64_t nx, int64_t na) {
+  void layout(Take&& take, int64_t m, int64_t n, int64_t nb) {
     const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
     mw = round_up(m, 8);
     nw = round_up(n, 8);
-    take(A, 2 * na * m * ldm);
-    take(XT, 2 * nx * n * ldm);
-    take(AX, 2 * nx * m * ldn);
-    take(B, 2 * nx * n * ldn);
+    take(A, 2 * nb * m * ldm);  // per matrix also where A is shared: X's scales go in (likewise B)
+    take(XA, 2 * nb * std::max(n * ldm, m * ldn));
+    take(AX, nb * m * ldn);
+    take(B, 2 * nb * n * ldn);
     // one operand's parts at a time: as many as its rows' or columns'
-    const int64_t pa = na * mw * std::max(absmax_row_parts(m), absmax_col_parts(m));
-    const int64_t px = nx * nw * absmax_col_parts(m);
-    const int64_t pb = nx * nw * std::max(absmax_row_parts(n), absmax_col_parts(n));
-    take(part, std::max(pa, std::max(px, pb)));
+    const int64_t pa = mw * std::max(std::max(absmax_row_parts(m), absmax_col_parts(m)), absmax_row_parts(n));
+    const int64_t pb = nw * std::max(std::max(absmax_row_parts(n), absmax_col_parts(n)), absmax_col_parts(m));
+    take(part, nb * std::max(pa, pb));
     take(bad, 1);
-    take(ea, na * mw);
-    take(ex, nx * nw);
-    take(eb, nx * nw);
+    for (int** e : {&rx, &ea, &eax}) take(*e, nb * mw);
+    for (int** e : {&ex, &eb}) take(*e, nb * nw);
   }
-  static size_t bytes(int64_t m, int64_t n, int64_t nx, int64_t na) {
+  static size_t bytes(int64_t m, int64_t n, int64_t nb) {
     ApplySplitWs w;
     size_t total = 256;
-    w.layout([&](auto*& p, int64_t count) { total = round_up(total, 256) + sizeof(*p) * (size_t)count; }, m, n, nx, na);
+    w.layout([&](auto*& p, int64_t count) { total = round_up(total, 256) + sizeof(*p) * (size_t)count; }, m, n, nb);
     return total + 256;
   }
-};
-
-// The raw sums of op(A)·X, scaled by 2^sh, as planes
-struct EpiPlanes {
-  typedef float S;
-  sp16* dst;
-  int64_t pl, ld, sd;
-  int sh;
-  typedef NoPre Pre;
-  typedef NoPre PreT;
-  static constexpr bool kVoIsV = true;
-  __device__ __forceinline__ bool has_t() const { return false; }
-  __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
-  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
-  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
-    S w[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      w[k] = ldexpf(v[k], sh);
-      vo[k] = v[k];
-    }
-    st8_split(dst + (int64_t)b * sd + (int64_t)i * ld + j0, pl, w, kbeg, n);
-  }
-  __device__ __forceinline__ void put_t(int, int, int, const S*, int, const PreT&) const {}
-  __device__ __forceinline__ void finish(int) const {}
 };
 
 int two_sided_split(const float* Am, const float* X, const float* Bm, float* out, int64_t batch, int64_t m, int64_t n,
                     int64_t sA, int64_t sX, int64_t sB, bool trans_a, bool trans_b, void* ws, size_t ws_bytes,
                     hipStream_t stream, const char* name_left, const char* name_right) {
   const int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
-  const int nb = (int)batch, na = sA ? nb : 1;
+  const int nb = (int)batch;
   Carver cv(ws, ws_bytes);
   ApplySplitWs w;
-  w.layout([&](auto*& p, int64_t count) { p = cv.take<std::remove_reference_t<decltype(*p)>>(count); }, m, n, batch, na);
+  w.layout([&](auto*& p, int64_t count) { p = cv.take<std::remove_reference_t<decltype(*p)>>(count); }, m, n, batch);
   PTO_REQUIRE(!cv.overflow, "two-sided product: workspace too small");
-  if (launch_fill<int>(w.bad, 1, 0, stream)) return -1;
-  // planes of rows (straight) or of columns (transposed) of one operand
-  auto pack = [&](const float* in, int64_t r, int64_t c, int64_t s_in, bool t, sp16* o, int64_t ld, int* e, int64_t ew,
-                  const int* pre, int cnt) {
-    const int64_t orows = t ? c : r;
-    SplitPack p{in, r, c, c, s_in, t ? nullptr : w.part, t ? w.part : nullptr, t ? 0 : ew, t ? ew : 0,
-                t ? nullptr : e, t ? e : nullptr, w.bad, t ? nullptr : o, orows * ld, ld, 2 * orows * ld,
-                t ? o : nullptr, orows * ld, ld, 2 * orows * ld, 0};
+  // planes of the rows (t: of the columns) of one operand, its other index scaled by 2^(off + mul·pre)
+  auto planes = [&](const float* in, int64_t r, int64_t c, int64_t ld_in, int64_t s_in, bool t, sp16* o, int64_t ld,
+                    int* e, int64_t ew, const int* pre, int64_t s_pre, int mul, int off) {
+    const int64_t pl = (t ? c : r) * ld;
+    SplitPack p{in, r, c, ld_in, s_in, t ? nullptr : w.part, t ? w.part : nullptr, ew, ew, t ? nullptr : e,
+                t ? e : nullptr, w.bad, t ? nullptr : o, pl, ld, 2 * pl, t ? o : nullptr, pl, ld, 2 * pl, 0};
     p.pre_r = t ? pre : nullptr;
     p.pre_c = t ? nullptr : pre;
-    p.s_pre = w.nw;
+    p.s_pre = s_pre;
+    p.pre_mul = mul;
+    p.pre_off = off;
     p.one_flag = 1;
-    return launch_split_pack_max(p, cnt, stream, false);
+    return p;
   };
-  if (pack(Am, m, m, sA, trans_a, w.A, ldm, w.ea, w.mw, nullptr, na)) return -1;
-  if (pack(X, m, n, sX, true, w.XT, ldm, w.ex, w.nw, nullptr, nb)) return -1;
-  if (pack(Bm, n, n, sB, !trans_b, w.B, ldn, w.eb, w.nw, w.ex, nb)) return -1;
-  PadList pads;
-  pads.add(w.AX, m, m, n, ldn, m * ldn, 2 * nb);
-  if (launch_zero_pads(pads, stream)) return -1;
-  int lk = 0;
-  while ((int64_t(1) << lk) < m) ++lk;
-  const int sh = -(kSplitTop + lk);
+  auto pack = [&](const SplitPack& p) { return launch_split_pack_max(p, nb, stream, false); };
+  if (launch_row_exp(X, m, n, n, sX, nb, w.rx, w.mw, w.bad, stream)) return -1;
+  if (pack(planes(X, m, n, n, sX, true, w.XA, ldm, w.ex, w.nw, w.rx, w.mw, 1, 0))) return -1;
+  if (pack(planes(Am, m, m, m, sA, trans_a, w.A, ldm, w.ea, w.mw, w.rx, w.mw, -1, kSplitTop))) return -1;
+  if (pack(planes(Bm, n, n, n, sB, !trans_b, w.B, ldn, w.eb, w.nw, w.ex, w.nw, -1, 0))) return -1;
   {
-    GemmArgs g{w.A, ldm, na > 1 ? 2 * m * ldm : 0, w.XT, ldm, 2 * n * ldm, (int)m, (int)n, (int)ldm, 0, 0, w.bad, 0, 0,
-               m * ldm, n * ldm};
-    const EpiPlanes e{w.AX, m * ldn, ldn, 2 * m * ldn, sh};
+    GemmArgs g{w.A, ldm, 2 * m * ldm, w.XA, ldm, 2 * n * ldm, (int)m, (int)n, (int)ldm, 0, 0, w.bad, 0, 0, m * ldm,
+               n * ldm};
+    const EpiStore<float, float> e{w.AX, ldn, m * ldn};
     if (launch_gemm<sp16, false>(g, e, nb, stream, name_left)) return -1;
   }
   {
-    GemmArgs g{w.AX, ldn, 2 * m * ldn, w.B, ldn, 2 * n * ldn, (int)m, (int)n, (int)ldn, 0, 0, w.bad, 0, 0, m * ldn,
+    SplitPack p = planes(w.AX, m, n, ldn, m * ldn, false, w.XA, ldn, w.eax, w.mw, nullptr, 0, 0, 0);
+    p.er_add = w.ea;
+    p.bad = nullptr;
+    if (pack(p)) return -1;
+  }
+  {
+    GemmArgs g{w.XA, ldn, 2 * m * ldn, w.B, ldn, 2 * n * ldn, (int)m, (int)n, (int)ldn, 0, 0, w.bad, 0, 0, m * ldn,
                n * ldn};
-    EpiDescale<EpiStore<float, float>> e{{out, n, m * n}, w.ea, w.eb, na > 1 ? w.mw : 0, w.nw};
-    e.off = -sh;
+    EpiDescale<EpiStore<float, float>> e{{out, n, m * n}, w.eax, w.eb, w.mw, w.nw};
+    e.off = -kSplitTop;
     if (launch_gemm<sp16, false>(g, e, nb, stream, name_right)) return -1;
   }
-  // a non-finite value anywhere: both products in plain fp32, op(A)·X where its planes would be
-  float* AX = reinterpret_cast<float*>(w.AX);
+  // a flagged value anywhere: both products in plain fp32
+  float* AX = w.AX;
   typedef EpiStore<float, float> Store;
   const PlainOperand a{Am, trans_a ? 1 : m, trans_a ? m : 1, sA, -1}, x{X, 1, n, sX, -1};
   const PlainOperand ax{AX, ldn, 1, m * ldn, -1}, b{Bm, trans_b ? n : 1, trans_b ? 1 : n, sB, -1};
@@ -154,8 +133,7 @@ int two_sided_split(const float* Am, const float* X, const float* Bm, float* out
 
 template <typename T>
 size_t apply_ws_bytes_t(int64_t m, int64_t n, int64_t batch = 1, bool shared_a = false, bool shared_b = false) {
-  if (std::is_same<T, float>::value && apply_split(batch, m, n))
-    return ApplySplitWs::bytes(m, n, batch, shared_a ? 1 : batch);
+  if (std::is_same<T, float>::value && apply_split(batch, m, n)) return ApplySplitWs::bytes(m, n, batch);
   int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   size_t bytes = 0;
   auto add = [&](size_t b) { bytes = round_up(bytes, 256) + b; };

@@ -13,11 +13,11 @@
 
 namespace pto {
 
-// Exponent e with max·2^e in (2^13, 2^14] for a finite bound max > 0. Non-finite
+// Exponent e with max·2^e in [2^13, 2^14) for a finite bound max > 0. Non-finite
 // operands never reach the products that read these planes; an empty row or
-// column says "tiny" (its values are all zero, and where its exponent scales
-// another operand's row that row must not outweigh the others).
-constexpr int kSplitTop = 14, kSplitZero = 120;
+// column has kSplitZero, which makes a zero of whatever another operand holds
+// against it.
+constexpr int kSplitTop = 14, kSplitZero = 1000;
 __device__ __forceinline__ int split_exp(float bound) {
   int k = 0;
   if (bound == 0.f) return kSplitZero;
@@ -131,102 +131,18 @@ __device__ __forceinline__ void st8_split(sp16* p, int64_t pl, const float* in, 
   }
 }
 
-// Largest |x| of the parts of a fp32 matrix's rows and columns, as bit patterns
-// (which order like the values, NaN above infinity): rpart[cb][r] of columns
-// 256·cb .. + 255, cpart[rb][c] of rows nr·rb .. + nr - 1; either may be null.
-// A workgroup takes nr rows (a multiple of 32) x 256 columns, a wave eight
-// rows at a time, 16 bytes per lane and all eight in flight (one row at a time
-// waited 32 times for memory: 30 us whatever the size). Parts need neither
-// zeroing nor atomics. Bound by memory: 4 bytes per element. Also clears
-// bad[b] (bad != nullptr). pre: x counts as x·2^-pre, pre per row or per column.
-[[maybe_unused]] static __global__ void __launch_bounds__(256) absmax_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
-                                                     int64_t ld, int64_t s_in, int nr, unsigned* __restrict__ rpart,
-                                                     int64_t mw, unsigned* __restrict__ cpart, int64_t nw,
-                                                     int* __restrict__ bad, const int* __restrict__ pre_r,
-                                                     const int* __restrict__ pre_c, int64_t s_pre) {
-  __shared__ unsigned cw[4][256];
-  const int b = blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t r0 = (int64_t)blockIdx.y * nr, c0 = (int64_t)blockIdx.x * 256 + lane * 4;
-  const float* ib = in + (int64_t)b * s_in;
-  if (bad && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) bad[b] = 0;
-  int pc[4] = {0, 0, 0, 0};
-  if (pre_c)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) pc[k] = c0 + k < cols ? pre_c[(int64_t)b * s_pre + c0 + k] : 0;
-  unsigned cm[4] = {0, 0, 0, 0};
-  for (int rr = wave * 8; rr < nr; rr += 32) {
-    uint4 q[8];
-    unsigned rm[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t r = r0 + rr + i;
-      q[i] = make_uint4(0, 0, 0, 0);
-      if (r < rows) {
-        if (c0 + 4 <= cols) {
-          q[i] = ld16(ib + r * ld + c0);
-        } else {
-          if (c0 < cols) q[i].x = __float_as_uint(ib[r * ld + c0]);
-          if (c0 + 1 < cols) q[i].y = __float_as_uint(ib[r * ld + c0 + 1]);
-          if (c0 + 2 < cols) q[i].z = __float_as_uint(ib[r * ld + c0 + 2]);
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      unsigned u[4] = {q[i].x & 0x7fffffffu, q[i].y & 0x7fffffffu, q[i].z & 0x7fffffffu, q[i].w & 0x7fffffffu};
-      if (pre_r || pre_c) {
-        const int64_t r = r0 + rr + i;
-        const int pr = pre_r && r < rows ? pre_r[(int64_t)b * s_pre + r] : 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) u[k] = __float_as_uint(ldexpf(__uint_as_float(u[k]), -pr - pc[k]));
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) cm[k] = max(cm[k], u[k]);
-      rm[i] = max(max(u[0], u[1]), max(u[2], u[3]));
-    }
-    if (rpart) {
-      // eight rows over 64 lanes: three exchanges that halve the rows a lane
-      // holds, three more within its eight lanes (10 shuffles for 48)
-      unsigned m4[4], m2[2];
-      const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        m4[i] = max(b5 ? rm[i + 4] : rm[i], (unsigned)__shfl_xor((int)(b5 ? rm[i] : rm[i + 4]), 32, 64));
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        m2[i] = max(b4 ? m4[i + 2] : m4[i], (unsigned)__shfl_xor((int)(b4 ? m4[i] : m4[i + 2]), 16, 64));
-      unsigned m = max(b3 ? m2[1] : m2[0], (unsigned)__shfl_xor((int)(b3 ? m2[0] : m2[1]), 8, 64));
-#pragma unroll
-      for (int off = 4; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, 64));
-      const int64_t r = r0 + rr + 4 * b5 + 2 * b4 + b3;
-      if ((lane & 7) == 0 && r < rows) rpart[((int64_t)b * gridDim.x + blockIdx.x) * mw + r] = m;
-    }
-  }
-  if (!cpart) return;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) cw[wave][lane * 4 + k] = cm[k];
-  __syncthreads();
-  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (c < cols)
-    cpart[((int64_t)b * gridDim.y + blockIdx.y) * nw + c] =
-        max(max(cw[0][threadIdx.x], cw[1][threadIdx.x]), max(cw[2][threadIdx.x], cw[3][threadIdx.x]));
-}
-// Parts of a matrix: row parts per 256 columns; column parts per 64 rows (256
-// rows a workgroup ran 4096² at 53 us for 15.5, one workgroup per CU), and at
-// most 64 of them, since every tile of the packing pass reads all of its
-// columns' parts.
-inline int absmax_rows(int64_t rows) { return rows <= 4096 ? 64 : (int)round_up((rows + 63) / 64, 32); }
-inline int64_t absmax_row_parts(int64_t cols) { return (cols + 255) / 256; }
-inline int64_t absmax_col_parts(int64_t rows) { return (rows + absmax_rows(rows) - 1) / absmax_rows(rows); }
-
 constexpr unsigned kInfBits = 0x7f800000u;
+constexpr unsigned kTinyBits = 0x0d800000u;  // 2^-100
 
-// Planes of a fp32 matrix in either or both layouts, from one read:
-//   out_s [rows][ld_s]: in(r, c)·2^er(r), out_t [cols + ones][ld_t]:
-//   in(r, c)·2^ec(c) transposed (with `ones`, a last row of ones),
-// pad columns zero, er and ec the split exponents of the parts' maxima, which
-// are stored too (batch strides mw, nw). A row or column with a non-finite
-// value sets bad[b].
+// Planes of a fp32 matrix in either or both layouts:
+//   out_s [rows][ld_s]: in(r, c)·2^(er(r) + pre), out_t [cols + ones][ld_t]:
+//   in(r, c)·2^(ec(c) + pre) transposed (with `ones`, a last row of ones),
+// pad columns zero, er and ec the split exponents of the maxima of
+// in(r, c)·2^pre, which are stored too (batch strides mw, nw; er plus er_add's).
+// pre = pre_off + pre_mul·(pre_r(r) or pre_c(c)): the scales that another
+// operand's rows carry, taken out of this one. A row or column with a
+// non-finite value, or whose maximum 2^pre takes to the ends of the fp32 range,
+// sets bad[b].
 struct SplitPack {
   const float* in;
   int64_t rows, cols, ld_in, s_in;
@@ -241,16 +157,111 @@ struct SplitPack {
   sp16* out_t;
   int64_t pl_t, ld_t, s_t;
   int ones;
-  // x is taken as x·2^-pre (after absmax's reading of the parts alike)
   const int* pre_r = nullptr;
   const int* pre_c = nullptr;
   int64_t s_pre = 0;
-  int one_flag = 0;  // bad is one word for the whole batch, cleared by the caller's first pack only
+  int pre_mul = 0, pre_off = 0;
+  const int* er_add = nullptr;  // stride mw
+  int one_flag = 0;  // bad is one word for the whole batch, cleared by the caller
+  __device__ __forceinline__ int pre(const int* p, int b, int64_t at, int64_t n) const {
+    return p && at < n ? pre_off + pre_mul * p[(int64_t)b * s_pre + at] : 0;
+  }
 };
+
+// |x|·2^e by bit patterns: what is not finite and what is not zero stay so,
+// but for the rows of an empty one (|e| near kSplitZero).
+__device__ __forceinline__ unsigned scaled_bits(unsigned u, int e) {
+  if (u >= kInfBits || u == 0) return u;
+  if (e < -kSplitZero / 2) return 0;
+  return max(1u, __float_as_uint(ldexpf(__uint_as_float(u), e)));
+}
+
+// Largest |x| of the parts of a fp32 matrix's rows and columns, as bit patterns
+// (which order like the values, NaN above infinity): rpart[cb][r] of columns
+// 256·cb .. + 255, cpart[rb][c] of rows nr·rb .. + nr - 1; written where out_s
+// (out_t) is. A workgroup takes nr rows (a multiple of 32) x 256 columns, a wave
+// eight rows at a time, 16 bytes per lane and all eight in flight (one row at a
+// time waited 32 times for memory: 30 us whatever the size). Parts need neither
+// zeroing nor atomics. Bound by memory: 4 bytes per element. clear: also clears
+// bad[b].
+[[maybe_unused]] static __global__ void __launch_bounds__(256) absmax_kernel(SplitPack a, int nr, int clear) {
+  __shared__ unsigned cw[4][256];
+  const int b = blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t r0 = (int64_t)blockIdx.y * nr, c0 = (int64_t)blockIdx.x * 256 + lane * 4;
+  const float* ib = a.in + (int64_t)b * a.s_in;
+  if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.bad[b] = 0;
+  int pc[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) pc[k] = a.pre(a.pre_c, b, c0 + k, a.cols);
+  unsigned cm[4] = {0, 0, 0, 0};
+  for (int rr = wave * 8; rr < nr; rr += 32) {
+    uint4 q[8];
+    unsigned rm[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int64_t r = r0 + rr + i;
+      q[i] = make_uint4(0, 0, 0, 0);
+      if (r < a.rows) {
+        if (c0 + 4 <= a.cols) {
+          q[i] = ld16(ib + r * a.ld_in + c0);
+        } else {
+          if (c0 < a.cols) q[i].x = __float_as_uint(ib[r * a.ld_in + c0]);
+          if (c0 + 1 < a.cols) q[i].y = __float_as_uint(ib[r * a.ld_in + c0 + 1]);
+          if (c0 + 2 < a.cols) q[i].z = __float_as_uint(ib[r * a.ld_in + c0 + 2]);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      unsigned u[4] = {q[i].x & 0x7fffffffu, q[i].y & 0x7fffffffu, q[i].z & 0x7fffffffu, q[i].w & 0x7fffffffu};
+      if (a.pre_r || a.pre_c) {
+        const int pr = a.pre(a.pre_r, b, r0 + rr + i, a.rows);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) u[k] = scaled_bits(u[k], pr + pc[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) cm[k] = max(cm[k], u[k]);
+      rm[i] = max(max(u[0], u[1]), max(u[2], u[3]));
+    }
+    if (a.out_s) {
+      // eight rows over 64 lanes: three exchanges that halve the rows a lane
+      // holds, three more within its eight lanes (10 shuffles for 48)
+      unsigned m4[4], m2[2];
+      const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        m4[i] = max(b5 ? rm[i + 4] : rm[i], (unsigned)__shfl_xor((int)(b5 ? rm[i] : rm[i + 4]), 32, 64));
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        m2[i] = max(b4 ? m4[i + 2] : m4[i], (unsigned)__shfl_xor((int)(b4 ? m4[i] : m4[i + 2]), 16, 64));
+      unsigned m = max(b3 ? m2[1] : m2[0], (unsigned)__shfl_xor((int)(b3 ? m2[0] : m2[1]), 8, 64));
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, 64));
+      const int64_t r = r0 + rr + 4 * b5 + 2 * b4 + b3;
+      if ((lane & 7) == 0 && r < a.rows) a.rpart[((int64_t)b * gridDim.x + blockIdx.x) * a.mw + r] = m;
+    }
+  }
+  if (!a.out_t) return;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) cw[wave][lane * 4 + k] = cm[k];
+  __syncthreads();
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c < a.cols)
+    a.cpart[((int64_t)b * gridDim.y + blockIdx.y) * a.nw + c] =
+        max(max(cw[0][threadIdx.x], cw[1][threadIdx.x]), max(cw[2][threadIdx.x], cw[3][threadIdx.x]));
+}
+// Parts of a matrix: row parts per 256 columns; column parts per 64 rows (256
+// rows a workgroup ran 4096² at 53 us for 15.5, one workgroup per CU), and at
+// most 64 of them, since every tile of the packing pass reads all of its
+// columns' parts.
+inline int absmax_rows(int64_t rows) { return rows <= 4096 ? 64 : (int)round_up((rows + 63) / 64, 32); }
+inline int64_t absmax_row_parts(int64_t cols) { return (cols + 255) / 256; }
+inline int64_t absmax_col_parts(int64_t rows) { return (rows + absmax_rows(rows) - 1) / absmax_rows(rows); }
+
 [[maybe_unused]] static __global__ void __launch_bounds__(256) split_pack_max_kernel(SplitPack a, int row_parts, int col_parts) {
   __shared__ float tile[64][65];
   __shared__ unsigned mx[4][64];
-  __shared__ int xr[64], xc[64];
+  __shared__ int xr[64], xc[64], pr[64], pc[64];
   const int b = blockIdx.z;
   const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
   const float* ib = a.in + (int64_t)b * a.s_in;
@@ -260,13 +271,11 @@ struct SplitPack {
     const int rr = ty + 4 * i;
     const int64_t r = r0 + rr, c = c0 + tx;
     float x = a.ones && r < a.rows && c == a.cols ? 1.f : 0.f;
-    if (r < a.rows && c < a.cols) {
-      x = ib[r * a.ld_in + c];
-      if (a.pre_r) x = ldexpf(x, -a.pre_r[(int64_t)b * a.s_pre + r]);
-      if (a.pre_c) x = ldexpf(x, -a.pre_c[(int64_t)b * a.s_pre + c]);
-    }
+    if (r < a.rows && c < a.cols) x = ib[r * a.ld_in + c];
     tile[rr][tx] = x;
   }
+  if (ty == 0) pr[tx] = a.pre(a.pre_r, b, r0 + tx, a.rows);
+  if (ty == 1) pc[tx] = a.pre(a.pre_c, b, c0 + tx, a.cols);
   // the tile's exponents: waves 0, 1 its rows' parts, waves 2, 3 its columns'
   {
     const bool row = ty < 2;
@@ -280,16 +289,20 @@ struct SplitPack {
     mx[ty][tx] = m;
   }
   __syncthreads();
+  auto check = [&](unsigned u) {
+    if (a.bad && (u >= kInfBits || ((a.pre_r || a.pre_c) && u != 0 && u < kTinyBits))) a.bad[a.one_flag ? 0 : b] = 1;
+  };
   if (ty == 0 && a.out_s) {
     const unsigned u = max(mx[0][tx], mx[1][tx]);
     xr[tx] = split_exp(__uint_as_float(u));
-    if (blockIdx.x == 0 && r0 + tx < a.rows) a.er[(int64_t)b * a.mw + r0 + tx] = xr[tx];
-    if (u >= kInfBits) a.bad[a.one_flag ? 0 : b] = 1;
+    const int64_t at = (int64_t)b * a.mw + r0 + tx;
+    if (blockIdx.x == 0 && r0 + tx < a.rows) a.er[at] = xr[tx] + (a.er_add ? a.er_add[at] : 0);
+    check(u);
   } else if (ty == 1 && a.out_t) {
     const unsigned u = max(mx[2][tx], mx[3][tx]);
     xc[tx] = split_exp(__uint_as_float(u));
     if (blockIdx.y == 0 && c0 + tx < a.cols + a.ones) a.ec[(int64_t)b * a.nw + c0 + tx] = xc[tx];
-    if (u >= kInfBits) a.bad[a.one_flag ? 0 : b] = 1;
+    check(u);
   }
   __syncthreads();
   for (int q = threadIdx.x; q < 64 * 8; q += 256) {
@@ -297,7 +310,7 @@ struct SplitPack {
     float v[8];
     if (a.out_s && r0 + u < a.rows && c0 + w < a.ld_s) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = c0 + w + k < a.cols ? ldexpf(tile[u][w + k], xr[u]) : 0.f;
+      for (int k = 0; k < 8; ++k) v[k] = c0 + w + k < a.cols ? ldexpf(tile[u][w + k], xr[u] + pr[u] + pc[w + k]) : 0.f;
       const Split8 s = split8(v);
       sp16* o = a.out_s + (int64_t)b * a.s_s + (r0 + u) * a.ld_s + c0 + w;
       *reinterpret_cast<uint4*>(o) = s.h;
@@ -305,7 +318,7 @@ struct SplitPack {
     }
     if (a.out_t && c0 + u < a.cols + a.ones && r0 + w < a.ld_t) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = ldexpf(tile[w + k][u], xc[u]);
+      for (int k = 0; k < 8; ++k) v[k] = ldexpf(tile[w + k][u], xc[u] + pc[u] + pr[w + k]);
       const Split8 s = split8(v);
       sp16* o = a.out_t + (int64_t)b * a.s_t + (c0 + u) * a.ld_t + r0 + w;
       *reinterpret_cast<uint4*>(o) = s.h;
@@ -320,12 +333,42 @@ inline int launch_split_pack_max(const SplitPack& a, int batch, hipStream_t stre
   const int64_t cext = std::max(a.cols + a.ones, a.out_s ? a.ld_s : 0);
   const dim3 gp((unsigned)((cext + 63) / 64), (unsigned)((rext + 63) / 64), (unsigned)batch);
   PTO_REQUIRE(gm.y < 65536 && gp.y < 65536 && batch < 65536, "split_pack: grid too large");
-  hipLaunchKernelGGL(absmax_kernel, gm, dim3(256), 0, stream, a.in, a.rows, a.cols, a.ld_in, a.s_in, nr,
-                     a.out_s ? a.rpart : nullptr, a.mw, a.out_t ? a.cpart : nullptr, a.nw, clear ? a.bad : nullptr,
-                     a.pre_r, a.pre_c, a.s_pre);
+  hipLaunchKernelGGL(absmax_kernel, gm, dim3(256), 0, stream, a, nr, clear ? 1 : 0);
   PTO_LAUNCHED("absmax");
   hipLaunchKernelGGL(split_pack_max_kernel, gp, dim3(256), 0, stream, a, (int)gm.x, (int)gm.y);
   PTO_LAUNCHED("split_pack_max");
+  return 0;
+}
+
+// Split exponents of the rows of a fp32 matrix: e[b·ew + r]. A wave takes a row,
+// 16 bytes per lane and four runs in flight. Bound by memory: 4 bytes per
+// element. Also clears bad[0].
+[[maybe_unused]] static __global__ void __launch_bounds__(256) row_exp_kernel(const float* __restrict__ in, int64_t rows,
+                                                                              int64_t cols, int64_t ld, int64_t s_in,
+                                                                              int* __restrict__ e, int64_t ew,
+                                                                              int* __restrict__ bad) {
+  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  if (blockIdx.x == 0 && b == 0 && threadIdx.x == 0) bad[0] = 0;
+  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= rows) return;
+  const float* row = in + (int64_t)b * s_in + r * ld;
+  unsigned m = 0;
+#pragma unroll 4
+  for (int64_t c = lane * 4; c + 4 <= cols; c += 256) {
+    const uint4 u = ld16(row + c);
+    m = max(max(m, u.x & 0x7fffffffu), max(max(u.y & 0x7fffffffu, u.z & 0x7fffffffu), u.w & 0x7fffffffu));
+  }
+  const int64_t t = cols / 4 * 4 + lane;
+  if (t < cols) m = max(m, __float_as_uint(row[t]) & 0x7fffffffu);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, 64));
+  if (lane == 0) e[(int64_t)b * ew + r] = split_exp(__uint_as_float(m));
+}
+inline int launch_row_exp(const float* in, int64_t rows, int64_t cols, int64_t ld, int64_t s_in, int batch, int* e,
+                          int64_t ew, int* bad, hipStream_t stream) {
+  hipLaunchKernelGGL(row_exp_kernel, dim3((unsigned)((rows + 3) / 4), (unsigned)batch), dim3(256), 0, stream, in, rows,
+                     cols, ld, s_in, e, ew, bad);
+  PTO_LAUNCHED("row_exp");
   return 0;
 }
 

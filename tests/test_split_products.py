@@ -195,3 +195,107 @@ def test_two_sided_split_batch_shared_factors_and_non_finite():
     got = ops.precond_apply_two_sided(A, X, B)
     assert torch.isnan(got[1]).all() and torch.isfinite(got[[0, 2]]).all()
     assert _rel(got[2], (A[2].double() @ X[2].double() @ B[2].double()).cpu()) < 5e-6
+
+
+# Row by row and entry by entry: a row far below the others keeps the error that
+# plain fp32 sums leave it.
+
+
+def _err(x, want, dim=-1):
+    """Relative error of every row (or column) that is not empty; an empty one
+    has to come out empty."""
+    x, size = x.double().cpu(), want.norm(dim=dim)
+    err = (x - want).norm(dim=dim)
+    assert (err[size == 0] == 0).all()
+    return err / size.clamp_min(1e-300)
+
+
+def _rows_no_worse(got, want, plain, dim=-1, roundings=4):
+    """One row's error is a sample of a few hundred roundings or more: 1.5 times
+    the plain one's, or `roundings` roundings of the result."""
+    e, p = _err(got, want, dim), _err(plain, want, dim)
+    worst = (e / torch.clamp(1.5 * p, min=roundings * 2.0 ** -24)).argmax()
+    assert (e <= torch.clamp(1.5 * p, min=roundings * 2.0 ** -24)).all(), (int(worst), e.flatten()[worst], p.flatten()[worst])
+
+
+SMALL = {3: 1e-2, 64: 1e-4, 130: 1e-6, 131: 1e-7, 700: 1e-8, 701: 1e-12, 1100: 0.0}
+
+
+@pytest.mark.parametrize("kind", ["identity", "near", "dense"])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_two_sided_split_keeps_small_rows_and_columns(kind, ta, tb):
+    m, n = 1830, 1900
+    A, X, B = (t[0] for t in _sides(1, m, n))
+    X = X * 1e3
+    if kind != "dense":
+        A = torch.eye(m) + (1e-5 * torch.randn(m, m, generator=torch.Generator().manual_seed(1)) if kind == "near" else 0)
+        B = torch.eye(n) + (1e-5 * torch.randn(n, n, generator=torch.Generator().manual_seed(2)) if kind == "near" else 0)
+    for i, s in SMALL.items():
+        X[i] *= s
+        X[:, i + 5] *= s
+    op = lambda T, t: T.mT if t else T
+    got = ops.two_sided_product(A.cuda(), X.cuda(), B.cuda(), transpose_a=ta, transpose_b=tb)
+    a, b = op(A, ta), op(B, tb)
+    want = a.double() @ X.double() @ b.double()
+    plain = _chain(_chain(a, X.mT), b.mT)
+    _rows_no_worse(got, want, plain)
+    _rows_no_worse(got, want, plain, dim=-2)
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-20, 1e18])
+def test_two_sided_split_scale_of_x(scale):
+    A, X, B = (t[0] for t in _sides(1, 1830, 1840))
+    X = X * 1e3 * scale
+    X[7] *= 1e-6
+    want = A.double() @ X.double() @ B.double()
+    got = ops.precond_apply_two_sided(A.cuda(), X.cuda(), B.cuda())
+    _rows_no_worse(got, want, _chain(_chain(A, X.mT), B.mT))
+
+
+@pytest.mark.parametrize("decades", [6, 8, 10])
+def test_two_sided_split_transports_second_moments(decades):
+    # SOAP: v = λ_i·μ_j (and some noise) between two bases that turned a little
+    m, n = 1830, 1900
+    g = torch.Generator().manual_seed(decades)
+
+    def turn(k):
+        s = torch.randn(k, k, generator=g, dtype=torch.float64) * (0.02 / math.sqrt(k))
+        return torch.linalg.qr(torch.eye(k, dtype=torch.float64) + s - s.mT)[0].float().pow(2)
+
+    A, B = turn(m), turn(n)
+    lam = torch.logspace(0, -decades, m, dtype=torch.float64)[torch.randperm(m, generator=g)]
+    mu = torch.logspace(0, -decades, n, dtype=torch.float64)[torch.randperm(n, generator=g)]
+    v = (lam[:, None] * mu * torch.exp(torch.randn(m, n, generator=g, dtype=torch.float64))).float()
+    want = A.double().mT @ v.double() @ B.double()
+    got = ops.two_sided_product(A.cuda(), v.cuda(), B.cuda(), transpose_a=True)
+    worst = lambda x: ((x.double().cpu() - want) / want).abs().max().item()
+    plain = _chain(_chain(A.mT, v.mT), B.mT)
+    assert worst(got) <= max(worst(plain), 16 * 2.0 ** -24)
+
+
+def test_two_sided_split_preconditions_with_its_own_factors():
+    # Shampoo: L^(-1/4)·G·R^(-1/4) of G's own factors, units that hardly fire among them
+    m, n = 1830, 1900
+    G = _randn(11, m, n)
+    for i, s in {3: 1e-4, 64: 1e-5, 700: 1e-6}.items():
+        G[i] *= s
+
+    def root(F):
+        lam, V = torch.linalg.eigh(F)
+        return ((V * lam.clamp_min(1e-14 * lam[-1]).pow(-0.25)) @ V.mT).float()
+
+    Gd = G.double()
+    A, B = root(Gd @ Gd.mT), root(Gd.mT @ Gd)
+    want = A.double() @ G.double() @ B.double()
+    got = ops.precond_apply_two_sided(A.cuda(), G.cuda(), B.cuda())
+    _rows_no_worse(got, want, _chain(_chain(A, G.mT), B.mT))
+
+
+def test_two_sided_split_non_finite_lands_where_fp32_puts_it():
+    A, X, B = (t[0] for t in _sides(1, 1830, 1840))
+    A, B = torch.eye(1830) * 2, torch.eye(1840) * 3
+    X[4, 6], X[9, 6], X[11] = math.inf, -math.inf, 0.0
+    A[5, 11] = math.inf  # against an empty row of X
+    plain = _chain(_chain(A, X.mT), B.mT)
+    got = ops.precond_apply_two_sided(A.cuda(), X.cuda(), B.cuda())
+    assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), plain.nan_to_num(7.0, 8.0, 9.0))
