@@ -193,6 +193,49 @@ struct NsExp {
 };
 constexpr int kNsSplitSteps = 32;  // per matrix: exponents of this many steps
 
+// x_{t+1}: max |p| over [0, x], with 1% for the products' rounding. |p| is largest
+// at the end of the interval or where p' = a + 3b·s² + 5c·s⁴ = 0.
+__host__ __device__ inline double ns_next_bound(double a, double b, double c, double x) {
+  const double u = x * x;
+  auto p = [&](double q) { return fabs(a + q * (b + q * c)) * sqrt(q); };  // q = s²
+  double top = p(u);
+  const double disc = 9.0 * b * b - 20.0 * a * c;
+  if (c != 0.0 && disc >= 0.0) {
+    for (int sg = -1; sg <= 1; sg += 2) {
+      const double q = (-3.0 * b + sg * sqrt(disc)) / (10.0 * c);
+      if (q > 0.0 && q < u) top = fmax(top, p(q));
+    }
+  } else if (c == 0.0 && b != 0.0) {
+    const double q = -a / (3.0 * b);
+    if (q > 0.0 && q < u) top = fmax(top, p(q));
+  }
+  return 1.01 * top;
+}
+
+// Coefficients that those bounds fit: they follow the largest singular value
+// that could be there, and the planes hold what is down to 2^-39 of it, so the
+// bound may not run away from the values that are. It stays at most 1.5 from
+// x_0 = 1, small singular values do not shrink (a >= 1) and none shrinks below
+// half in a step (q(s²) = p(s)/s >= 1/2 on [0, x_t]). The usual triple stays at
+// 1.22 with q >= 0.64. With (4.1, -2.9, 0.55) the bound goes 2.0, 2.7, 30, 1e7, ...
+// and five steps lost every bit of the result; such calls keep the fp32 chain.
+inline bool ns_split_coeffs(int64_t steps, double a, double b, double c, double eps) {
+  if (!(a >= 1.0) || !(eps >= 0.0) || steps < 1 || steps > kNsSplitSteps) return false;
+  double x = 1.0;
+  for (int64_t t = 0; t < steps; ++t) {
+    const double u = x * x;
+    auto q = [&](double v) { return a + v * (b + v * c); };
+    double least = std::min(a, q(u));
+    if (c != 0.0) {
+      const double v = -b / (2.0 * c);
+      if (v > 0.0 && v < u) least = std::min(least, q(v));
+    }
+    x = ns_next_bound(a, b, c, x);
+    if (!(least >= 0.5) || !(x <= 1.5)) return false;
+  }
+  return true;
+}
+
 // Clamped to exponents that fp32 values (and so their bounds) have.
 __device__ __forceinline__ int ns_exp(double bound) {
   int k = 0;
@@ -215,20 +258,7 @@ __global__ void __launch_bounds__(256) ns_split_scale_kernel(const double* __res
   int ex_t = ns_exp(x);
   for (int t = 0; t < steps; ++t) {
     const double u = x * x;
-    // |p| is largest at the end of [0, x] or where p' = a + 3b·s² + 5c·s⁴ = 0
-    auto p = [&](double q) { return fabs(a + q * (b + q * c)) * sqrt(q); };  // q = s²
-    double top = p(u);
-    const double disc = 9.0 * b * b - 20.0 * a * c;
-    if (c != 0.0 && disc >= 0.0) {
-      for (int sg = -1; sg <= 1; sg += 2) {
-        const double q = (-3.0 * b + sg * sqrt(disc)) / (10.0 * c);
-        if (q > 0.0 && q < u) top = fmax(top, p(q));
-      }
-    } else if (c == 0.0 && b != 0.0) {
-      const double q = -a / (3.0 * b);
-      if (q > 0.0 && q < u) top = fmax(top, p(q));
-    }
-    x = 1.01 * top;  // the products' rounding
+    x = ns_next_bound(a, b, c, x);
     const int nxt = ns_exp(x);
     e[t] = NsExp{ex_t, ns_exp(u), ns_exp(fabs(a) + fabs(b) * u + fabs(c) * u * u), nxt};
     ex_t = nxt;
@@ -382,8 +412,8 @@ size_t ns5_split_ws_bytes(int64_t batch, int64_t m, int64_t n) {
 // against 11.3). Sides just above a multiple of 128, whose planes would not
 // fit the workspace of the fp32 chain, keep that chain.
 constexpr int64_t kNsSplitMinSide = 128, kNsSplitMinWork = 512 * 512;
-inline bool ns5_split(int64_t batch, int64_t m, int64_t n, int64_t steps) {
-  return m >= kNsSplitMinSide && batch * m * m >= kNsSplitMinWork && steps >= 1 && steps <= kNsSplitSteps &&
+inline bool ns5_split(int64_t batch, int64_t m, int64_t n, int64_t steps, double a, double b, double c, double eps) {
+  return m >= kNsSplitMinSide && batch * m * m >= kNsSplitMinWork && ns_split_coeffs(steps, a, b, c, eps) &&
          ns5_split_ws_bytes(batch, m, n) <= ns5_ws_bytes_t<float>(batch, m, n);
 }
 
@@ -478,7 +508,7 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
   PTO_REQUIRE(!aliased || g0 == o0, "newton_schulz_orthogonalize: out partially overlaps G");
 
   if constexpr (std::is_same<T, float>::value) {
-    if (ns5_split(batch, m, n, steps))
+    if (ns5_split(batch, m, n, steps, a, b, c, eps))
       return ns5_split_run(G, out, batch, rows, cols, steps, a, b, c, eps, ws, ws_bytes, stream);
   }
 

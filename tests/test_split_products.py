@@ -101,6 +101,16 @@ def test_ns5_split_non_finite_matrix_only(bad):
     assert torch.equal(ops.newton_schulz_orthogonalize(Z), Z)
 
 
+@pytest.mark.parametrize("steps,coeffs", [
+    (5, (4.1, -2.9, 0.55)), (4, (4.1, -2.9, 0.55)), (3, (8.2872, -23.5959, 17.3004)), (5, (2.0, 0.5, 0.5)),
+    (4, (2.0, 1.0, 1.0)), (3, (9.0, 3.0, 1.0)), (32, (0.6, 0.4, 0.0)), (12, (0.3, 0.0, 0.0)), (5, (0.01, 0.5, 0.0)),
+    (32, (1.5, -0.5, 0.0)), (33, (1.5, -0.5, 0.0))])
+def test_ns5_coefficients_off_the_usual(steps, coeffs):
+    G = torch.randn(640, 576, generator=torch.Generator().manual_seed(9))
+    got = ops.newton_schulz_orthogonalize(G.cuda(), steps=steps, coeffs=coeffs)
+    _no_worse(got, _ns64(G, steps, coeffs), _ns_chain(G, steps, coeffs), roundings=2 * steps)
+
+
 # ---------------------------------------------------------------- factor updates
 
 KRON = [(1025, 3500), (2049, 2050), (3001, 1030)]
