@@ -61,7 +61,7 @@ struct ApplySplitWs {
     const int64_t pa = mw * std::max(std::max(absmax_row_parts(m), absmax_col_parts(m)), absmax_row_parts(n));
     const int64_t pb = nw * std::max(std::max(absmax_row_parts(n), absmax_col_parts(n)), absmax_col_parts(m));
     take(part, nb * std::max(pa, pb));
-    take(bad, 1);
+    take(bad, nb);
     for (int** e : {&rx, &ea, &eax}) take(*e, nb * mw);
     for (int** e : {&ex, &eb}) take(*e, nb * nw);
   }
@@ -93,7 +93,6 @@ int two_sided_split(const float* Am, const float* X, const float* Bm, float* out
     p.s_pre = s_pre;
     p.pre_mul = mul;
     p.pre_off = off;
-    p.one_flag = 1;
     return p;
   };
   auto pack = [&](const SplitPack& p) { return launch_split_pack_max(p, nb, stream, false); };
@@ -102,9 +101,11 @@ int two_sided_split(const float* Am, const float* X, const float* Bm, float* out
   if (pack(planes(Am, m, m, m, sA, trans_a, w.A, ldm, w.ea, w.mw, w.rx, w.mw, -1, kSplitTop))) return -1;
   if (pack(planes(Bm, n, n, n, sB, !trans_b, w.B, ldn, w.eb, w.nw, w.ex, w.nw, -1, 0))) return -1;
   {
-    GemmArgs g{w.A, ldm, 2 * m * ldm, w.XA, ldm, 2 * n * ldm, (int)m, (int)n, (int)ldm, 0, 0, w.bad, 0, 0, m * ldm,
-               n * ldm};
-    const EpiStore<float, float> e{w.AX, ldn, m * ldn};
+    SplitArgs g{{w.A, ldm, 2 * m * ldm, w.XA, ldm, 2 * n * ldm, (int)m, (int)n, (int)ldm}, m * ldm, n * ldm, w.bad, 1};
+    g.fP = PlainOperand{Am, trans_a ? 1 : m, trans_a ? m : 1, sA, -1};
+    g.fQ = PlainOperand{X, 1, n, sX, -1};
+    g.fK = (int)m;
+    const EpiRaw e{{w.AX, ldn, m * ldn}};
     if (launch_gemm<sp16, false>(g, e, nb, stream, name_left)) return -1;
   }
   {
@@ -113,22 +114,13 @@ int two_sided_split(const float* Am, const float* X, const float* Bm, float* out
     p.bad = nullptr;
     if (pack(p)) return -1;
   }
-  {
-    GemmArgs g{w.XA, ldn, 2 * m * ldn, w.B, ldn, 2 * n * ldn, (int)m, (int)n, (int)ldn, 0, 0, w.bad, 0, 0, m * ldn,
-               n * ldn};
-    EpiDescale<EpiStore<float, float>> e{{out, n, m * n}, w.eax, w.eb, w.mw, w.nw};
-    e.off = -kSplitTop;
-    if (launch_gemm<sp16, false>(g, e, nb, stream, name_right)) return -1;
-  }
-  // a flagged value anywhere: both products in plain fp32
-  float* AX = w.AX;
-  typedef EpiStore<float, float> Store;
-  const PlainOperand a{Am, trans_a ? 1 : m, trans_a ? m : 1, sA, -1}, x{X, 1, n, sX, -1};
-  const PlainOperand ax{AX, ldn, 1, m * ldn, -1}, b{Bm, trans_b ? n : 1, trans_b ? 1 : n, sB, -1};
-  const PlainProduct<Store> left{a, x, m, n, m, Store{AX, ldn, m * ldn}};
-  const PlainProduct<Store> right{ax, b, m, n, n, Store{out, n, m * n}};
-  if (launch_plain_product(w.bad, nb, left, (const PlainProduct<Store>*)nullptr, stream, true)) return -1;
-  return launch_plain_product(w.bad, nb, right, (const PlainProduct<Store>*)nullptr, stream, true);
+  SplitArgs g{{w.XA, ldn, 2 * m * ldn, w.B, ldn, 2 * n * ldn, (int)m, (int)n, (int)ldn}, m * ldn, n * ldn, w.bad, 1};
+  g.fP = PlainOperand{w.AX, ldn, 1, m * ldn, -1};
+  g.fQ = PlainOperand{Bm, trans_b ? n : 1, trans_b ? 1 : n, sB, -1};
+  g.fK = (int)n;
+  EpiDescale<EpiStore<float, float>> e{{out, n, m * n}, w.eax, w.eb, w.mw, w.nw};
+  e.off = -kSplitTop;
+  return launch_gemm<sp16, false>(g, e, nb, stream, name_right);
 }
 
 template <typename T>

@@ -40,7 +40,7 @@ typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 // fp32 operands as pairs of fp16 ("split"): x·2^-e = h + l with h = fp16(x·2^-e)
 // and l = fp16(x·2^-e - h), held as two planes of the same layout, l's at
-// GemmArgs::pP (pQ) elements from h's. e is an exponent per row of the
+// SplitArgs::pP (pQ) elements from h's. e is an exponent per row of the
 // operand (or one per matrix) that puts the row's largest value at 2^13..2^14,
 // so h + l keeps 22-24 bits of every value down to 2^-16 of that largest one
 // and 2^-39 of it below. A product is h·h + h·l + l·h in fp32 accumulators
@@ -153,8 +153,27 @@ struct GemmArgs {
   const int* guard;  // if non-null and guard[b * guard_stride] != 0, matrix b is skipped
   int guard_stride;  // ints between the guard words of consecutive matrices (0: one word)
   int cus;           // compute units of the device (set by the launcher)
-  int64_t pP = 0, pQ = 0;  // split operands: elements from the h plane to the l plane
 };
+
+// A fp32 operand as it lies in memory: element (r, kk) of matrix b at
+// p[b·batch + r·row + kk·k], row or k being 1; row `ones_at` is all ones (-1:
+// none).
+struct PlainOperand {
+  const float* p;
+  int64_t row, k, batch;
+  int64_t ones_at;
+};
+// Split operands: matrices whose planes do not serve (plain[b * plain_stride]
+// != 0, decided on the device) run on the fp32 MFMA from fP and fQ, K of fK.
+struct SplitArgs : GemmArgs {
+  int64_t pP, pQ;  // elements from the h plane to the l plane
+  const int* plain = nullptr;
+  int plain_stride = 0;
+  PlainOperand fP{}, fQ{};
+  int fK = 0;
+};
+template <typename T>
+using ArgsOf = std::conditional_t<std::is_same<T, sp16>::value, SplitArgs, GemmArgs>;
 
 // Workgroups are dispatched to the 8 XCDs round-robin by linear id, each
 // XCD has its own L2, and all XCDs share the memory-side Infinity Cache.
@@ -496,12 +515,118 @@ __device__ __forceinline__ void store_rows(const typename MF::cvec_t (&acc)[FM][
   }
 }
 
+// Epilogues of split operands have one more argument, whether the values come
+// from the fp32 MFMA and carry no scales.
+template <class Epi>
+struct SplitEpi {
+  typedef typename Epi::S S;
+  typedef typename Epi::Pre Pre;
+  typedef typename Epi::PreT PreT;
+  static constexpr bool kVoIsV = Epi::kVoIsV;
+  const Epi& e;
+  bool plain;
+  __device__ __forceinline__ bool has_t() const { return e.has_t(); }
+  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
+    e.load(b, i, j0, kbeg, n, p, plain);
+  }
+  __device__ __forceinline__ void load_t(int b, int j, int i0, int n, PreT& p) const { e.load_t(b, j, i0, n, p, plain); }
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& p, S* vo) const {
+    e.put(b, i, j0, v, kbeg, n, p, vo, plain);
+  }
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT& p) const {
+    e.put_t(b, j, i0, v, n, p, plain);
+  }
+};
+
+// The sums of a tile of a matrix whose planes do not serve: the fp32 MFMA over K
+// tiles of 16 from the fp32 operands as they lie, with the LDS rows (64 bytes, the
+// same swizzle), fragments and k order of the fp32 kernels, so the sums have
+// their bits. A K tile is loaded into registers while the one before it is
+// multiplied, and two stages let one barrier a tile do. Factor update of a 4096²
+// gradient with an infinity: 1.45 ms, against 1.12 on the fp32 kernels and 23.6
+// in scalar multiply-adds.
+template <class Cfg, int FM, int FN>
+__device__ __forceinline__ void plain_sums(const SplitArgs& g, int b, int row0, int col0, int wave, int lane, char* st0,
+                                           char* st1, Mfma<float>::cvec_t (&acc)[FM][FN]) {
+  typedef Mfma<float> MF;
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, WTM = 16 * FM, WTN = 16 * FN;
+  constexpr int CH = (BM + BN) * 4, PER = CH / Cfg::NT;
+  static_assert(Cfg::KG == 1 && CH % Cfg::NT == 0 && BM * 4 % 64 == 0, "whole chunks per thread, one operand per wave");
+  const int tid = wave * 64 + lane, wm = wave / Cfg::WN, wn = wave % Cfg::WN;
+  const int lr = lane & 15, ch = (lane >> 4) ^ swz(lr);
+  uint4 v[PER];
+  // chunk e of a K tile: k 4c .. 4c + 3 of row r of its operand (lanes along
+  // whichever index is contiguous)
+  auto place = [&](int e, int& r, int& c) {
+    const bool isp = e < BM * 4;
+    const int i = isp ? e : e - BM * 4, rows = isp ? BM : BN;
+    const bool along_k = (isp ? g.fP : g.fQ).k == 1;
+    r = along_k ? i >> 2 : i % rows;
+    c = along_k ? i & 3 : i / rows;
+  };
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int e = tid + q * Cfg::NT;
+      const bool isp = e < BM * 4;
+      const PlainOperand& o = isp ? g.fP : g.fQ;
+      int r, c;
+      place(e, r, c);
+      const int64_t row = (isp ? row0 : col0) + r;
+      const int kk = k0 + 4 * c, n = row < (isp ? g.M : g.N) ? min(4, g.fK - kk) : 0;
+      const float* p = o.p + (int64_t)b * o.batch + row * o.row + kk * o.k;
+      v[q] = make_uint4(0, 0, 0, 0);
+      if (row == o.ones_at) {
+        const unsigned one = __float_as_uint(1.f);
+        v[q] = make_uint4(n > 0 ? one : 0, n > 1 ? one : 0, n > 2 ? one : 0, n > 3 ? one : 0);
+      } else if (o.k == 1 && n == 4) {
+        __builtin_memcpy(&v[q], p, 16);
+      } else {
+        if (n > 0) v[q].x = __float_as_uint(p[0]);
+        if (n > 1) v[q].y = __float_as_uint(p[o.k]);
+        if (n > 2) v[q].z = __float_as_uint(p[2 * o.k]);
+        if (n > 3) v[q].w = __float_as_uint(p[3 * o.k]);
+      }
+    }
+  };
+  auto step = [&](int k0, char* st) {
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int e = tid + q * Cfg::NT;
+      int r, c;
+      place(e, r, c);
+      if (e >= BM * 4) r += BM;
+      *reinterpret_cast<uint4*>(st + r * kRowBytes + (c ^ swz(r)) * 16) = v[q];
+    }
+    stage_barrier();
+    if (k0 + 16 < g.fK) fetch(k0 + 16);
+    uint4 bf[FN];
+#pragma unroll
+    for (int fn = 0; fn < FN; ++fn)
+      bf[fn] = *reinterpret_cast<const uint4*>(st + (BM + wn * WTN + fn * 16 + lr) * kRowBytes + ch * 16);
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) {
+      const uint4 af = *reinterpret_cast<const uint4*>(st + (wm * WTM + fm * 16 + lr) * kRowBytes + ch * 16);
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = MF::mma(af, bf[fn], ii, acc[fm][fn]);
+    }
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < g.fK; k0 += 32) {
+    step(k0, st0);
+    if (k0 + 16 < g.fK) step(k0 + 16, st1);
+  }
+  stage_barrier();  // the arrays host the epilogue staging next
+}
+
 // PT: P is stored [K][M] (M contiguous) and read like a QN operand. For a
 // symmetric P (B' in X' = B'·X, A in A·A) that is P itself: its rows are
 // its columns, so the product reads it with conflict-free transposing LDS
 // reads and 512-byte DMA rows instead of 16-byte row chunks.
-template <typename T, class Cfg, bool UPPER, class Epi, bool QN = false, bool PT = false, bool COMP = false>
-__global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
+template <typename T, class Cfg, bool UPPER, class Epi, bool QN, bool PT, bool COMP, class Args>
+__global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(Args g, Epi epi) {
   typedef Mfma<T> MF;
   typedef typename MF::cvec_t cvec_t;
   typedef typename Epi::S S;
@@ -642,6 +767,24 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
     for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
       for (int r = 0; r < MF::NACC; ++r) acc[fm][fn][r] = 0;
+  bool plain = false;
+  if constexpr (kSplit) {
+    plain = g.plain != nullptr && g.plain[(int64_t)b * g.plain_stride] != 0;
+    if (plain) {
+      plain_sums<Cfg>(g, b, row0, col0, wave, lane, st0, st1, acc);
+      if constexpr (COMP) {
+        // an epilogue of its own: joining the block sums' one cost the 64² tile
+        // 8% of every call (the kernels without them are 0.7% faster joined)
+        const int wa = wave / Plan::WPA;
+        char* arr = wa == 0 ? st0 : wa == 1 ? st1 : wa == 2 ? st2 : wa == 3 ? st3 : wa == 4 ? st4 : wa == 5 ? st5 : wa == 6 ? st6 : st7;
+        S* stg = reinterpret_cast<S*>(arr) + (wave % Plan::WPA) * Plan::RPP * Plan::SP;
+        SplitEpi<Epi> se{epi, true};
+        store_rows<MF, Plan, UPPER, 0>(acc, stg, se, g, b, row0 + wm * WTM, col0 + wn * WTN, UPPER && ti == tj, lane);
+        epi.finish(b);
+        return;
+      }
+    }
+  }
 
   const int lr = lane % MF::MN, lg = lane / MF::MN;
   const int sw = swz(lr);  // rows of every fragment are lr mod 16
@@ -813,7 +956,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
   // outstanding). The launchers require K to be a multiple of NS tiles, so
   // every step of the unrolled group is a real one and the MFMAs need no
   // branch.
-  const int KT = (kSplit ? 2 : 1) * (g.K / BK);
+  const int KT = kSplit ? (plain && !COMP ? 0 : 2 * (g.K / BK)) : g.K / BK;
   if constexpr (KG == 2) {
     // K groups: waves 0..NWG-1 (group 0) take the even K tiles, the others
     // the odd ones, each group accumulating the whole tile in its own
@@ -1200,7 +1343,10 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(GemmArgs g, Epi epi) {
 #undef PTO_EXCHANGE
 #undef PTO_SLOT
   }
-  if constexpr (KG == 1) {
+  if constexpr (kSplit) {
+    SplitEpi<Epi> se{epi, plain && !COMP};
+    store_rows<MF, Plan, UPPER, 0>(acc, stg, se, g, b, wr0, wc0, diag, lane);
+  } else if constexpr (KG == 1) {
     store_rows<MF, Plan, UPPER, 0>(acc, stg, epi, g, b, wr0, wc0, diag, lane);
   } else {
     if (kg == 0)
@@ -1330,7 +1476,7 @@ inline int device_cus() {
 }
 
 template <typename T, class Cfg, bool UPPER, class Epi, bool QN = false, bool PT = false, bool COMP = false>
-int launch_gemm_cfg(GemmArgs g, const Epi& epi, int batch, hipStream_t stream, const char* name) {
+int launch_gemm_cfg(ArgsOf<T> g, const Epi& epi, int batch, hipStream_t stream, const char* name) {
   g.tiles_m = (g.M + Cfg::BM - 1) / Cfg::BM;
   g.tiles_n = (g.N + Cfg::BN - 1) / Cfg::BN;
   g.cus = device_cus();
@@ -1339,8 +1485,8 @@ int launch_gemm_cfg(GemmArgs g, const Epi& epi, int batch, hipStream_t stream, c
   // the kernel numbers workgroups across the batch in 32-bit arithmetic
   PTO_REQUIRE(batch < 65536 && tiles * batch < (1ll << 31), std::string(name) + ": grid too large");
   ProfScope ps(name, stream);
-  hipLaunchKernelGGL((gemm_nt_kernel<T, Cfg, UPPER, Epi, QN, PT, COMP>), dim3((unsigned)tiles, (unsigned)batch),
-                     dim3(Cfg::NT), 0, stream, g, epi);
+  hipLaunchKernelGGL((gemm_nt_kernel<T, Cfg, UPPER, Epi, QN, PT, COMP, ArgsOf<T>>),
+                     dim3((unsigned)tiles, (unsigned)batch), dim3(Cfg::NT), 0, stream, g, epi);
   PTO_LAUNCHED(name);
   return 0;
 }
@@ -1402,7 +1548,7 @@ int pick_tile(int64_t M, int64_t N, int64_t batch) {
 // Validate the operand contract and pick a tile size. COMP: blocked fp32
 // accumulation (see the main loop).
 template <typename T, bool UPPER, class Epi, bool COMP = false>
-int launch_gemm(const GemmArgs& g, const Epi& epi, int batch, hipStream_t stream, const char* name) {
+int launch_gemm(const ArgsOf<T>& g, const Epi& epi, int batch, hipStream_t stream, const char* name) {
   typedef typename PickTiles<T, UPPER>::Big Big;
   typedef typename PickTiles<T, UPPER>::Small Small;
   static_assert(!UPPER || (Big::BM == Big::BN && Small::BM == Small::BN), "symmetric products need square tiles");
@@ -1437,7 +1583,7 @@ int launch_gemm(const GemmArgs& g, const Epi& epi, int batch, hipStream_t stream
 // mirrored, as in launch_gemm.
 // pick: the tile (pick_tile's codes), or -1 to let pick_tile choose.
 template <class Epi, bool PT = false, bool UPPER = false, typename T = bf16>
-int launch_gemm_qn(const GemmArgs& g, const Epi& epi, int batch, hipStream_t stream, const char* name,
+int launch_gemm_qn(const ArgsOf<T>& g, const Epi& epi, int batch, hipStream_t stream, const char* name,
                    int pick = -1) {
   static_assert(PT || !UPPER, "symmetric QN products need PT");
   typedef typename PickTiles<T, UPPER>::Big Big;

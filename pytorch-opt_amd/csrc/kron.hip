@@ -75,20 +75,17 @@ int kron_split_run(const EpiL& el, const EpiL& er, const float* G, int64_t batch
                     w.Gp, m * ldn, ldn, 2 * m * ldn, w.GT,  n * ldm, ldm,     2 * n * ldm, 0};
   if (launch_split_pack_max(p, nb, stream)) return -1;
   {
-    GemmArgs g{w.Gp, ldn, 2 * m * ldn, w.Gp, ldn, 2 * m * ldn, (int)m, (int)m, (int)ldn, 0, 0, w.bad, 1, 0, m * ldn,
-               m * ldn};
+    SplitArgs g{{w.Gp, ldn, 2 * m * ldn, w.Gp, ldn, 2 * m * ldn, (int)m, (int)m, (int)ldn}, m * ldn, m * ldn, w.bad, 1};
+    g.fP = g.fQ = PlainOperand{G, n, 1, m * n, -1};
+    g.fK = (int)n;
     const EpiDescale<EpiL> e{el, w.er, w.er, w.mw, w.mw};
     if (launch_gemm<sp16, true, EpiDescale<EpiL>, true>(g, e, nb, stream, "kron_left")) return -1;
   }
-  {
-    GemmArgs g{w.GT, ldm, 2 * n * ldm, w.GT, ldm, 2 * n * ldm, (int)n, (int)n, (int)ldm, 0, 0, w.bad, 1, 0, n * ldm,
-               n * ldm};
-    const EpiDescale<EpiL> e{er, w.ec, w.ec, w.nw, w.nw};
-    if (launch_gemm<sp16, true, EpiDescale<EpiL>, true>(g, e, nb, stream, "kron_right")) return -1;
-  }
-  const PlainOperand gl{G, n, 1, m * n, -1}, gr{G, 1, n, m * n, -1};
-  const PlainProduct<EpiL> left{gl, gl, m, m, n, el}, right{gr, gr, n, n, m, er};
-  return launch_plain_product(w.bad, nb, left, &right, stream);
+  SplitArgs g{{w.GT, ldm, 2 * n * ldm, w.GT, ldm, 2 * n * ldm, (int)n, (int)n, (int)ldm}, n * ldm, n * ldm, w.bad, 1};
+  g.fP = g.fQ = PlainOperand{G, 1, n, m * n, -1};
+  g.fK = (int)m;
+  const EpiDescale<EpiL> e{er, w.ec, w.ec, w.nw, w.nw};
+  return launch_gemm<sp16, true, EpiDescale<EpiL>, true>(g, e, nb, stream, "kron_right");
 }
 
 template <typename T>
@@ -234,12 +231,11 @@ int gram_split_run(const Epi& epi, const float* X, int64_t rows, int64_t d, int 
   const SplitPack p{X, rows, d, d, 0, nullptr, cpart, 0, dw, nullptr, ec, bad, nullptr, 0, 0, 0, XT, dd * ldr, ldr,
                     0, ones};
   if (launch_split_pack_max(p, 1, stream)) return -1;
-  GemmArgs g{XT, ldr, 0, XT, ldr, 0, (int)dd, (int)dd, (int)ldr, 0, 0, bad, 0, 0, dd * ldr, dd * ldr};
+  SplitArgs g{{XT, ldr, 0, XT, ldr, 0, (int)dd, (int)dd, (int)ldr}, dd * ldr, dd * ldr, bad, 0};
+  g.fP = g.fQ = PlainOperand{X, 1, d, 0, ones ? d : -1};
+  g.fK = (int)rows;
   const EpiDescale<Epi> e{epi, ec, ec, 0, 0};
-  if (launch_gemm<sp16, true, EpiDescale<Epi>, true>(g, e, 1, stream, "gram_update")) return -1;
-  const PlainOperand x{X, 1, d, 0, ones ? d : -1};
-  return launch_plain_product(bad, 1, PlainProduct<Epi>{x, x, dd, dd, rows, epi}, (const PlainProduct<Epi>*)nullptr,
-                              stream);
+  return launch_gemm<sp16, true, EpiDescale<Epi>, true>(g, e, 1, stream, "gram_update");
 }
 
 // bf16 X without the ones column is already the [K][M] operand of the

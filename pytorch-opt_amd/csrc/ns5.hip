@@ -275,8 +275,8 @@ struct EpiNsGramSplit {
   typedef NoPre PreT;
   static constexpr bool kVoIsV = true;
   __device__ __forceinline__ bool has_t() const { return false; }
-  __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
-  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
+  __device__ __forceinline__ void load(int, int, int, int, int, Pre&, bool) const {}
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&, bool) const {}
   __device__ __forceinline__ void store(int b, int64_t o, const S* v, int kbeg, int n) const {
     const NsExp e = ex[(int64_t)b * kNsSplitSteps];
     S w[8];
@@ -284,12 +284,12 @@ struct EpiNsGramSplit {
     for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], e.a - 2 * e.x);
     st8_split(dst + (int64_t)b * sd + o, pl, w, kbeg, n);
   }
-  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo, bool) const {
     store(b, (int64_t)i * ld + j0, v, kbeg, n);
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = v[k];
   }
-  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool) const {
     store(b, (int64_t)j * ld + i0, v, 0, n);
   }
   __device__ __forceinline__ void finish(int) const {}
@@ -309,16 +309,16 @@ struct EpiNsSqSplit {
   typedef NoPre PreT;
   static constexpr bool kVoIsV = false;  // the mirror stores B', not the raw product
   __device__ __forceinline__ bool has_t() const { return false; }
-  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
+  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p, bool) const {
     if (full_run(kbeg, n)) {
       const sp16* q = Asrc + (int64_t)b * sd + (int64_t)i * ld + j0;
       p.h = ld16(q);
       p.l = ld16(q + pl);
     }
   }
-  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&, bool) const {}
   __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre,
-                                      S* vo) const {
+                                      S* vo, bool) const {
     const NsExp e = ex[(int64_t)b * kNsSplitSteps];
     const int64_t o = (int64_t)b * sd + (int64_t)i * ld + j0;
     S a[8];
@@ -339,7 +339,7 @@ struct EpiNsSqSplit {
     }
     st8_split(dst + o, pl, w, kbeg, n);
   }
-  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool) const {
     const NsExp e = ex[(int64_t)b * kNsSplitSteps];
     S w[8];
 #pragma unroll
@@ -363,9 +363,9 @@ struct EpiNsUpdateSplit {
   typedef NoPre PreT;
   static constexpr bool kVoIsV = true;
   __device__ __forceinline__ bool has_t() const { return dstT != nullptr; }
-  __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
-  __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
-  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo) const {
+  __device__ __forceinline__ void load(int, int, int, int, int, Pre&, bool) const {}
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&, bool) const {}
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo, bool) const {
     const NsExp e = ex[(int64_t)b * kNsSplitSteps];
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = v[k];
@@ -380,7 +380,7 @@ struct EpiNsUpdateSplit {
       st8<float, S>(dst + (int64_t)b * s_o + (int64_t)i * ld_o + j0, w, kbeg, n);
     }
   }
-  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&) const {
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool) const {
     const NsExp e = ex[(int64_t)b * kNsSplitSteps];
     S w[8];
 #pragma unroll
@@ -460,12 +460,12 @@ int ns5_split_run(const float* G, float* out, int64_t batch, int64_t rows, int64
     const bool last = t == steps - 1;
     const sp16* Xc = X[t & 1];
     {
-      GemmArgs g{Xc, ldn, sX, Xc, ldn, sX, (int)m, (int)m, (int)ldn, 0, 0, nullptr, 0, 0, plX, plX};
+      SplitArgs g{{Xc, ldn, sX, Xc, ldn, sX, (int)m, (int)m, (int)ldn}, plX, plX};
       EpiNsGramSplit e{Ab, plA, ldm, sA, ex + t};
       if (launch_gemm<sp16, true>(g, e, nb, stream, "ns5_gram")) return -1;
     }
     {
-      GemmArgs g{Ab, ldm, sA, Ab, ldm, sA, (int)m, (int)m, (int)ldm, 0, 0, nullptr, 0, 0, plA, plA};
+      SplitArgs g{{Ab, ldm, sA, Ab, ldm, sA, (int)m, (int)m, (int)ldm}, plA, plA};
       EpiNsSqSplit e{Ab, Bb, plA, ldm, sA, (float)a, (float)b, (float)c, ex + t};
       // A's rows are its columns: read K-contiguous by the 256² and 192² tiles
       // (12 x 2048²: 310 us against 325 with transposing reads), transposing
@@ -478,7 +478,7 @@ int ns5_split_run(const float* G, float* out, int64_t batch, int64_t rows, int64
       }
     }
     {
-      GemmArgs g{Bb, ldm, sA, Xc, ldn, sX, (int)m, (int)n, (int)ldm, 0, 0, nullptr, 0, 0, plA, plX};
+      SplitArgs g{{Bb, ldm, sA, Xc, ldn, sX, (int)m, (int)n, (int)ldm}, plA, plX};
       EpiNsUpdateSplit e{last ? nullptr : X[(t & 1) ^ 1], plX, ldn, sX, last && !transposed ? out : nullptr,
                          last && transposed ? out : nullptr, cols, sG, ex + t};
       if (launch_gemm_qn<EpiNsUpdateSplit, true, false, sp16>(g, e, nb, stream, "ns5_update")) return -1;

@@ -162,7 +162,6 @@ struct SplitPack {
   int64_t s_pre = 0;
   int pre_mul = 0, pre_off = 0;
   const int* er_add = nullptr;  // stride mw
-  int one_flag = 0;  // bad is one word for the whole batch, cleared by the caller
   __device__ __forceinline__ int pre(const int* p, int b, int64_t at, int64_t n) const {
     return p && at < n ? pre_off + pre_mul * p[(int64_t)b * s_pre + at] : 0;
   }
@@ -290,7 +289,7 @@ inline int64_t absmax_col_parts(int64_t rows) { return (rows + absmax_rows(rows)
   }
   __syncthreads();
   auto check = [&](unsigned u) {
-    if (a.bad && (u >= kInfBits || ((a.pre_r || a.pre_c) && u != 0 && u < kTinyBits))) a.bad[a.one_flag ? 0 : b] = 1;
+    if (a.bad && (u >= kInfBits || ((a.pre_r || a.pre_c) && u != 0 && u < kTinyBits))) a.bad[b] = 1;
   };
   if (ty == 0 && a.out_s) {
     const unsigned u = max(mx[0][tx], mx[1][tx]);
@@ -342,13 +341,13 @@ inline int launch_split_pack_max(const SplitPack& a, int batch, hipStream_t stre
 
 // Split exponents of the rows of a fp32 matrix: e[b·ew + r]. A wave takes a row,
 // 16 bytes per lane and four runs in flight. Bound by memory: 4 bytes per
-// element. Also clears bad[0].
+// element. Also clears bad[b].
 [[maybe_unused]] static __global__ void __launch_bounds__(256) row_exp_kernel(const float* __restrict__ in, int64_t rows,
                                                                               int64_t cols, int64_t ld, int64_t s_in,
                                                                               int* __restrict__ e, int64_t ew,
                                                                               int* __restrict__ bad) {
   const int b = blockIdx.y, lane = threadIdx.x & 63;
-  if (blockIdx.x == 0 && b == 0 && threadIdx.x == 0) bad[0] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) bad[b] = 0;
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= rows) return;
   const float* row = in + (int64_t)b * s_in + r * ld;
@@ -387,99 +386,52 @@ struct EpiDescale {
   typedef typename In::PreT PreT;
   static constexpr bool kVoIsV = true;  // the transposed pass takes the raw value and scales it itself
   __device__ __forceinline__ bool has_t() const { return false; }
-  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p) const {
+  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p, bool) const {
     in.load(b, i, j0, kbeg, n, p);
   }
-  __device__ __forceinline__ void load_t(int b, int j, int i0, int n, PreT& p) const { in.load_t(b, j, i0, n, p); }
-  __device__ __forceinline__ void scaled(int b, int i, int j0, const S* v, int n, S* w) const {
+  __device__ __forceinline__ void load_t(int b, int j, int i0, int n, PreT& p, bool) const {
+    in.load_t(b, j, i0, n, p);
+  }
+  __device__ __forceinline__ void scaled(int b, int i, int j0, const S* v, int n, S* w, bool plain) const {
     const int ei = er[(int64_t)b * s_r + i];
     const int* ej = ec + (int64_t)b * s_c + j0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) w[k] = k < n ? ldexpf(v[k], off - ei - ej[k]) : 0.f;
+    for (int k = 0; k < 8; ++k) w[k] = k < n ? (plain ? v[k] : ldexpf(v[k], off - ei - ej[k])) : 0.f;
   }
-  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre,
-                                      S* vo) const {
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre, S* vo,
+                                      bool plain) const {
     S w[8], drop[8];
-    scaled(b, i, j0, v, n, w);
+    scaled(b, i, j0, v, n, w, plain);
     in.put(b, i, j0, w, kbeg, n, pre, drop);
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = v[k];
   }
   // symmetric products only (er == ec)
-  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT& pre) const {
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT& pre, bool plain) const {
     S w[8];
-    scaled(b, j, i0, v, n, w);
+    scaled(b, j, i0, v, n, w, plain);
     in.put_t(b, j, i0, w, n, pre);
   }
   __device__ __forceinline__ void finish(int) const {}
 };
 
-// The products of matrices with a non-finite value (bad[b] != 0), which the
-// split products skip: plain fp32 multiply-adds in k order, so that infinities
-// and NaN land where fp32 arithmetic puts them. C(i, j) = sum_k P(i, k)·Q(j, k)
-// with element strides for rows and k; row `ones_at` of an operand is all ones
-// (-1: none). One launch whatever the batch; with nothing flagged its blocks
-// leave after one read each (3 us).
-struct PlainOperand {
-  const float* p;
-  int64_t row, k, batch;
-  int64_t ones_at;
-  __device__ __forceinline__ float at(int b, int64_t r, int64_t kk) const {
-    return r == ones_at ? 1.f : p[(int64_t)b * batch + r * row + kk * k];
+// Epilogue that stores the products of split operands in fp32 with their scales in.
+struct EpiRaw {
+  typedef float S;
+  EpiStore<float, float> in;
+  typedef NoPre Pre;
+  typedef NoPre PreT;
+  static constexpr bool kVoIsV = true;
+  __device__ __forceinline__ bool has_t() const { return false; }
+  __device__ __forceinline__ void load(int, int, int, int, int, Pre&, bool) const {}
+  __device__ __forceinline__ void load_t(int, int, int, int, PreT&, bool) const {}
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& p, S* vo,
+                                      bool) const {
+    in.put(b, i, j0, v, kbeg, n, p, vo);
   }
+  __device__ __forceinline__ void put_t(int, int, int, const S*, int, const PreT&, bool) const {}
+  __device__ __forceinline__ void finish(int) const {}
 };
-template <class Epi>
-struct PlainProduct {
-  PlainOperand P, Q;
-  int64_t M, N, K;
-  Epi epi;
-};
-template <class Epi>
-__global__ void __launch_bounds__(128) plain_product_kernel(const int* __restrict__ bad, int bad_stride, int nb,
-                                                            PlainProduct<Epi> one, PlainProduct<Epi> two) {
-  __shared__ float ps[32][33], qs[32][33];
-  PlainProduct<Epi>& a = blockIdx.y ? two : one;
-  const int64_t tn = (a.N + 31) / 32, tiles = (a.M + 31) / 32 * tn;
-  const int r = threadIdx.x / 4, c = threadIdx.x % 4 * 8;
-  for (int b = 0; b < nb; ++b) {
-    if (bad[b * bad_stride] == 0) continue;
-    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-      const int64_t i0 = t / tn * 32, j0 = t % tn * 32;
-      float v[8] = {0, 0, 0, 0, 0, 0, 0, 0}, vo[8];
-      for (int64_t k0 = 0; k0 < a.K; k0 += 32) {
-        for (int e = threadIdx.x; e < 1024; e += 128) {
-          const int64_t rr = e / 32, kk = k0 + e % 32;
-          ps[rr][e % 32] = i0 + rr < a.M && kk < a.K ? a.P.at(b, i0 + rr, kk) : 0.f;
-          qs[rr][e % 32] = j0 + rr < a.N && kk < a.K ? a.Q.at(b, j0 + rr, kk) : 0.f;
-        }
-        __syncthreads();
-        const int kn = (int)min((int64_t)32, a.K - k0);
-        for (int kk = 0; kk < kn; ++kk)
-#pragma unroll
-          for (int x = 0; x < 8; ++x) v[x] = fmaf(ps[r][kk], qs[c + x][kk], v[x]);
-        __syncthreads();
-      }
-      const int n = (int)min((int64_t)8, a.N - j0 - c);
-      if (i0 + r < a.M && n > 0) {
-        typename Epi::Pre pre;
-        a.epi.load(b, (int)(i0 + r), (int)(j0 + c), 0, n, pre);
-        a.epi.put(b, (int)(i0 + r), (int)(j0 + c), v, 0, n, pre, vo);
-      }
-    }
-  }
-}
-// One product, or two of the same kind (two != nullptr).
-template <class Epi>
-int launch_plain_product(const int* bad, int nb, const PlainProduct<Epi>& one, const PlainProduct<Epi>* two,
-                         hipStream_t stream, bool one_flag = false) {
-  auto tiles = [](const PlainProduct<Epi>& a) { return ((a.M + 31) / 32) * ((a.N + 31) / 32); };
-  const int64_t t = std::max(tiles(one), two ? tiles(*two) : 0);
-  const unsigned gx = (unsigned)std::min<int64_t>(t, 2 * device_cus());
-  hipLaunchKernelGGL((plain_product_kernel<Epi>), dim3(gx, two ? 2 : 1), dim3(128), 0, stream, bad, one_flag ? 0 : 1, nb, one,
-                     two ? *two : one);
-  PTO_LAUNCHED("plain_product");
-  return 0;
-}
 
 // Zero the pads of up to kPadBufs batched [rows][ld] buffers in one launch:
 // columns [cols, ld) of rows [0, rows) and all of rows [rows, prows).

@@ -309,3 +309,14 @@ def test_two_sided_split_non_finite_lands_where_fp32_puts_it():
     plain = _chain(_chain(A, X.mT), B.mT)
     got = ops.precond_apply_two_sided(A.cuda(), X.cuda(), B.cuda())
     assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), plain.nan_to_num(7.0, 8.0, 9.0))
+
+
+@pytest.mark.parametrize("b,m,n", [(4, 1830, 1840)])
+def test_two_sided_batch_gives_single_bits(b, m, n):
+    A, X, B = (t.cuda() for t in _sides(b, m, n))
+    X[1, 4, 6], B[2, 1, 7] = math.nan, math.inf
+    for a, bb in ((A, B), (A[:1], B), (A, B[:1])):
+        got = ops.precond_apply_two_sided(a, X, bb)
+        for i in range(b):
+            one = ops.precond_apply_two_sided(a[i % len(a)], X[i], bb[i % len(bb)])
+            assert torch.equal(got[i].nan_to_num(7.0, 8.0, 9.0), one.nan_to_num(7.0, 8.0, 9.0))
