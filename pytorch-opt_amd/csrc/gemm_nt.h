@@ -515,6 +515,12 @@ __device__ __forceinline__ void store_rows(const typename MF::cvec_t (&acc)[FM][
   }
 }
 
+// kOwnPlain: the plain values take an epilogue of their own in the kernel.
+template <class E, class = void>
+struct OwnPlain : std::false_type {};
+template <class E>
+struct OwnPlain<E, std::enable_if_t<E::kOwnPlain>> : std::true_type {};
+
 // Epilogues of split operands have one more argument, whether the values come
 // from the fp32 MFMA and carry no scales.
 template <class Epi>
@@ -546,15 +552,18 @@ struct SplitEpi {
 // gradient with an infinity: 1.45 ms, against 1.12 on the fp32 kernels and 23.6
 // in scalar multiply-adds.
 template <class Cfg, int FM, int FN>
-__device__ __forceinline__ void plain_sums(const SplitArgs& g, int b, int row0, int col0, int wave, int lane, char* st0,
-                                           char* st1, Mfma<float>::cvec_t (&acc)[FM][FN]) {
+__device__ __forceinline__ void plain_sums(const SplitArgs& g, int b, int row0, int col0, int wave, int lane,
+                                           char* const (&st)[8], Mfma<float>::cvec_t (&acc)[FM][FN]) {
   typedef Mfma<float> MF;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, WTM = 16 * FM, WTN = 16 * FN;
   constexpr int CH = (BM + BN) * 4, PER = CH / Cfg::NT;
+  // K tiles of 16 per step: the small tiles' MFMAs do not cover the loads of one
+  // (768² NS5 with a small row 525 us with one, 477 with four)
+  constexpr int KU = PER > 3 ? 1 : Cfg::NS / 2;
   static_assert(Cfg::KG == 1 && CH % Cfg::NT == 0 && BM * 4 % 64 == 0, "whole chunks per thread, one operand per wave");
   const int tid = wave * 64 + lane, wm = wave / Cfg::WN, wn = wave % Cfg::WN;
   const int lr = lane & 15, ch = (lane >> 4) ^ swz(lr);
-  uint4 v[PER];
+  uint4 v[KU][PER];
   // chunk e of a K tile: k 4c .. 4c + 3 of row r of its operand (lanes along
   // whichever index is contiguous)
   auto place = [&](int e, int& r, int& c) {
@@ -566,57 +575,67 @@ __device__ __forceinline__ void plain_sums(const SplitArgs& g, int b, int row0, 
   };
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      const int e = tid + q * Cfg::NT;
-      const bool isp = e < BM * 4;
-      const PlainOperand& o = isp ? g.fP : g.fQ;
-      int r, c;
-      place(e, r, c);
-      const int64_t row = (isp ? row0 : col0) + r;
-      const int kk = k0 + 4 * c, n = row < (isp ? g.M : g.N) ? min(4, g.fK - kk) : 0;
-      const float* p = o.p + (int64_t)b * o.batch + row * o.row + kk * o.k;
-      v[q] = make_uint4(0, 0, 0, 0);
-      if (row == o.ones_at) {
-        const unsigned one = __float_as_uint(1.f);
-        v[q] = make_uint4(n > 0 ? one : 0, n > 1 ? one : 0, n > 2 ? one : 0, n > 3 ? one : 0);
-      } else if (o.k == 1 && n == 4) {
-        __builtin_memcpy(&v[q], p, 16);
-      } else {
-        if (n > 0) v[q].x = __float_as_uint(p[0]);
-        if (n > 1) v[q].y = __float_as_uint(p[o.k]);
-        if (n > 2) v[q].z = __float_as_uint(p[2 * o.k]);
-        if (n > 3) v[q].w = __float_as_uint(p[3 * o.k]);
+    for (int u = 0; u < KU; ++u)
+#pragma unroll
+      for (int q = 0; q < PER; ++q) {
+        const int e = tid + q * Cfg::NT;
+        const bool isp = e < BM * 4;
+        const PlainOperand& o = isp ? g.fP : g.fQ;
+        int r, c;
+        place(e, r, c);
+        const int64_t row = (isp ? row0 : col0) + r;
+        const int kk = k0 + 16 * u + 4 * c, n = row < (isp ? g.M : g.N) ? min(4, g.fK - kk) : 0;
+        const float* p = o.p + (int64_t)b * o.batch + row * o.row + kk * o.k;
+        uint4& w = v[u][q];
+        w = make_uint4(0, 0, 0, 0);
+        if (row == o.ones_at) {
+          const unsigned one = __float_as_uint(1.f);
+          w = make_uint4(n > 0 ? one : 0, n > 1 ? one : 0, n > 2 ? one : 0, n > 3 ? one : 0);
+        } else if (o.k == 1 && n == 4) {
+          __builtin_memcpy(&w, p, 16);
+        } else {
+          if (n > 0) w.x = __float_as_uint(p[0]);
+          if (n > 1) w.y = __float_as_uint(p[o.k]);
+          if (n > 2) w.z = __float_as_uint(p[2 * o.k]);
+          if (n > 3) w.w = __float_as_uint(p[3 * o.k]);
+        }
+      }
+  };
+  auto step = [&](int k0, auto set) {
+    constexpr int S0 = decltype(set)::value * KU;
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+#pragma unroll
+      for (int q = 0; q < PER; ++q) {
+        const int e = tid + q * Cfg::NT;
+        int r, c;
+        place(e, r, c);
+        if (e >= BM * 4) r += BM;
+        *reinterpret_cast<uint4*>(st[S0 + u] + r * kRowBytes + (c ^ swz(r)) * 16) = v[u][q];
+      }
+    stage_barrier();
+    if (k0 + 16 * KU < g.fK) fetch(k0 + 16 * KU);
+#pragma unroll
+    for (int u = 0; u < KU; ++u) {
+      const char* s = st[S0 + u];
+      uint4 bf[FN];
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+        bf[fn] = *reinterpret_cast<const uint4*>(s + (BM + wn * WTN + fn * 16 + lr) * kRowBytes + ch * 16);
+#pragma unroll
+      for (int fm = 0; fm < FM; ++fm) {
+        const uint4 af = *reinterpret_cast<const uint4*>(s + (wm * WTM + fm * 16 + lr) * kRowBytes + ch * 16);
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+          for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = MF::mma(af, bf[fn], ii, acc[fm][fn]);
       }
     }
   };
-  auto step = [&](int k0, char* st) {
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      const int e = tid + q * Cfg::NT;
-      int r, c;
-      place(e, r, c);
-      if (e >= BM * 4) r += BM;
-      *reinterpret_cast<uint4*>(st + r * kRowBytes + (c ^ swz(r)) * 16) = v[q];
-    }
-    stage_barrier();
-    if (k0 + 16 < g.fK) fetch(k0 + 16);
-    uint4 bf[FN];
-#pragma unroll
-    for (int fn = 0; fn < FN; ++fn)
-      bf[fn] = *reinterpret_cast<const uint4*>(st + (BM + wn * WTN + fn * 16 + lr) * kRowBytes + ch * 16);
-#pragma unroll
-    for (int fm = 0; fm < FM; ++fm) {
-      const uint4 af = *reinterpret_cast<const uint4*>(st + (wm * WTM + fm * 16 + lr) * kRowBytes + ch * 16);
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-        for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = MF::mma(af, bf[fn], ii, acc[fm][fn]);
-    }
-  };
   fetch(0);
-  for (int k0 = 0; k0 < g.fK; k0 += 32) {
-    step(k0, st0);
-    if (k0 + 16 < g.fK) step(k0 + 16, st1);
+  for (int k0 = 0; k0 < g.fK; k0 += 32 * KU) {
+    step(k0, std::integral_constant<int, 0>{});
+    if (k0 + 16 * KU < g.fK) step(k0 + 16 * KU, std::integral_constant<int, 1>{});
   }
   stage_barrier();  // the arrays host the epilogue staging next
 }
@@ -768,13 +787,16 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(Args g, Epi epi) {
 #pragma unroll
       for (int r = 0; r < MF::NACC; ++r) acc[fm][fn][r] = 0;
   bool plain = false;
+  constexpr bool kOwnPlain = kSplit && (COMP || OwnPlain<Epi>::value);
   if constexpr (kSplit) {
     plain = g.plain != nullptr && g.plain[(int64_t)b * g.plain_stride] != 0;
     if (plain) {
-      plain_sums<Cfg>(g, b, row0, col0, wave, lane, st0, st1, acc);
-      if constexpr (COMP) {
+      char* const st[8] = {st0, st1, st2, st3, st4, st5, st6, st7};
+      plain_sums<Cfg>(g, b, row0, col0, wave, lane, st, acc);
+      if constexpr (kOwnPlain) {
         // an epilogue of its own: joining the block sums' one cost the 64² tile
-        // 8% of every call (the kernels without them are 0.7% faster joined)
+        // 8% of every call, and the choice of format in NS5's stores 1.5%; the
+        // others are 0.7% faster joined
         const int wa = wave / Plan::WPA;
         char* arr = wa == 0 ? st0 : wa == 1 ? st1 : wa == 2 ? st2 : wa == 3 ? st3 : wa == 4 ? st4 : wa == 5 ? st5 : wa == 6 ? st6 : st7;
         S* stg = reinterpret_cast<S*>(arr) + (wave % Plan::WPA) * Plan::RPP * Plan::SP;
@@ -956,7 +978,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(Args g, Epi epi) {
   // outstanding). The launchers require K to be a multiple of NS tiles, so
   // every step of the unrolled group is a real one and the MFMAs need no
   // branch.
-  const int KT = kSplit ? (plain && !COMP ? 0 : 2 * (g.K / BK)) : g.K / BK;
+  const int KT = kSplit ? (plain && !kOwnPlain ? 0 : 2 * (g.K / BK)) : g.K / BK;
   if constexpr (KG == 2) {
     // K groups: waves 0..NWG-1 (group 0) take the even K tiles, the others
     // the odd ones, each group accumulating the whole tile in its own
@@ -1344,7 +1366,7 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_nt_kernel(Args g, Epi epi) {
 #undef PTO_SLOT
   }
   if constexpr (kSplit) {
-    SplitEpi<Epi> se{epi, plain && !COMP};
+    SplitEpi<Epi> se{epi, plain && !kOwnPlain};
     store_rows<MF, Plan, UPPER, 0>(acc, stg, se, g, b, wr0, wc0, diag, lane);
   } else if constexpr (KG == 1) {
     store_rows<MF, Plan, UPPER, 0>(acc, stg, epi, g, b, wr0, wc0, diag, lane);

@@ -191,7 +191,24 @@ size_t ns5_ws_bytes_t(int64_t batch, int64_t rows, int64_t cols) {
 struct NsExp {
   int x, a, b, xn;  // planes hold X·2^x, A·2^a, B'·2^b; the next iterate's x
 };
-constexpr int kNsSplitSteps = 32;  // per matrix: exponents of this many steps
+constexpr int kNsSplitSteps = 31;
+struct NsMat {
+  NsExp e[kNsSplitSteps];
+  int plain;  // planes do not serve: the fp32 chain, in the same buffers
+  int pad[3];
+};
+constexpr int kNsMatExp = sizeof(NsMat) / sizeof(NsExp), kNsMatInt = sizeof(NsMat) / sizeof(int);
+
+// A matrix keeps the planes if the largest value of every row and column that is
+// not empty is at least 2^-16 of ρ. Their scales follow ρ and the bounds x_t, so
+// a value is held to about 2^-39 of ρ, and every step rounds so again. A row of a
+// 1500² matrix at 2^-15.2 of ρ comes out 2.4e-6 off (3.6e-6 on the fp32 chain);
+// at 2^-17 it would pass that, and one at 1e-8 of the others was 13% off. The
+// rows of a random matrix lie at 2^-7 (512²) to 2^-11 (4096 x 11008). A unit that
+// hardly fires makes a smaller one, and its matrix takes the fp32 chain (2048²
+// 2.47 ms, against 0.70 on planes and 1.57 on the fp32 kernels; one of twelve
+// 2048² 11.4 ms for all, against 5.3 and 16.4).
+constexpr float kNsSpread = 1.f / 65536;
 
 // x_{t+1}: max |p| over [0, x], with 1% for the products' rounding. |p| is largest
 // at the end of the interval or where p' = a + 3b·s² + 5c·s⁴ = 0.
@@ -244,53 +261,73 @@ __device__ __forceinline__ int ns_exp(double bound) {
   return max(-120, min(120, kSplitTop - k));
 }
 
-// 1 / (‖G‖ + eps) as ns_scale_kernel gives it, and the exponents of all steps.
+// 1 / (‖G‖ + eps) as ns_scale_kernel gives it, the exponents of all steps and the
+// choice of arithmetic, from the maxima of G's rows and columns (one thread each,
+// over their parts).
 __global__ void __launch_bounds__(256) ns_split_scale_kernel(const double* __restrict__ partial, double eps, int steps,
-                                                             double a, double b, double c, float* __restrict__ scale,
-                                                             NsExp* __restrict__ ex) {
-  const double s = block_sum_partials(partial, blockIdx.x);
-  if (threadIdx.x != 0) return;
-  const float norm = static_cast<float>(sqrt(s));
+                                                             double a, double b, double c, SplitPack g, int row_parts,
+                                                             int col_parts, int sums, float* __restrict__ scale,
+                                                             NsMat* __restrict__ mat) {
+  const int bm = blockIdx.y;
+  const float norm = static_cast<float>(sqrt(block_sum_partials(partial, bm, sums)));
+  const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const bool row = at < g.rows;
+  if (row || at - g.rows < g.cols) {
+    const int64_t i = row ? at : at - g.rows, w = row ? g.mw : g.nw;
+    const int parts = row ? row_parts : col_parts;
+    const unsigned* p = (row ? g.rpart : g.cpart) + (int64_t)bm * parts * w + i;
+    unsigned m = 0;
+#pragma unroll 8
+    for (int k = 0; k < parts; ++k) m = max(m, p[k * w]);
+    if (m >= kInfBits || (m != 0 && !(__uint_as_float(m) >= kNsSpread * norm))) mat[bm].plain = 1;
+  }
+  if (at != 0) return;
   const float sc = 1.f / (norm + static_cast<float>(eps));
-  scale[blockIdx.x] = sc;
-  NsExp* e = ex + (int64_t)blockIdx.x * kNsSplitSteps;
+  scale[bm] = sc;
   double x = (double)norm * sc;
-  int ex_t = ns_exp(x);
+  int ex = ns_exp(x);
   for (int t = 0; t < steps; ++t) {
     const double u = x * x;
     x = ns_next_bound(a, b, c, x);
     const int nxt = ns_exp(x);
-    e[t] = NsExp{ex_t, ns_exp(u), ns_exp(fabs(a) + fabs(b) * u + fabs(c) * u * u), nxt};
-    ex_t = nxt;
+    mat[bm].e[t] = NsExp{ex, ns_exp(u), ns_exp(fabs(a) + fabs(b) * u + fabs(c) * u * u), nxt};
+    ex = nxt;
   }
+}
+
+// The exponents of matrix b in the step that ex points at
+__device__ __forceinline__ NsExp ns_exps(const NsExp* ex, int b, bool plain) {
+  return plain ? NsExp{0, 0, 0, 0} : ex[(int64_t)b * kNsMatExp];
 }
 
 // A = v·2^-2x, into its planes
 struct EpiNsGramSplit {
   typedef float S;
+  static constexpr bool kOwnPlain = true;
   sp16* dst;
   int64_t pl, ld, sd;
-  const NsExp* ex;  // matrix b: ex[b * kNsSplitSteps]
+  const NsExp* ex;  // matrix b: ex[b * kNsMatExp]
   typedef NoPre Pre;
   typedef NoPre PreT;
   static constexpr bool kVoIsV = true;
   __device__ __forceinline__ bool has_t() const { return false; }
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&, bool) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&, bool) const {}
-  __device__ __forceinline__ void store(int b, int64_t o, const S* v, int kbeg, int n) const {
-    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+  __device__ __forceinline__ void store(int b, int64_t o, const S* v, int kbeg, int n, bool plain) const {
+    const NsExp e = ns_exps(ex, b, plain);
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], e.a - 2 * e.x);
-    st8_split(dst + (int64_t)b * sd + o, pl, w, kbeg, n);
+    st8_split(dst + (int64_t)b * sd, o, pl, w, kbeg, n, plain);
   }
-  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo, bool) const {
-    store(b, (int64_t)i * ld + j0, v, kbeg, n);
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo,
+                                      bool plain) const {
+    store(b, (int64_t)i * ld + j0, v, kbeg, n, plain);
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = v[k];
   }
-  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool) const {
-    store(b, (int64_t)j * ld + i0, v, 0, n);
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool plain) const {
+    store(b, (int64_t)j * ld + i0, v, 0, n, plain);
   }
   __device__ __forceinline__ void finish(int) const {}
 };
@@ -298,38 +335,44 @@ struct EpiNsGramSplit {
 // B' = a·I + b·A + c·v·2^-2a
 struct EpiNsSqSplit {
   typedef float S;
+  static constexpr bool kOwnPlain = true;
   const sp16* Asrc;
   sp16* dst;
   int64_t pl, ld, sd;
   float ac, bc, cc;
   const NsExp* ex;
   struct Pre {
-    uint4 h, l;
+    uint4 h, l;  // plain: eight fp32 values
   };
   typedef NoPre PreT;
   static constexpr bool kVoIsV = false;  // the mirror stores B', not the raw product
   __device__ __forceinline__ bool has_t() const { return false; }
-  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p, bool) const {
+  __device__ __forceinline__ void load(int b, int i, int j0, int kbeg, int n, Pre& p, bool plain) const {
     if (full_run(kbeg, n)) {
-      const sp16* q = Asrc + (int64_t)b * sd + (int64_t)i * ld + j0;
+      const int64_t o = (int64_t)i * ld + j0;
+      const sp16* q = Asrc + (int64_t)b * sd + (plain ? 2 * o : o);
       p.h = ld16(q);
-      p.l = ld16(q + pl);
+      p.l = ld16(q + (plain ? 8 : pl));
     }
   }
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&, bool) const {}
-  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre,
-                                      S* vo, bool) const {
-    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
-    const int64_t o = (int64_t)b * sd + (int64_t)i * ld + j0;
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre& pre, S* vo,
+                                      bool plain) const {
+    const NsExp e = ns_exps(ex, b, plain);
+    const int64_t o = (int64_t)i * ld + j0;
+    const sp16* A = Asrc + (int64_t)b * sd;
     S a[8];
     if (full_run(kbeg, n)) {
       const f16x8_t h = __builtin_bit_cast(f16x8_t, pre.h), l = __builtin_bit_cast(f16x8_t, pre.l);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) a[k] = static_cast<S>(h[k]) + static_cast<S>(l[k]);
-    } else {
+      const unsigned u[8] = {pre.h.x, pre.h.y, pre.h.z, pre.h.w, pre.l.x, pre.l.y, pre.l.z, pre.l.w};
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        a[k] = k >= kbeg && k < n ? static_cast<S>(Asrc[o + k].v) + static_cast<S>(Asrc[o + pl + k].v) : S(0);
+        a[k] = plain ? __uint_as_float(u[k]) : static_cast<S>(h[k]) + static_cast<S>(l[k]);
+    } else {
+      for (int k = 0; k < 8; ++k)
+        a[k] = k < kbeg || k >= n ? S(0)
+               : plain            ? reinterpret_cast<const float*>(A)[o + k]
+                                  : static_cast<S>(A[o + k].v) + static_cast<S>(A[o + pl + k].v);
     }
     S w[8];
 #pragma unroll
@@ -337,14 +380,14 @@ struct EpiNsSqSplit {
       vo[k] = fma(cc, ldexpf(v[k], -2 * e.a), fma(bc, ldexpf(a[k], -e.a), i == j0 + k ? ac : 0.f));
       w[k] = ldexpf(vo[k], e.b);
     }
-    st8_split(dst + o, pl, w, kbeg, n);
+    st8_split(dst + (int64_t)b * sd, o, pl, w, kbeg, n, plain);
   }
-  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool) const {
-    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool plain) const {
+    const NsExp e = ns_exps(ex, b, plain);
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], e.b);
-    st8_split(dst + (int64_t)b * sd + (int64_t)j * ld + i0, pl, w, 0, n);
+    st8_split(dst + (int64_t)b * sd, (int64_t)j * ld + i0, pl, w, 0, n, plain);
   }
   __device__ __forceinline__ void finish(int) const {}
 };
@@ -353,6 +396,7 @@ struct EpiNsSqSplit {
 // fp32 into out, row-major (dst) or transposed (dstT).
 struct EpiNsUpdateSplit {
   typedef float S;
+  static constexpr bool kOwnPlain = false;
   sp16* planes;
   int64_t pl, ld, sd;
   float* dst;
@@ -365,23 +409,24 @@ struct EpiNsUpdateSplit {
   __device__ __forceinline__ bool has_t() const { return dstT != nullptr; }
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&, bool) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&, bool) const {}
-  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo, bool) const {
-    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+  __device__ __forceinline__ void put(int b, int i, int j0, const S* v, int kbeg, int n, const Pre&, S* vo,
+                                      bool plain) const {
+    const NsExp e = ns_exps(ex, b, plain);
 #pragma unroll
     for (int k = 0; k < 8; ++k) vo[k] = v[k];
     S w[8];
     if (planes) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], e.xn - e.b - e.x);
-      st8_split(planes + (int64_t)b * sd + (int64_t)i * ld + j0, pl, w, kbeg, n);
+      st8_split(planes + (int64_t)b * sd, (int64_t)i * ld + j0, pl, w, kbeg, n, plain);
     } else if (dst) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], -e.b - e.x);
       st8<float, S>(dst + (int64_t)b * s_o + (int64_t)i * ld_o + j0, w, kbeg, n);
     }
   }
-  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool) const {
-    const NsExp e = ex[(int64_t)b * kNsSplitSteps];
+  __device__ __forceinline__ void put_t(int b, int j, int i0, const S* v, int n, const PreT&, bool plain) const {
+    const NsExp e = ns_exps(ex, b, plain);
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = ldexpf(v[k], -e.b - e.x);
@@ -396,7 +441,7 @@ size_t ns5_split_ws_bytes(int64_t batch, int64_t m, int64_t n) {
   auto add = [&](size_t b) { bytes = round_up(bytes, 256) + b; };
   add(sizeof(double) * kRedBlocks * batch);
   add(sizeof(float) * batch);
-  add(sizeof(NsExp) * kNsSplitSteps * batch);
+  add(sizeof(NsMat) * batch);
   add(sizeof(sp16) * 2 * batch * ldm * ldm);  // A
   add(sizeof(sp16) * 2 * batch * ldm * ldm);  // B'
   add(sizeof(sp16) * 2 * batch * ldm * ldn);  // X ping
@@ -427,28 +472,49 @@ int ns5_split_run(const float* G, float* out, int64_t batch, int64_t rows, int64
   Carver cv(ws, ws_bytes);
   double* partial = cv.take<double>(kRedBlocks * batch);
   float* scale = cv.take<float>(batch);
-  NsExp* ex = cv.take<NsExp>(kNsSplitSteps * batch);
+  NsMat* mat = cv.take<NsMat>(batch);
   sp16* Ab = cv.take<sp16>(batch * sA);
   sp16* Bb = cv.take<sp16>(batch * sA);
   sp16* X[2];
   for (sp16*& x : X) x = cv.take<sp16>(batch * sX);
   PTO_REQUIRE(!cv.overflow, "newton_schulz_orthogonalize: workspace too small");
 
-  if (launch_sumsq<float>(G, rows, cols, cols, sG, nb, partial, stream)) return -1;
-  hipLaunchKernelGGL(ns_split_scale_kernel, dim3(nb), dim3(256), 0, stream, partial, eps, (int)steps, a, b, c, scale,
-                     ex);
+  // ‖G‖ and the maxima of its rows and columns from one read, at most kRedBlocks
+  // workgroups a matrix; the maxima's parts lie where the second iterate will
+  const int64_t gx = absmax_row_parts(cols), gy = std::min((rows + 31) / 32, kRedBlocks / std::min<int64_t>(gx, kRedBlocks));
+  const int nr = (int)round_up((rows + gy - 1) / gy, 32);
+  const int64_t ny = (rows + nr - 1) / nr;
+  SplitPack g{G, rows, cols, cols, sG};
+  g.rpart = reinterpret_cast<unsigned*>(X[1]);
+  g.cpart = g.rpart + batch * rows * gx;
+  g.mw = rows;
+  g.nw = cols;
+  g.bad = &mat->plain;
+  g.bad_stride = kNsMatInt;
+  PTO_REQUIRE(4 * (rows * gx + cols * ny) <= (int64_t)sizeof(sp16) * sX, "newton_schulz_orthogonalize: workspace too small");
+  const bool one_read = gx * ny <= kRedBlocks;
+  const dim3 grid((unsigned)gx, (unsigned)ny, (unsigned)nb);
+  if (one_read) {
+    hipLaunchKernelGGL((absmax_kernel<true>), grid, dim3(256), 0, stream, g, nr, 1, partial);
+  } else {
+    if (launch_sumsq<float>(G, rows, cols, cols, sG, nb, partial, stream)) return -1;
+    hipLaunchKernelGGL((absmax_kernel<false>), grid, dim3(256), 0, stream, g, nr, 1, partial);
+  }
+  PTO_LAUNCHED("absmax");
+  hipLaunchKernelGGL(ns_split_scale_kernel, dim3((unsigned)((rows + cols + 255) / 256), (unsigned)nb), dim3(256), 0,
+                     stream, partial, eps, (int)steps, a, b, c, g, (int)gx, (int)ny,
+                     one_read ? (int)(gx * ny) : kRedBlocks, scale, mat);
   PTO_LAUNCHED("ns_split_scale");
-  const int* ex0 = &ex->x;
-  const int ex_stride = kNsSplitSteps * (int)(sizeof(NsExp) / sizeof(int));
+  const int* ex0 = &mat->e[0].x;
   if (!transposed) {
     const unsigned gx = (unsigned)std::min<int64_t>((ldm * (ldn / 8) + 255) / 256, 4096);
     hipLaunchKernelGGL(split_pack_kernel, dim3(gx, (unsigned)nb), dim3(256), 0, stream, G, rows, cols, cols, sG, scale,
-                       ex0, ex_stride, X[0], plX, ldm, ldn, sX);
+                       ex0, kNsMatInt, &mat->plain, X[0], plX, ldm, ldn, sX);
   } else {
     const dim3 grid((unsigned)(ldm / 64), (unsigned)(ldn / 64), (unsigned)nb);
     PTO_REQUIRE(grid.y < 65536, "newton_schulz_orthogonalize: shape too large");
-    hipLaunchKernelGGL(split_pack_t_kernel, grid, dim3(256), 0, stream, G, rows, cols, cols, sG, scale, ex0, ex_stride,
-                       X[0], plX, ldm, ldn, sX);
+    hipLaunchKernelGGL(split_pack_t_kernel, grid, dim3(256), 0, stream, G, rows, cols, cols, sG, scale, ex0, kNsMatInt,
+                       &mat->plain, X[0], plX, ldm, ldn, sX);
   }
   PTO_LAUNCHED("split_pack");
   PadList pads;
@@ -456,17 +522,25 @@ int ns5_split_run(const float* G, float* out, int64_t batch, int64_t rows, int64
   if (steps > 1) pads.add(X[1], m, ldm, n, ldn, plX, 2 * nb);
   if (launch_zero_pads(pads, stream)) return -1;
 
+  // the buffers of a plain matrix, as fp32 of the same extents
+  auto rows_of = [](const sp16* p, int64_t ld, int64_t pl) {
+    return PlainOperand{reinterpret_cast<const float*>(p), ld, 1, pl, -1};
+  };
+  auto args = [&](const sp16* P, int64_t ldp, int64_t plP, const sp16* Q, int64_t ldq, int64_t plQ, int64_t N, int64_t K) {
+    return SplitArgs{{P, ldp, 2 * plP, Q, ldq, 2 * plQ, (int)m, (int)N, (int)round_up(K, kPadK)}, plP, plQ,
+                     &mat->plain, kNsMatInt, rows_of(P, ldp, plP), rows_of(Q, ldq, plQ), (int)K};
+  };
   for (int64_t t = 0; t < steps; ++t) {
     const bool last = t == steps - 1;
     const sp16* Xc = X[t & 1];
+    const NsExp* ex = &mat->e[t];
     {
-      SplitArgs g{{Xc, ldn, sX, Xc, ldn, sX, (int)m, (int)m, (int)ldn}, plX, plX};
-      EpiNsGramSplit e{Ab, plA, ldm, sA, ex + t};
-      if (launch_gemm<sp16, true>(g, e, nb, stream, "ns5_gram")) return -1;
+      EpiNsGramSplit e{Ab, plA, ldm, sA, ex};
+      if (launch_gemm<sp16, true>(args(Xc, ldn, plX, Xc, ldn, plX, m, n), e, nb, stream, "ns5_gram")) return -1;
     }
     {
-      SplitArgs g{{Ab, ldm, sA, Ab, ldm, sA, (int)m, (int)m, (int)ldm}, plA, plA};
-      EpiNsSqSplit e{Ab, Bb, plA, ldm, sA, (float)a, (float)b, (float)c, ex + t};
+      const SplitArgs g = args(Ab, ldm, plA, Ab, ldm, plA, m, m);
+      EpiNsSqSplit e{Ab, Bb, plA, ldm, sA, (float)a, (float)b, (float)c, ex};
       // A's rows are its columns: read K-contiguous by the 256² and 192² tiles
       // (12 x 2048²: 310 us against 325 with transposing reads), transposing
       // by the smaller ones, whose LDS reads bound them (128² 317 against 350)
@@ -478,9 +552,10 @@ int ns5_split_run(const float* G, float* out, int64_t batch, int64_t rows, int64
       }
     }
     {
-      SplitArgs g{{Bb, ldm, sA, Xc, ldn, sX, (int)m, (int)n, (int)ldm}, plA, plX};
+      SplitArgs g = args(Bb, ldm, plA, Xc, ldn, plX, n, m);
+      std::swap(g.fQ.row, g.fQ.k);  // X as [K][N]
       EpiNsUpdateSplit e{last ? nullptr : X[(t & 1) ^ 1], plX, ldn, sX, last && !transposed ? out : nullptr,
-                         last && transposed ? out : nullptr, cols, sG, ex + t};
+                         last && transposed ? out : nullptr, cols, sG, ex};
       if (launch_gemm_qn<EpiNsUpdateSplit, true, false, sp16>(g, e, nb, stream, "ns5_update")) return -1;
     }
   }

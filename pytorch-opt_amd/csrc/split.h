@@ -43,7 +43,7 @@ __device__ __forceinline__ Split8 split8(const float* v) {
 }
 
 // p[k] and p[pl + k] = the planes of in[k] for k in [kbeg, n)
-__device__ __forceinline__ void st8_split(sp16* p, int64_t pl, const float* in, int kbeg, int n) {
+__device__ __forceinline__ void st8_planes(sp16* p, int64_t pl, const float* in, int kbeg, int n) {
   const Split8 s = split8(in);
   if (full_run(kbeg, n)) {
     st16(p, s.h);
@@ -60,21 +60,31 @@ __device__ __forceinline__ void st8_split(sp16* p, int64_t pl, const float* in, 
   }
 }
 
+// Elements o + k of a matrix held at m as planes, or as fp32 in their place
+__device__ __forceinline__ void st8_split(sp16* m, int64_t o, int64_t pl, const float* in, int kbeg, int n, bool plain) {
+  if (plain)
+    st8<float, float>(reinterpret_cast<float*>(m) + o, in, kbeg, n);
+  else
+    st8_planes(m + o, pl, in, kbeg, n);
+}
+
 // Split planes of a fp32 matrix: out (h plane [orows][ld], l plane pl
 // elements on) = planes of in(r, c)·scale_b·2^e, pads (columns to ld, rows to
-// orows) zero. e = e_mat[b * e_mat_stride] (per matrix).
+// orows) zero. e = e_mat[b * e_mat_stride] (per matrix). A matrix with
+// plain[b * e_mat_stride] != 0 is stored as fp32 in the place of its planes.
 // Each thread takes eight consecutive output columns: 32 bytes in, 16 + 16
 // out. Bound by memory: 8 bytes per element.
 [[maybe_unused]] static __global__ void __launch_bounds__(256) split_pack_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
                                                          int64_t ld_in, int64_t s_in, const float* __restrict__ scale,
                                                          const int* __restrict__ e_mat, int e_mat_stride,
-                                                         sp16* __restrict__ out, int64_t pl, int64_t orows, int64_t ld,
-                                                         int64_t s_out) {
+                                                         const int* __restrict__ plain, sp16* __restrict__ out,
+                                                         int64_t pl, int64_t orows, int64_t ld, int64_t s_out) {
   const int b = blockIdx.y;
   const float* ib = in + (int64_t)b * s_in;
   sp16* ob = out + (int64_t)b * s_out;
   const float sc = scale ? scale[b] : 1.f;
-  const int e = e_mat[(int64_t)b * e_mat_stride];
+  const bool as_is = plain[(int64_t)b * e_mat_stride] != 0;
+  const int e = as_is ? 0 : e_mat[(int64_t)b * e_mat_stride];
   const int64_t nch = ld / 8, total = orows * nch;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
     const int64_t r = i / nch, c0 = (i - r * nch) * 8;
@@ -89,6 +99,10 @@ __device__ __forceinline__ void st8_split(sp16* p, int64_t pl, const float* in, 
       for (int k = 0; k < 8; ++k)
         v[k] = r < rows && c0 + k < cols ? ldexpf(ib[r * ld_in + c0 + k] * sc, e) : 0.f;
     }
+    if (as_is) {
+      st8<float, float>(reinterpret_cast<float*>(ob) + r * ld + c0, v, 0, 8);
+      continue;
+    }
     const Split8 s = split8(v);
     *reinterpret_cast<uint4*>(ob + r * ld + c0) = s.h;
     *reinterpret_cast<uint4*>(ob + pl + r * ld + c0) = s.l;
@@ -101,15 +115,16 @@ __device__ __forceinline__ void st8_split(sp16* p, int64_t pl, const float* in, 
 [[maybe_unused]] static __global__ void __launch_bounds__(256) split_pack_t_kernel(const float* __restrict__ in, int64_t rows, int64_t cols,
                                                            int64_t ld_in, int64_t s_in, const float* __restrict__ scale,
                                                            const int* __restrict__ e_mat, int e_mat_stride,
-                                                           sp16* __restrict__ out, int64_t pl, int64_t orows,
-                                                           int64_t ld, int64_t s_out) {
+                                                           const int* __restrict__ plain, sp16* __restrict__ out,
+                                                           int64_t pl, int64_t orows, int64_t ld, int64_t s_out) {
   __shared__ float tile[64][65];
   const int b = blockIdx.z;
   const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
   const float* ib = in + (int64_t)b * s_in;
   sp16* ob = out + (int64_t)b * s_out;
   const float sc = scale ? scale[b] : 1.f;
-  const int e = e_mat[(int64_t)b * e_mat_stride];
+  const bool as_is = plain[(int64_t)b * e_mat_stride] != 0;
+  const int e = as_is ? 0 : e_mat[(int64_t)b * e_mat_stride];
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -125,6 +140,10 @@ __device__ __forceinline__ void st8_split(sp16* p, int64_t pl, const float* in, 
     float v[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = tile[rr + k][cc];
+    if (as_is) {
+      st8<float, float>(reinterpret_cast<float*>(ob) + c * ld + r, v, 0, 8);
+      continue;
+    }
     const Split8 s = split8(v);
     *reinterpret_cast<uint4*>(ob + c * ld + r) = s.h;
     *reinterpret_cast<uint4*>(ob + pl + c * ld + r) = s.l;
@@ -162,6 +181,7 @@ struct SplitPack {
   int64_t s_pre = 0;
   int pre_mul = 0, pre_off = 0;
   const int* er_add = nullptr;  // stride mw
+  int bad_stride = 1;
   __device__ __forceinline__ int pre(const int* p, int b, int64_t at, int64_t n) const {
     return p && at < n ? pre_off + pre_mul * p[(int64_t)b * s_pre + at] : 0;
   }
@@ -177,22 +197,25 @@ __device__ __forceinline__ unsigned scaled_bits(unsigned u, int e) {
 
 // Largest |x| of the parts of a fp32 matrix's rows and columns, as bit patterns
 // (which order like the values, NaN above infinity): rpart[cb][r] of columns
-// 256·cb .. + 255, cpart[rb][c] of rows nr·rb .. + nr - 1; written where out_s
-// (out_t) is. A workgroup takes nr rows (a multiple of 32) x 256 columns, a wave
+// 256·cb .. + 255, cpart[rb][c] of rows nr·rb .. + nr - 1; either may be null. A
+// workgroup takes nr rows (a multiple of 32) x 256 columns, a wave
 // eight rows at a time, 16 bytes per lane and all eight in flight (one row at a
 // time waited 32 times for memory: 30 us whatever the size). Parts need neither
 // zeroing nor atomics. Bound by memory: 4 bytes per element. clear: also clears
-// bad[b].
-[[maybe_unused]] static __global__ void __launch_bounds__(256) absmax_kernel(SplitPack a, int nr, int clear) {
+// bad[b]. SUM: also partial[b·kRedBlocks + workgroup] = the sum of its squares, in
+// fp64 (a read of its own and a launch were 5 us of a 768² NS5's 195).
+template <bool SUM>
+__global__ void __launch_bounds__(256) absmax_kernel(SplitPack a, int nr, int clear, double* __restrict__ partial) {
   __shared__ unsigned cw[4][256];
   const int b = blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t r0 = (int64_t)blockIdx.y * nr, c0 = (int64_t)blockIdx.x * 256 + lane * 4;
   const float* ib = a.in + (int64_t)b * a.s_in;
-  if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.bad[b] = 0;
+  if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.bad[(int64_t)b * a.bad_stride] = 0;
   int pc[4] = {0, 0, 0, 0};
 #pragma unroll
   for (int k = 0; k < 4; ++k) pc[k] = a.pre(a.pre_c, b, c0 + k, a.cols);
   unsigned cm[4] = {0, 0, 0, 0};
+  double sum = 0.0;
   for (int rr = wave * 8; rr < nr; rr += 32) {
     uint4 q[8];
     unsigned rm[8];
@@ -210,6 +233,17 @@ __device__ __forceinline__ unsigned scaled_bits(unsigned u, int e) {
         }
       }
     }
+    if constexpr (SUM) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const unsigned w[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const double d = __uint_as_float(w[k]);
+          sum += d * d;
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       unsigned u[4] = {q[i].x & 0x7fffffffu, q[i].y & 0x7fffffffu, q[i].z & 0x7fffffffu, q[i].w & 0x7fffffffu};
@@ -222,7 +256,7 @@ __device__ __forceinline__ unsigned scaled_bits(unsigned u, int e) {
       for (int k = 0; k < 4; ++k) cm[k] = max(cm[k], u[k]);
       rm[i] = max(max(u[0], u[1]), max(u[2], u[3]));
     }
-    if (a.out_s) {
+    if (a.rpart) {
       // eight rows over 64 lanes: three exchanges that halve the rows a lane
       // holds, three more within its eight lanes (10 shuffles for 48)
       unsigned m4[4], m2[2];
@@ -240,7 +274,16 @@ __device__ __forceinline__ unsigned scaled_bits(unsigned u, int e) {
       if ((lane & 7) == 0 && r < a.rows) a.rpart[((int64_t)b * gridDim.x + blockIdx.x) * a.mw + r] = m;
     }
   }
-  if (!a.out_t) return;
+  if constexpr (SUM) {
+    __shared__ double sw[4];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    if (lane == 0) sw[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      partial[(int64_t)b * kRedBlocks + blockIdx.y * gridDim.x + blockIdx.x] = (sw[0] + sw[1]) + (sw[2] + sw[3]);
+  }
+  if (!a.cpart) return;
 #pragma unroll
   for (int k = 0; k < 4; ++k) cw[wave][lane * 4 + k] = cm[k];
   __syncthreads();
@@ -289,7 +332,7 @@ inline int64_t absmax_col_parts(int64_t rows) { return (rows + absmax_rows(rows)
   }
   __syncthreads();
   auto check = [&](unsigned u) {
-    if (a.bad && (u >= kInfBits || ((a.pre_r || a.pre_c) && u != 0 && u < kTinyBits))) a.bad[b] = 1;
+    if (a.bad && (u >= kInfBits || ((a.pre_r || a.pre_c) && u != 0 && u < kTinyBits))) a.bad[(int64_t)b * a.bad_stride] = 1;
   };
   if (ty == 0 && a.out_s) {
     const unsigned u = max(mx[0][tx], mx[1][tx]);
@@ -325,16 +368,22 @@ inline int64_t absmax_col_parts(int64_t rows) { return (rows + absmax_rows(rows)
     }
   }
 }
-inline int launch_split_pack_max(const SplitPack& a, int batch, hipStream_t stream, bool clear = true) {
-  const int nr = absmax_rows(a.rows);
+inline int launch_absmax(const SplitPack& a, int batch, hipStream_t stream, bool clear) {
   const dim3 gm((unsigned)absmax_row_parts(a.cols), (unsigned)absmax_col_parts(a.rows), (unsigned)batch);
+  PTO_REQUIRE(gm.y < 65536 && batch < 65536, "absmax: grid too large");
+  hipLaunchKernelGGL((absmax_kernel<false>), gm, dim3(256), 0, stream, a, absmax_rows(a.rows), clear ? 1 : 0,
+                     (double*)nullptr);
+  PTO_LAUNCHED("absmax");
+  return 0;
+}
+inline int launch_split_pack_max(const SplitPack& a, int batch, hipStream_t stream, bool clear = true) {
   const int64_t rext = a.out_t ? std::max(a.rows, a.ld_t) : a.rows;
   const int64_t cext = std::max(a.cols + a.ones, a.out_s ? a.ld_s : 0);
   const dim3 gp((unsigned)((cext + 63) / 64), (unsigned)((rext + 63) / 64), (unsigned)batch);
-  PTO_REQUIRE(gm.y < 65536 && gp.y < 65536 && batch < 65536, "split_pack: grid too large");
-  hipLaunchKernelGGL(absmax_kernel, gm, dim3(256), 0, stream, a, nr, clear ? 1 : 0);
-  PTO_LAUNCHED("absmax");
-  hipLaunchKernelGGL(split_pack_max_kernel, gp, dim3(256), 0, stream, a, (int)gm.x, (int)gm.y);
+  PTO_REQUIRE(gp.y < 65536, "split_pack: grid too large");
+  if (launch_absmax(a, batch, stream, clear)) return -1;
+  hipLaunchKernelGGL(split_pack_max_kernel, gp, dim3(256), 0, stream, a, (int)absmax_row_parts(a.cols),
+                     (int)absmax_col_parts(a.rows));
   PTO_LAUNCHED("split_pack_max");
   return 0;
 }

@@ -224,8 +224,9 @@ def _rows_no_worse(got, want, plain, dim=-1, roundings=4):
     """One row's error is a sample of a few hundred roundings or more: 1.5 times
     the plain one's, or `roundings` roundings of the result."""
     e, p = _err(got, want, dim), _err(plain, want, dim)
-    worst = (e / torch.clamp(1.5 * p, min=roundings * 2.0 ** -24)).argmax()
-    assert (e <= torch.clamp(1.5 * p, min=roundings * 2.0 ** -24)).all(), (int(worst), e.flatten()[worst], p.flatten()[worst])
+    over = e / torch.clamp(1.5 * p, min=roundings * 2.0 ** -24)
+    worst = int(over.argmax())
+    assert over[worst].item() <= 1, (worst, e[worst].item(), p[worst].item())
 
 
 SMALL = {3: 1e-2, 64: 1e-4, 130: 1e-6, 131: 1e-7, 700: 1e-8, 701: 1e-12, 1100: 0.0}
@@ -320,3 +321,21 @@ def test_two_sided_batch_gives_single_bits(b, m, n):
         for i in range(b):
             one = ops.precond_apply_two_sided(a[i % len(a)], X[i], bb[i % len(bb)])
             assert torch.equal(got[i].nan_to_num(7.0, 8.0, 9.0), one.nan_to_num(7.0, 8.0, 9.0))
+
+
+@pytest.mark.parametrize("shape", [(576, 700), (700, 576), (1500, 1500)])
+@pytest.mark.parametrize("s", [1e-1, 1e-2, 1e-3, 1e-4, 1e-6, 1e-9, 1e-12])
+def test_ns5_split_keeps_small_rows_and_columns(shape, s):
+    G = _randn(21, *shape)
+    G[3] *= s
+    G[:, 130] *= s
+    G[64] = 0.0
+    got = ops.newton_schulz_orthogonalize(G.cuda())
+    want, plain = _ns64(G, 5, NS), _ns_chain(G, 5, NS)
+    _no_worse(got, want, plain)
+    # single rows' errors lie along the few smallest singular directions and so
+    # spread more than independent roundings (up to 1.6 times between two fp32
+    # chains); the small row and column are as near as any other
+    for dim, at in ((-1, 3), (-2, 130)):
+        e, p = _err(got, want, dim), _err(plain, want, dim)
+        assert e.max() <= 2 * p.max() and e[at] <= 1.5 * max(p[at].item(), _rel(plain, want))
