@@ -54,7 +54,9 @@ int pto_runtime_version(void);
  * G and out are [batch, rows, cols] of `dtype`. bf16 computes with bf16
  * operands and fp32 accumulation when min(rows, cols) >= 128 (below that
  * the fp32 chain runs and the result is rounded once, as the reference
- * computes every bf16 input); f32/f64 stay in their own precision.
+ * computes every bf16 input); f32/f64 stay in their own precision. In f32
+ * and f64 every matrix of a batch gets the bits of its single call (in bf16
+ * the tile, and so the last bits, depend on the batch).
  * out may be G itself (in place) but must not otherwise overlap it. G may
  * sit at any element alignment (a G that is not 16-byte aligned is copied
  * into the workspace first).
@@ -189,7 +191,8 @@ int pto_two_sided_product(const void* A, const void* X, const void* B, void* out
  * pytorch_opt/ops/reference.py:117-121, batched there by torch.matmul),
  * which the harnesses use for same-shape parameters (SOAP rotations,
  * K-FAC and EKFAC preconditioning, Shampoo's apply). shared_a / shared_b
- * in the workspace query: the matching stride is 0.
+ * in the workspace query: the matching stride is 0. In f32 and f64 every
+ * matrix gets the bits of its single call, shared factors or not.
  */
 size_t pto_two_sided_product_batched_workspace_bytes(int dtype, int64_t batch, int64_t m, int64_t n, int shared_a,
                                                      int shared_b);

@@ -30,16 +30,18 @@ namespace {
 // scale per row of its own maxima: with one shift for its largest possible value
 // a row at 1e-6 of the others was 2e-2 off. Without the row scales and that pass
 // 16 x 2048² takes 1.98 ms instead of 2.24.
-// From a short side of 512 and this work up: below, the passes for the scales
-// and eight more launches cost what the products save (one 1300² 127 us against
-// 117 on the fp32 MFMA, one 4096 x 512 178 against 161, before the row scales;
-// with them 8 x 512 x 2048 345 against 383, 8 x 1024² 238 against 282, one
-// 1024 x 4096 247 against 359, one 2048² 206 against 279, sixteen 2240 against
-// 4076, one 4096² 807 against 2006).
-constexpr int64_t kApplySplitSide = 512;
-constexpr double kApplySplitWork = 1.2e10;  // batch·m·n·(m + n)
-inline bool apply_split(int64_t batch, int64_t m, int64_t n) {
-  return std::min(m, n) >= kApplySplitSide && (double)batch * m * n * (m + n) >= kApplySplitWork;
+// By one matrix alone, so that a matrix gets the same bits in every batch. From a
+// short side of 512 and this work up, or of 1500: below, the passes for the scales
+// and the more launches cost a single call what the products save (us against the
+// fp32 MFMA: 1024² 108 / 51, 1300² 145 / 115, 4096 x 512 195 / 159; 1536² 152 /
+// 160, 1700² 174 / 198, 4096 x 640 208 / 236, 1024 x 3000 198 / 221, 2048² 204 /
+// 279, 4096² 820 / 2006, sixteen 2048² 2240 / 4076; eight 1024² would gain: 238 /
+// 282).
+constexpr int64_t kApplySplitSide = 512, kApplySplitSquare = 1500;
+constexpr double kApplySplitWork = 1.2e10;  // m·n·(m + n)
+inline bool apply_split(int64_t m, int64_t n) {
+  const int64_t side = std::min(m, n);
+  return side >= kApplySplitSquare || (side >= kApplySplitSide && (double)m * n * (m + n) >= kApplySplitWork);
 }
 
 struct ApplySplitWs {
@@ -125,7 +127,7 @@ int two_sided_split(const float* Am, const float* X, const float* Bm, float* out
 
 template <typename T>
 size_t apply_ws_bytes_t(int64_t m, int64_t n, int64_t batch = 1, bool shared_a = false, bool shared_b = false) {
-  if (std::is_same<T, float>::value && apply_split(batch, m, n)) return ApplySplitWs::bytes(m, n, batch);
+  if (std::is_same<T, float>::value && apply_split(m, n)) return ApplySplitWs::bytes(m, n, batch);
   int64_t ldm = round_up(m, kPadK), ldn = round_up(n, kPadK);
   size_t bytes = 0;
   auto add = [&](size_t b) { bytes = round_up(bytes, 256) + b; };
@@ -153,7 +155,7 @@ int two_sided_t(const T* Am, const T* X, const T* Bm, T* out, int64_t batch, int
   PTO_REQUIRE(sA >= 0 && sX >= 0 && sB >= 0, "two-sided product: negative stride");
   if (m == 0 || n == 0 || batch == 0) return 0;
   if constexpr (std::is_same<T, float>::value) {
-    if (apply_split(batch, m, n))
+    if (apply_split(m, n))
       return two_sided_split(Am, X, Bm, out, batch, m, n, sA, sX, sB, trans_a, trans_b, ws, ws_bytes, stream, name_left,
                              name_right);
   }

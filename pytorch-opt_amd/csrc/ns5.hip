@@ -449,17 +449,20 @@ size_t ns5_split_ws_bytes(int64_t batch, int64_t m, int64_t n) {
   return bytes + 256;
 }
 
-// Sizes that run on split operands. Below batch·m² = 512² the launches have
-// too few of the split products' 64² tiles and wait for their loads (one
-// 256 x 4096 273 us against 229 on the fp32 MFMA's 32² tiles, 384 x 1536 186
-// against 164, 512 x 512 the same, 768 x 768 183 against 221, 2048 x 2048 800
-// against 1569; eight of 256 x 1024 178 against 210, of 2048 x 2048 3.85 ms
-// against 11.3). Sides just above a multiple of 128, whose planes would not
-// fit the workspace of the fp32 chain, keep that chain.
-constexpr int64_t kNsSplitMinSide = 128, kNsSplitMinWork = 512 * 512;
-inline bool ns5_split(int64_t batch, int64_t m, int64_t n, int64_t steps, double a, double b, double c, double eps) {
-  return m >= kNsSplitMinSide && batch * m * m >= kNsSplitMinWork && ns_split_coeffs(steps, a, b, c, eps) &&
-         ns5_split_ws_bytes(batch, m, n) <= ns5_ws_bytes_t<float>(batch, m, n);
+// Sizes that run on split operands: by one matrix alone, so that a matrix gets the
+// same bits in every batch. Below a short side of 384 a single call has too few of
+// the split products' 64² tiles and waits for their loads (256 x 4096 279 us
+// against 229 on the fp32 MFMA's 32² tiles, 256² 116 against 106); from 512 on it
+// is as fast or faster (512² the same, 768² 187 against 219, 2048² 0.70 ms against
+// 1.57). Between, single calls lose (384² 132 us against 126, 384 x 1536 188
+// against 165) and buckets, which is how Muon calls it, win (eight 384 x 1024 192
+// against 293). Sides just above a multiple of 128, whose planes would not fit
+// the workspace of the fp32 chain, keep that chain (a sum that grows with the
+// batch on both sides alike).
+constexpr int64_t kNsSplitMinSide = 384;
+inline bool ns5_split(int64_t m, int64_t n, int64_t steps, double a, double b, double c, double eps) {
+  return m >= kNsSplitMinSide && ns_split_coeffs(steps, a, b, c, eps) &&
+         ns5_split_ws_bytes(1, m, n) <= ns5_ws_bytes_t<float>(1, m, n);
 }
 
 int ns5_split_run(const float* G, float* out, int64_t batch, int64_t rows, int64_t cols, int64_t steps, double a,
@@ -583,7 +586,7 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
   PTO_REQUIRE(!aliased || g0 == o0, "newton_schulz_orthogonalize: out partially overlaps G");
 
   if constexpr (std::is_same<T, float>::value) {
-    if (ns5_split(batch, m, n, steps, a, b, c, eps))
+    if (ns5_split(m, n, steps, a, b, c, eps))
       return ns5_split_run(G, out, batch, rows, cols, steps, a, b, c, eps, ws, ws_bytes, stream);
   }
 

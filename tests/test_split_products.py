@@ -312,7 +312,7 @@ def test_two_sided_split_non_finite_lands_where_fp32_puts_it():
     assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), plain.nan_to_num(7.0, 8.0, 9.0))
 
 
-@pytest.mark.parametrize("b,m,n", [(4, 1830, 1840)])
+@pytest.mark.parametrize("b,m,n", [(8, 1024, 1024), (16, 512, 700), (3, 1500, 1501), (4, 1830, 1840)])
 def test_two_sided_batch_gives_single_bits(b, m, n):
     A, X, B = (t.cuda() for t in _sides(b, m, n))
     X[1, 4, 6], B[2, 1, 7] = math.nan, math.inf
@@ -339,3 +339,13 @@ def test_ns5_split_keeps_small_rows_and_columns(shape, s):
     for dim, at in ((-1, 3), (-2, 130)):
         e, p = _err(got, want, dim), _err(plain, want, dim)
         assert e.max() <= 2 * p.max() and e[at] <= 1.5 * max(p[at].item(), _rel(plain, want))
+
+
+@pytest.mark.parametrize("shape", [(8, 256, 1024), (16, 128, 200), (8, 384, 512), (3, 576, 700), (4, 700, 576)])
+def test_ns5_batch_gives_single_bits(shape):
+    G = _randn(31, *shape).cuda()
+    G[1, 5] *= 1e-8
+    G[-1, 2, 3] = math.inf
+    got = ops.newton_schulz_orthogonalize(G)
+    for g, o in zip(G, got):
+        assert torch.equal(o.nan_to_num(7.0), ops.newton_schulz_orthogonalize(g).nan_to_num(7.0))
