@@ -3,7 +3,7 @@ float64: their error may not exceed that of the same computation in plain fp32
 multiply-adds over k, which is how the fp32 matrix instructions sum.
 
 Sizes sit at the edges of the 64, 128, 192 and 256 tiles, at the K padding of
-128 and at the smallest sizes that take the path.
+128 and on both sides of the smallest sizes that take the path.
 """
 
 import math
@@ -73,7 +73,8 @@ def _ns64(G, steps, coeffs, eps=1e-7):
 # tiny and its planes' exponents follow ‖X0‖)
 @pytest.mark.parametrize("shape,scale", [
     ((512, 512), 1.0), ((512, 513), 1e-3), ((700, 520), 1e-3), ((4, 257, 1025), 1e-9), ((8, 192, 200), 1e3),
-    ((8, 321, 185), 1e-14), ((1, 770, 2049), 1e-25), ((16, 128, 130), 1.0)])
+    ((8, 321, 185), 1e-14), ((1, 770, 2049), 1e-25), ((16, 128, 130), 1.0), ((384, 384), 1.0), ((2, 511, 700), 1e3),
+    ((3000, 447), 1e-14)])
 def test_ns5_split_error_is_fp32s(shape, scale):
     G = _randn(sum(shape), *shape, scale=scale)
     got = ops.newton_schulz_orthogonalize(G.cuda())
@@ -175,6 +176,17 @@ def test_gram_split_error_is_fp32s(rows, d, ones):
     assert torch.equal(torch.isnan(got).cpu(), hit)
 
 
+def test_gram_split_constant_column():
+    # l·l, which the products leave out, is largest against h·h for a significand
+    # just below 1 + 2^-11 (2^-22), and always positive on the diagonal
+    X = torch.randn(8193, 1024, generator=torch.Generator().manual_seed(4))
+    X[:, 0] = 1 + 2.0 ** -11 - 2.0 ** -23
+    F = torch.zeros(1024, 1024, device="cuda")
+    ops.gram_update_(F, X.cuda(), beta=0.0, alpha=1.0)
+    want = X[:, 0].double().square().sum().item()
+    assert abs(F[0, 0].item() / want - 1) <= 2.0 ** -21
+
+
 # ---------------------------------------------------------------- two-sided products
 
 
@@ -253,7 +265,7 @@ def test_two_sided_split_keeps_small_rows_and_columns(kind, ta, tb):
     _rows_no_worse(got, want, plain, dim=-2)
 
 
-@pytest.mark.parametrize("scale", [1e-30, 1e-20, 1e18])
+@pytest.mark.parametrize("scale", [1e-33, 1e-30, 1e-20, 1e18])
 def test_two_sided_split_scale_of_x(scale):
     A, X, B = (t[0] for t in _sides(1, 1830, 1840))
     X = X * 1e3 * scale
