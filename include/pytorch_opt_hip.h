@@ -54,7 +54,10 @@ int pto_runtime_version(void);
  * G and out are [batch, rows, cols] of `dtype`. bf16 computes with bf16
  * operands and fp32 accumulation when min(rows, cols) >= 128 (below that
  * the fp32 chain runs and the result is rounded once, as the reference
- * computes every bf16 input); f32/f64 stay in their own precision. In f32
+ * computes every bf16 input); f32/f64 stay in their own precision (f32 with
+ * a short side of 384 or more holds X and its products' operands as two fp16
+ * planes where coefficients, rows and columns allow, with errors no larger
+ * than the f32 chain's). In f32
  * and f64 every matrix of a batch gets the bits of its single call (in bf16
  * the tile, and so the last bits, depend on the batch).
  * out may be G itself (in place) but must not otherwise overlap it. G may
@@ -192,7 +195,10 @@ int pto_two_sided_product(const void* A, const void* X, const void* B, void* out
  * which the harnesses use for same-shape parameters (SOAP rotations,
  * K-FAC and EKFAC preconditioning, Shampoo's apply). shared_a / shared_b
  * in the workspace query: the matching stride is 0. In f32 and f64 every
- * matrix gets the bits of its single call, shared factors or not.
+ * matrix gets the bits of its single call, shared factors or not. Large f32
+ * products (short side from 1500, or from 512 with m*n*(m+n) >= 1.2e10)
+ * scale each matrix's factors by its own X, so there a shared factor takes
+ * as much workspace as separate ones.
  */
 size_t pto_two_sided_product_batched_workspace_bytes(int dtype, int64_t batch, int64_t m, int64_t n, int shared_a,
                                                      int shared_b);

@@ -38,18 +38,17 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
-// fp32 operands as pairs of fp16 ("split"): x·2^-e = h + l with h = fp16(x·2^-e)
-// and l = fp16(x·2^-e - h), held as two planes of the same layout, l's at
-// SplitArgs::pP (pQ) elements from h's. e is an exponent per row of the
-// operand (or one per matrix) that puts the row's largest value at 2^13..2^14,
-// so h + l keeps 22-24 bits of every value down to 2^-16 of that largest one
-// and 2^-39 of it below. A product is h·h + h·l + l·h in fp32 accumulators
-// (l·l is below 2^-24 of h·h), in 3/16 of the fp32 MFMA's time. That one
-// rounds its accumulator after every k; the fp16 one after every eight (its
-// products are exact, and subnormal operands are kept), so the errors come out
-// below those of the fp32 MFMA: fp32 NS5 12 x 2048² 2.7e-6 against 4.2e-6 of
-// the exact result, at 16.3 -> 5.4 ms (126 -> 380 TFLOP/s; 256² tiles of the
-// update sustain 467, the MFMAs 56% of the time busy).
+// fp32 operands as pairs of fp16 ("split"): x·2^e = h + l with h = fp16(x·2^e)
+// and l = fp16(x·2^e - h), held as two planes of the same layout, l's at
+// SplitArgs::pP (pQ) elements from h's, with an exponent e per row of the operand
+// or one per matrix (split.h says which, and how many bits are left). A product
+// is h·h + h·l + l·h in fp32 accumulators, in 3/16 of the fp32 MFMA's time. That
+// one rounds its accumulator after every k; the fp16 one after every eight (its
+// products are exact, and subnormal operands are kept), so over evenly scaled
+// operands the errors come out below those of the fp32 MFMA: fp32 NS5 12 x 2048²
+// 2.8e-6 against 4.2e-6 of the exact result, at 16.3 -> 5.35 ms (126 -> 385
+// TFLOP/s; its 256² update sustains 458, the MFMAs 71% of the time busy, gram and
+// square 56 and 51%).
 struct sp16 {
   _Float16 v;
 };

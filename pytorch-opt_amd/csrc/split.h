@@ -1,11 +1,28 @@
-// Split operands (sp16): fp32 matrices as two fp16 planes for the fp16 MFMA.
+// Split operands (sp16): fp32 matrices as two fp16 planes for the fp16 MFMA, the
+// products h·h + h·l + l·h in fp32 accumulators (Markidis, Der Chien, Laure, Peng
+// and Vetter, IPDPS workshops 2018; Ootomo and Yokota, IJHPCA 2022).
 //
-// Whoever makes the planes picks power-of-two scales (exact) so that the
-// largest value of each row, column or matrix lands in 2^13 .. 2^14; the
-// product's epilogue takes them out again with ldexp. The fp16 range below
-// that is 2^38 wide (subnormals included: the MFMA keeps them), so what a
-// value loses against its fp32 form is below 2^-39 of the largest value that
-// shares its scale, or 2^-23 of itself, whichever is larger.
+// Whoever makes the planes picks power-of-two scales (exact); the product's
+// epilogue takes them out again with ldexp. Two kinds:
+//   * measured (factor updates, Grams, two-sided products): the largest value of
+//     each row, or column, lands in [2^13, 2^14);
+//   * from an a-priori bound (NS5): the bound does, the values lie below it by as
+//     much as the bound is wide, 2^7 to 2^11 for an ordinary X.
+// h has 11 significant bits and l 11 of what is left, down to fp16's smallest
+// step of 2^-24 (the MFMA keeps subnormals). So a value is off by at most 2^-22 of
+// itself, or by half that step, 2^-38 of a row's largest value (2^-39 of what it
+// is scaled to), whichever is larger, and the product left out, l·l, is at most
+// 2^-22 of h·h. What is smaller than 2^-16 of its row's largest value is held to
+// fewer than 22 bits; what that means for each path:
+//   * factor updates and Grams: an entry (i, j) is right to about 2^-22 of
+//     |g_i|·|g_j| (the geometric mean of the two diagonal entries), not of the sum
+//     of the |g_ik·g_jk|, which can be far smaller where two rows hold their large
+//     values at different k;
+//   * two-sided products: a row or column that is small as a whole keeps its bits
+//     (apply.hip); an entry that is below 2^-16 of its row's and of its column's
+//     largest value is held to 2^-38 of them;
+//   * NS5: matrices with a row or column so small that this would show run the
+//     fp32 chain (ns5.hip).
 #pragma once
 
 #include "aux_kernels.h"
