@@ -425,6 +425,10 @@ __device__ __forceinline__ void store_rows(const typename MF::cvec_t (&acc)[FM][
   // transposed runs: 8 lanes share a column c and cover 64 consecutive rows
   constexpr int CBT = WTN / 8;
   constexpr int ITEMS_T = ((RPP / 8 + 7) / 8) * CBT;
+  // where this lane's accumulators go: element r of a fragment lies a constant
+  // number of rows from element 0, so the writes pair up on one address (bf16 4 x
+  // 768² NS5 245.9 -> 244.8 us)
+  S* const own = stg + MF::row(lane, 0) * SP + MF::col(lane, 0);
 #pragma unroll
   for (int hp = 0; hp < WTE / RPP; ++hp) {
     const int pr0 = wr0 + EFM * MF::MN + hp * RPP;  // first output row of this pass
@@ -446,11 +450,8 @@ __device__ __forceinline__ void store_rows(const typename MF::cvec_t (&acc)[FM][
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-        for (int r = 0; r < MF::NACC; ++r) {
-          const int li = (fm - EFM) * MF::MN - hp * RPP + MF::row(lane, r);
-          const int lj = fn * MF::MN + MF::col(lane, r);
-          stg[li * SP + lj] = static_cast<S>(acc[fm][fn][r]);
-        }
+        for (int r = 0; r < MF::NACC; ++r)
+          own[((fm - EFM) * MF::MN - hp * RPP + MF::row(0, r)) * SP + fn * MF::MN] = static_cast<S>(acc[fm][fn][r]);
     __builtin_amdgcn_s_waitcnt(PTO_LGKM0);
     __builtin_amdgcn_wave_barrier();
 #pragma unroll

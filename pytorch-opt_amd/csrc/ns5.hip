@@ -45,8 +45,10 @@ __global__ void __launch_bounds__(256) ns_scale_kernel(const double* __restrict_
 }
 
 // A = s²·v: the first gram reads the input itself when no pack is needed,
-// so the 1/(‖G‖ + eps) scale lands here (scale == nullptr: A = v).
-template <typename T, typename A>
+// so the 1/(‖G‖ + eps) scale lands here (SCALED; without it A = v). A choice at
+// run time put a branch and a scalar load on every run of the epilogue, gram and
+// update: bf16 4 x 768² 243.8 -> 240.0 us with kernels of their own.
+template <typename T, typename A, bool SCALED = false>
 struct EpiNsGram {
   typedef A S;
   T* dst;
@@ -59,7 +61,7 @@ struct EpiNsGram {
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
   __device__ __forceinline__ void store(T* p, int b, const S* v, int kbeg, int n) const {
-    const S s2 = scale ? scale[b] * scale[b] : S(1);
+    const S s2 = SCALED ? scale[b] * scale[b] : S(1);
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = s2 * v[k];
@@ -109,10 +111,10 @@ struct EpiNsSq {
   __device__ __forceinline__ void finish(int) const {}
 };
 
-// X' = s·v (s per matrix, scale == nullptr: s = 1; the first update of an
-// unpacked input applies 1/(‖G‖ + eps) here), stored to dst (row-major)
+// X' = s·v (s per matrix where SCALED: the first update of an unpacked input
+// applies 1/(‖G‖ + eps) here), stored to dst (row-major)
 // and/or dstT (transposed copy).
-template <typename T, typename A>
+template <typename T, typename A, bool SCALED = false>
 struct EpiNsUpdate {
   typedef A S;
   T* dst;
@@ -127,7 +129,7 @@ struct EpiNsUpdate {
   __device__ __forceinline__ void load(int, int, int, int, int, Pre&) const {}
   __device__ __forceinline__ void load_t(int, int, int, int, PreT&) const {}
   __device__ __forceinline__ void store(T* p, int b, const S* v, int kbeg, int n) const {
-    const S s = scale ? scale[b] : S(1);
+    const S s = SCALED ? scale[b] : S(1);
     S w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = s * v[k];
@@ -667,12 +669,13 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
     // iteration 0 of an unpacked input reads G (stride sG == sX, no pads)
     const bool from_g = direct && t == 0;
     const T* Xc = from_g ? G : X[cur];
-    const A* s0 = from_g ? scale : nullptr;
     // 1. A = X·Xᵀ
     {
       GemmArgs g{Xc, ldn, sX, Xc, ldn, sX, (int)m, (int)m, (int)ldn, 0, 0, nullptr};
-      EpiNsGram<T, A> e{Ab, ldm, sAB, s0};
-      if (launch_gemm<T, true>(g, e, nb, stream, "ns5_gram")) return -1;
+      if constexpr (QN) {
+        if (from_g && launch_gemm<T, true>(g, EpiNsGram<T, A, true>{Ab, ldm, sAB, scale}, nb, stream, "ns5_gram")) return -1;
+      }
+      if (!from_g && launch_gemm<T, true>(g, EpiNsGram<T, A>{Ab, ldm, sAB, nullptr}, nb, stream, "ns5_gram")) return -1;
     }
     // 2. B' = a·I + b·A + c·A·A
     {
@@ -691,7 +694,6 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
     //    transpose, X written in place since this product does not read it)
     {
       EpiNsUpdate<T, A> e{};
-      e.scale = s0;
       if (!last && QN) {
         e.dst = X[cur ^ 1]; e.ld_d = ldn; e.s_d = sX;
         e.dstT = nullptr;
@@ -708,7 +710,12 @@ int ns5_t(const T* G, T* out, int64_t batch, int64_t rows, int64_t cols, int64_t
       if constexpr (QN) {
         // B' is symmetric: read as its own transpose (PT), like X (QN)
         GemmArgs g{Bb, ldm, sAB, Xc, ldn, sX, (int)m, (int)n, (int)ldm, 0, 0, nullptr};
-        if (launch_gemm_qn<EpiNsUpdate<T, A>, true>(g, e, nb, stream, "ns5_update")) return -1;
+        if (from_g) {
+          const EpiNsUpdate<T, A, true> es{e.dst, e.ld_d, e.s_d, e.dstT, e.ld_t, e.s_t, scale};
+          if (launch_gemm_qn<EpiNsUpdate<T, A, true>, true>(g, es, nb, stream, "ns5_update")) return -1;
+        } else if (launch_gemm_qn<EpiNsUpdate<T, A>, true>(g, e, nb, stream, "ns5_update")) {
+          return -1;
+        }
       } else {
         GemmArgs g{Bb, ldm, sAB, XT[cur], ldm, n * ldm, (int)m, (int)n, (int)ldm, 0, 0, nullptr};
         if (launch_gemm<T, false>(g, e, nb, stream, "ns5_update")) return -1;
