@@ -361,3 +361,42 @@ def test_ns5_batch_gives_single_bits(shape):
     got = ops.newton_schulz_orthogonalize(G)
     for g, o in zip(G, got):
         assert torch.equal(o.nan_to_num(7.0), ops.newton_schulz_orthogonalize(g).nan_to_num(7.0))
+
+
+# A matrix whose planes do not serve, over the split products' tiles: the bits of
+# the fp32 kernels, which a negative eps (lost in the norm's rounding) asks for.
+@pytest.mark.parametrize("shape", [(512, 640), (1000, 1100), (2048, 2048), (3100, 3000), (4, 2048, 2100), (12, 1024, 1024),
+                                   (2, 3072, 768), (4096, 4096)])
+def test_ns5_flagged_matrix_gets_the_fp32_kernels_bits(shape):
+    G = _randn(41, *shape).cuda()
+    G[..., 3, :] *= 1e-9
+    got = ops.newton_schulz_orthogonalize(G, eps=0.0)
+    assert torch.equal(got, ops.newton_schulz_orthogonalize(G, eps=-1e-30))
+
+
+@pytest.mark.parametrize("m,n", KRON + [(1024, 6000), (4096, 4100)])
+def test_kron_flagged_over_tiles(m, n):
+    G = _randn(m + n, m, n)
+    G[7, 9], G[m - 1, n - 1] = math.inf, math.nan
+    L, R = torch.zeros(m, m, device="cuda"), torch.zeros(n, n, device="cuda")
+    ops.kron_factor_update_(L, R, G.cuda(), beta2=1.0)
+    for got, P in ((L, G), (R, G.mT)):
+        plain = _chain(P, P)
+        assert torch.equal(got.isnan(), plain.isnan()) and torch.equal(got.isposinf(), plain.isposinf())
+        ok = torch.isfinite(plain)
+        diff = (got[ok].double() - plain[ok].double()).norm() / plain[ok].double().norm()
+        assert diff.item() <= 4e-6  # two orders of up to 6000 fp32 additions
+
+
+@pytest.mark.parametrize("m,n", [(1500, 1500), (640, 4096), (2049, 1700), (3000, 3100), (4096, 4096)])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+def test_two_sided_flagged_over_tiles(m, n, ta, tb):
+    # a row of op(A) that meets only a row of X at 1e-34: its scale would leave fp32
+    A, X, B = (t[0] for t in _sides(1, m, n))
+    X, a = X * 1e3, A.mT if ta else A
+    X[5] *= 1e-34
+    a[5], a[5, 5] = 0.0, 2.0
+    b = B.mT if tb else B
+    got = ops.two_sided_product(A.cuda(), X.cuda(), B.cuda(), transpose_a=ta, transpose_b=tb)
+    want = (a.double().cuda() @ X.double().cuda() @ b.double().cuda()).cpu()
+    _rows_no_worse(got, want, _chain(_chain(a, X.mT), b.mT))
